@@ -621,14 +621,54 @@ std::vector<Plan> factor_candidates(unsigned long long N) {
 std::map<unsigned long long, int> g_tuned;
 std::map<unsigned long long, int> g_tuned_batch;
 
-// Untuned choice: a two-pass split whose strided pass still moves >= 8
-// columns (128-byte runs) per row; otherwise the three-pass split with the
-// largest inner pass <= 4096 and the shortest first pass, so every strided
-// pass runs 16 columns wide (narrow strided tiles reach about half the
-// bandwidth of 16-column ones on MI355X).
-int default_candidate(const std::vector<Plan> &c) {
-  for (size_t i = 0; i < c.size(); i++)
-    if (c[i].P <= 2 && (c[i].P == 1 || c[i].C[0] >= 8)) return (int)i;
+// Untuned choice, from every split timed for one product of each length on one
+// MI355X (the best and the chosen one lie within 4 % from 2^19 points up, and
+// within run-to-run noise below):
+//  * up to 2^23 points two passes of 256 rows (512 or 1024 once the inner pass
+//    would pass 8192 points; fewer rows once it would fall under 128): 256
+//    inner blocks give every CU one, which at 3 * 2^17 points is 63 us against
+//    75 us for 64 blocks of 6144, and at 2^20 75 us against 91 us for 128 of
+//    8192;
+//  * beyond, three passes of 256 x 256 x inner (512 rows in the second pass once
+//    the inner pass would pass 2048 points): short inner blocks leave eight or
+//    more workgroups on a CU, whose LDS, FP64 and memory phases overlap, and the
+//    middle passes of these tiles run chunked; at 2^26 points 2.50 ms against
+//    2.87 ms for 64 x 256 x 4096;
+//  * 16 columns per strided tile where that leaves at least 384 of them and two
+//    workgroups' LDS on a CU (so not with 512 rows), else 8: 8 against 16 columns
+//    is 75 us against 79 us at 2^20 points, 107 us against 100 us at 2^21 and
+//    8.6 ms against 9.2 ms in the 512-row pass at 3 * 2^26.
+// The products of a batched class fill the GPU together, so its short lengths
+// keep the longest inner pass and 16 columns (4096 products of 16 to 16384
+// words: 1.10 ms against 1.16 ms with the split of single products).
+int default_candidate(const std::vector<Plan> &c, bool batched = false) {
+  const unsigned long long N = c[0].N;
+  auto find = [&](int P, unsigned long long l0, unsigned long long l1, int c0) {
+    for (size_t i = 0; i < c.size(); i++)
+      if (c[i].P == P && c[i].L[0] == (int)l0 && (P < 3 || c[i].L[1] == (int)l1) && c[i].C[0] == c0 &&
+          (P < 3 || c[i].C[1] == (l1 == 512 ? 8 : 16)))
+        return (int)i;
+    return -1;
+  };
+  if (c[0].P == 1) return 0;
+  if (batched && N <= (1ull << 17))
+    for (size_t i = 0; i < c.size(); i++)
+      if (c[i].P == 2 && c[i].C[0] >= 8) return (int)i;
+  const unsigned long long max_in = is_three(N) ? 6144 : 8192;
+  if (N <= (1ull << 23)) {
+    unsigned long long rows = 256;
+    while (N / rows > max_in) rows *= 2;
+    while (rows > 64 && N / rows < 128) rows /= 2;
+    const int cols = rows <= 256 && N / rows >= 16 * 384 ? 16 : 8;
+    const int i = find(2, rows, 0, cols);
+    if (i >= 0) return i;
+  } else {
+    const unsigned long long l1 = N / 65536 > 2048 ? 512 : 256;
+    const int i = find(3, 256, l1, 16);
+    if (i >= 0) return i;
+  }
+  // the longest transforms: a three-pass split with the largest inner pass <=
+  // 4096 and the shortest first pass, or whatever there is
   int best = -1;
   for (size_t i = 0; i < c.size(); i++) {
     if (c[i].P != 3 || c[i].L[2] > 4096) continue;
@@ -661,7 +701,7 @@ bool factor_cached(unsigned long long N, Plan &p, bool batched = false) {
   if (it == g_cands.end()) it = g_cands.emplace(N, factor_candidates(N)).first;
   const std::vector<Plan> &c = it->second;
   if (c.empty()) return false;
-  int idx = default_candidate(c);
+  int idx = default_candidate(c, batched);
   auto t = g_tuned.find(N);
   if (t != g_tuned.end() && t->second >= 0 && t->second < (int)c.size()) idx = t->second;
   if (batched) {

@@ -66,7 +66,13 @@ fwd_fn pick_inv_keep(int L, int C) {
 mid_fn pick_mid_keep(int L) {
   switch (L) {
     case 192: return &mid_keep<192>;
+    case 256: return &mid_keep<256>;
+    case 384: return &mid_keep<384>;
+    case 512: return &mid_keep<512>;
+    case 768: return &mid_keep<768>;
     case 1024: return &mid_keep<1024>;
+    case 1536: return &mid_keep<1536>;
+    case 2048: return &mid_keep<2048>;
   }
   return nullptr;
 }
