@@ -1028,7 +1028,7 @@ int run_chunk(const Plan &p, const ChunkPlan &ch, const PassArgs &f, const PassA
     y.data = da + off;
     y.data_b = db + off;
     ProfScope ps(BCG_K_MID, s);
-    if (ch.mid(square, false, (int)(jc * ch.S1 / (unsigned long long)p.L[2]), 1, s, y))
+    if (ch.mid(square, (int)(jc * ch.S1 / (unsigned long long)p.L[2]), 1, s, y))
       return fail(BCG_E_ARG, "kernel rejected this pass");
     HIPCHK(hipGetLastError());
   }
@@ -1043,7 +1043,8 @@ int run_chunk(const Plan &p, const ChunkPlan &ch, const PassArgs &f, const PassA
   return 0;
 }
 
-// Run the transforms of plan p up to the rounded coefficients (in bufB).
+// Run the transforms of the multi-pass plan p up to the rounded coefficients or
+// their group sums (in bufB).
 int run_transforms(const Plan &p, const uint32_t *A, unsigned long long AL, const uint32_t *B,
                    unsigned long long BL, bool square, hipStream_t s) {
   const size_t arr = (size_t)p.N * sizeof(cd);
@@ -1061,18 +1062,6 @@ int run_transforms(const Plan &p, const uint32_t *A, unsigned long long AL, cons
   a.bl = BL;
   a.margin = (unsigned int *)g.margin.p;
   a.margin_mask = MARGIN_SLOTS - 1;
-  if (p.P == 1) {
-    if (int rc = pass_args(p, 0, a)) return rc;
-    a.data = da;
-    a.data_b = db;
-    a.coef = coef;
-    mid_fn f = pick_mid(p.L[0]);
-    if (!f) return fail(BCG_E_ARG, "no kernel for this length");
-    ProfScope ps(BCG_K_MID, s);
-    if (f(square, true, 1, 1, s, a)) return fail(BCG_E_ARG, "kernel rejected this pass");
-    HIPCHK(hipGetLastError());
-    return 0;
-  }
   ChunkPlan ch;
   const bool chunked = chunk_plan(p, square, ch);
   // forward outer passes for A (and B)
@@ -1115,7 +1104,7 @@ int run_transforms(const Plan &p, const uint32_t *A, unsigned long long AL, cons
     mid_fn f = pick_mid(p.L[i]);
     if (!f) return fail(BCG_E_ARG, "no middle kernel for this length");
     ProfScope ps(BCG_K_MID, s);
-    if (f(square, false, (int)(p.N / (unsigned long long)p.L[i]), 1, s, b)) return fail(BCG_E_ARG, "kernel rejected this pass");
+    if (f(square, (int)(p.N / (unsigned long long)p.L[i]), 1, s, b)) return fail(BCG_E_ARG, "kernel rejected this pass");
     HIPCHK(hipGetLastError());
   }
   // inverse outer passes, the outermost one rounding into coefficients
@@ -1220,35 +1209,19 @@ int fill_zero(uint32_t *C, size_t CL, hipStream_t s) {
   return 0;
 }
 
-// Workgroups resident per CU for a one-pass class kernel (LDS bound).
-int mul1_grid(int L, int count) {
-  size_t lds = (size_t)(L + L / 16) * 16 + 256;
-  int per_cu = (int)(160 * 1024 / lds);
-  if (per_cu < 1) per_cu = 1;
-  if (per_cu > 8) per_cu = 8;
-  int grid = 256 * per_cu;
-  return count < grid ? count : grid;
-}
-
-__global__ void k_zero_i32(int *p, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
 // Launch the one-pass products desc[first .. first+count) of length class L
 // (descriptors and margin slots already on the device).
-int run_class(int L, const MulDesc *ddesc, int count, unsigned int *dmargins, int *dcounter, hipStream_t s) {
+int run_class(int L, const MulDesc *ddesc, int count, unsigned int *dmargins, hipStream_t s) {
   ClassArgs ca;
   ca.desc = ddesc;
   ca.count = count;
   if (int rc = get_roots((unsigned long long)L, &ca.roots)) return rc;
   if (int rc = get_ltab(L, &ca.tl)) return rc;
   ca.margins = dmargins;
-  ca.next = dcounter;
   mul1_fn f = pick_mul1(L);
   if (!f) return fail(BCG_E_ARG, "no one-pass kernel for this length");
   ProfScope ps(BCG_K_MID, s);
-  f(mul1_grid(L, count), s, ca);
+  f(count, s, ca);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1257,7 +1230,6 @@ int run_class(int L, const MulDesc *ddesc, int count, unsigned int *dmargins, in
 int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL,
                 hipStream_t s, double *margin, const uint32_t *D = nullptr, size_t DL = 0) {
   if (int rc = ensure(g.desc, sizeof(MulDesc))) return rc;
-  if (int rc = ensure(g.counters, 64)) return rc;
   MulDesc d;
   d.a = A;
   d.b = B;
@@ -1271,23 +1243,21 @@ int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t
   d.cbits = coef_bits(p);
   if (int rc = h2d(g.desc.p, &d, sizeof d, s)) return rc;
   if (int rc = zero_margin(s)) return rc;
-  LAUNCH(k_zero_i32, 1, 64, s, (int *)g.counters.p, 1);
-  if (int rc = run_class(p.L[0], (const MulDesc *)g.desc.p, 1, (unsigned int *)g.margin.p, (int *)g.counters.p, s))
-    return rc;
+  if (int rc = run_class(p.L[0], (const MulDesc *)g.desc.p, 1, (unsigned int *)g.margin.p, s)) return rc;
   return read_margin(s, margin);
 }
 
 // Batched multi-pass products of one plan (same N and pass split): every pass
 // is one launch over (tiles x products); product p owns arrays p*N in the
 // batch buffers and margin slot p. Descriptors already on the device.
-// Scratch of batched launches: descriptors, margins, class counters, the
+// Scratch of batched launches: descriptors, margins, the
 // batched transform arrays and carry block functions. The plain batch call
 // uses the engine's set; a captured batch owns one (its graph keeps the
 // addresses).
 struct BatchBufs {
-  DevBuf tdesc, mdesc, cdesc, margins, counters, tA, tB, blk;
+  DevBuf tdesc, mdesc, cdesc, margins, tA, tB, blk;
   void release() {
-    for (DevBuf *b : {&tdesc, &mdesc, &cdesc, &margins, &counters, &tA, &tB, &blk}) {
+    for (DevBuf *b : {&tdesc, &mdesc, &cdesc, &margins, &tA, &tB, &blk}) {
       if (b->p) (void)hipFree(b->p);
       b->p = nullptr;
       b->bytes = 0;
@@ -1340,7 +1310,7 @@ int run_multipass_class(const Plan &p, const MulDesc *ddesc, const std::vector<M
     mid_fn f = pick_mid(p.L[i]);
     if (!f) return fail(BCG_E_ARG, "no middle kernel for this length");
     ProfScope ps(BCG_K_MID, s);
-    if (f(false, false, (int)(p.N / (unsigned long long)p.L[i]), count, s, b)) return fail(BCG_E_ARG, "kernel rejected this pass");
+    if (f(false, (int)(p.N / (unsigned long long)p.L[i]), count, s, b)) return fail(BCG_E_ARG, "kernel rejected this pass");
     HIPCHK(hipGetLastError());
   }
   // group mode when every product of the class has exact group sums: the last
@@ -2233,7 +2203,6 @@ int batch_upload(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
   if (int rc = ensure(bb.mdesc, nm * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.cdesc, nc * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.margins, (nm + nc) * sizeof(unsigned int))) return rc;
-  if (int rc = ensure(bb.counters, (bp.cgroups.size() + 1) * sizeof(int))) return rc;
   size_t arr = 0, blk = 16;
   for (auto &gr : bp.mgroups) {
     const Plan &p = gr.first;
@@ -2263,7 +2232,6 @@ int batch_launch(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
   const size_t nm = bp.mdesc.size(), nc = bp.cdesc.size();
   unsigned int *mm = (unsigned int *)bb.margins.p, *cm = mm + nm;
   if (nm + nc) LAUNCH(k_zero_u32, (int)((nm + nc + 255) / 256), 256, s, mm, (int)(nm + nc));
-  if (!bp.cgroups.empty()) LAUNCH(k_zero_i32, 1, 64, s, (int *)bb.counters.p, (int)bp.cgroups.size());
   HIPCHK(hipGetLastError());
   // one-pass length classes: independent persistent launches, spread over the
   // side streams (largest class first), beside the multi-pass groups on s, so
@@ -2296,8 +2264,7 @@ int batch_launch(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
       const int ci = order[k];
       const auto &gr = bp.cgroups[ci];
       const size_t first = gr.second.first, n = gr.second.second;
-      rc = run_class(gr.first, (const MulDesc *)bb.cdesc.p + first, (int)n, cm + first, (int *)bb.counters.p + ci,
-                     g.aux[k % Engine::NAUX]);
+      rc = run_class(gr.first, (const MulDesc *)bb.cdesc.p + first, (int)n, cm + first, g.aux[k % Engine::NAUX]);
     }
   }
   if (!rc && !bp.tiny.empty()) {

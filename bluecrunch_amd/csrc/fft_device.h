@@ -434,6 +434,187 @@ __device__ __forceinline__ void dft3(cd &a, cd &b, cd &c) {
   c = csub(m, r);
 }
 
+// ------------------------------------------------------ contiguous blocks
+//
+// A length-L DFT of one contiguous block of points in one workgroup (middle
+// passes and one-pass products), E points per thread: L/E threads, radix-E
+// stages in registers (the first takes the remainder bits) and LDS exchanges
+// between them. E = 8 leaves enough waves to hide LDS, memory and FP64 latency
+// where few workgroups share a CU (24 points a thread were four waves per CU at
+// 6144 points); E = 16 saves an exchange and wins where many short blocks fill
+// the CU anyway. One slot of padding every E points keeps the 16-byte accesses
+// of a stage on distinct banks. Spans are compile-time constants, so the row
+// offsets of a butterfly become instruction offsets.
+// Values a thread holds after the innermost stage: E, or (E = 8) three radix-3
+// butterflies (the third only in threads tid < T - T/3).
+constexpr int row_xr(int L, int E) { return L % 3 == 0 ? 9 : E; }
+
+template <int L, int E = 8>
+struct Row {
+  static constexpr bool THREE = Len<L>::THREE;
+  static constexpr int LOG = Len<L>::LOG;
+  static constexpr int RB = ilog2c(E);
+  static constexpr int T = L / E;
+  static constexpr int NST2 = (LOG + RB - 1) / RB;  // radix-2^b stages
+  static constexpr int FIRSTB = LOG - RB * (NST2 - 1);
+  static constexpr int R0 = 1 << FIRSTB;
+  static constexpr int PER0 = E / R0;
+  static constexpr int XR = row_xr(L, E);
+  static constexpr int LDS_ELEMS = L + L / E;
+  // rows of a butterfly block of stage s
+  static constexpr int span(int s) { return s == 0 ? L : L >> (FIRSTB + RB * (s - 1)); }
+  // LDS slot of point e
+  __device__ static __forceinline__ int pad(int e) { return e + (e >> RB); }
+  // pad(r + t * S) for t < E, linear in t when E | S, or S = 1 and E | r.
+  template <int S>
+  __device__ static __forceinline__ int slot(int r, int t) {
+    if constexpr (S % E == 0) return pad(r) + t * (S + S / E);
+    else if constexpr (S == 1) return pad(r) + t;
+    else return pad(r + t * S);
+  }
+  static_assert(E == 8 || (E == 16 && !THREE), "eight or sixteen points per thread");
+  static_assert(NST2 >= 2 && L % E == 0, "length too short for the row stages");
+};
+
+// A thread index the compiler cannot see through: the level twiddles of A's, B's
+// and the inverse transform are the same values, and keeping them all from one
+// transform to the next takes about 100 registers, and with them half the waves;
+// reloading them from the caches is cheaper.
+__device__ __forceinline__ int row_opaque(int tid) {
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
+
+// Stage s >= 1 (radix E) in LDS. Twiddles are loaded ahead of the barrier that
+// orders the previous stage's writes before this stage's reads; a butterfly
+// writes back its own slots, so a stage needs no other barrier. KEEP: the
+// butterfly stays in x instead (innermost forward stage).
+template <class RC, int L, int S, bool INV, bool KEEP>
+__device__ __forceinline__ void row_stage(cd *lds, const cd *__restrict__ tl, int tid, cd (&x)[1 << RC::RB]) {
+  constexpr int E = 1 << RC::RB, SPAN = RC::span(S), SUB = SPAN / E;
+  const int q = SUB > 1 ? tid % SUB : 0, r = (tid / SUB) * SPAN + q;
+  cd tb[RC::RB];
+  if constexpr (SUB > 1) level_bases<RC::RB>(tl, q, L / SPAN, tb);
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < E; t++) x[t] = lds[RC::template slot<SUB>(r, t)];
+  if constexpr (SUB == 1) {
+    if constexpr (INV) dit_levels_q0<RC::RB>(x);
+    else dif_levels_q0<RC::RB>(x);
+  } else {
+    if constexpr (INV) dit_levels<RC::RB>(x, tb);
+    else dif_levels<RC::RB>(x, tb);
+  }
+  if constexpr (!KEEP) {
+#pragma unroll
+    for (int t = 0; t < E; t++) lds[RC::template slot<SUB>(r, t)] = x[t];
+  }
+}
+
+template <class RC, int L, int S>
+__device__ __forceinline__ void row_forward_stages(cd *lds, const cd *__restrict__ tl, int tid,
+                                                   cd (&x)[1 << RC::RB]) {
+  constexpr int LAST = RC::NST2 - 1;
+  if constexpr (S < LAST || (S == LAST && RC::THREE)) {
+    row_stage<RC, L, S, false, false>(lds, tl, tid, x);
+    row_forward_stages<RC, L, S + 1>(lds, tl, tid, x);
+  } else if constexpr (S == LAST) {
+    row_stage<RC, L, S, false, true>(lds, tl, tid, x);
+  }
+}
+
+template <class RC, int L, int S>
+__device__ __forceinline__ void row_inverse_stages(cd *lds, const cd *__restrict__ tl, int tid,
+                                                   cd (&x)[1 << RC::RB]) {
+  if constexpr (S >= 1) {
+    row_stage<RC, L, S, true, false>(lds, tl, tid, x);
+    row_inverse_stages<RC, L, S - 1>(lds, tl, tid, x);
+  }
+}
+
+// Forward DIF of the rows x[h] = point tid + h T (natural order); xr receives
+// the innermost stage's outputs. LDS must be free (barrier) on entry; on exit
+// every thread has read only slots that row_inverse lets it write.
+template <int L, int E>
+__device__ __forceinline__ void row_forward(cd (&x)[E], cd (&xr)[row_xr(L, E)], cd *lds, const cd *__restrict__ tl,
+                                            int tid) {
+  using RC = Row<L, E>;
+  tid = row_opaque(tid);
+#pragma unroll
+  for (int i = 0; i < RC::PER0; i++) {
+    cd v[RC::R0];
+#pragma unroll
+    for (int t = 0; t < RC::R0; t++) v[t] = x[i + t * RC::PER0];
+    dif_levels<RC::FIRSTB>(v, tl, tid + i * RC::T, 1);
+#pragma unroll
+    for (int t = 0; t < RC::R0; t++) lds[RC::template slot<RC::T>(tid, i + t * RC::PER0)] = v[t];
+  }
+  cd y[E];
+  row_forward_stages<RC, L, 1>(lds, tl, tid, y);
+  if constexpr (RC::THREE) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int b = tid + i * RC::T;
+      if (i < 2 || b < L / 3) {
+        cd p = lds[RC::pad(3 * b)], q = lds[RC::pad(3 * b + 1)], r = lds[RC::pad(3 * b + 2)];
+        dft3<false>(p, q, r);
+        xr[3 * i] = p;
+        xr[3 * i + 1] = q;
+        xr[3 * i + 2] = r;
+      } else {
+        xr[3 * i] = xr[3 * i + 1] = xr[3 * i + 2] = make_double2(0.0, 0.0);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < E; t++) xr[t] = y[t];
+  }
+}
+
+// The mirror image: xr in row_forward's layout, x[h] = point tid + h T out.
+template <int L, int E>
+__device__ __forceinline__ void row_inverse(cd (&xr)[row_xr(L, E)], cd (&x)[E], cd *lds, const cd *__restrict__ tl,
+                                            int tid) {
+  using RC = Row<L, E>;
+  tid = row_opaque(tid);
+  cd y[E];
+  if constexpr (RC::THREE) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int b = tid + i * RC::T;
+      if (i < 2 || b < L / 3) {
+        cd p = xr[3 * i], q = xr[3 * i + 1], r = xr[3 * i + 2];
+        dft3<true>(p, q, r);
+        lds[RC::pad(3 * b)] = p;
+        lds[RC::pad(3 * b + 1)] = q;
+        lds[RC::pad(3 * b + 2)] = r;
+      }
+    }
+    row_inverse_stages<RC, L, RC::NST2 - 1>(lds, tl, tid, y);
+  } else {
+#pragma unroll
+    for (int t = 0; t < E; t++) y[t] = xr[t];
+    dit_levels_q0<RC::RB>(y);
+#pragma unroll
+    for (int t = 0; t < E; t++) lds[RC::template slot<1>(E * tid, t)] = y[t];
+    row_inverse_stages<RC, L, RC::NST2 - 2>(lds, tl, tid, y);
+  }
+  cd tb[RC::PER0][RC::FIRSTB];
+#pragma unroll
+  for (int i = 0; i < RC::PER0; i++) level_bases<RC::FIRSTB>(tl, tid + i * RC::T, 1, tb[i]);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < RC::PER0; i++) {
+    cd v[RC::R0];
+#pragma unroll
+    for (int t = 0; t < RC::R0; t++) v[t] = lds[RC::template slot<RC::T>(tid, i + t * RC::PER0)];
+    dit_levels<RC::FIRSTB>(v, tb[i]);
+#pragma unroll
+    for (int t = 0; t < RC::R0; t++) x[i + t * RC::PER0] = v[t];
+  }
+}
+
 // --------------------------------------------------------- LDS stage helpers
 
 // One radix-2^RB stage of span `span` over the whole tile, LDS in and out.

@@ -102,18 +102,6 @@ __device__ __forceinline__ double digit_at(const uint32_t *__restrict__ w, unsig
   return (double)((v >> sh) & ((1ull << bits) - 1ull));
 }
 
-// Digit pair (a_j, a_{j+N}) of right-angle input point j.
-__device__ __forceinline__ cd packed_digits(const PassArgs &a, const uint32_t *__restrict__ w,
-                                            unsigned long long wl, unsigned long long j) {
-  return make_double2(digit_at(w, wl, j, a.bits), digit_at(w, wl, j + a.N, a.bits));
-}
-
-// Right-angle input point j: (a_j + i a_{j+N}) * Omega^j.
-__device__ __forceinline__ cd packed_point(const PassArgs &a, const uint32_t *__restrict__ w, unsigned long long wl,
-                                           unsigned long long j) {
-  return cmul(packed_digits(a, w, wl, j), omega_pow(a.roots, j));
-}
-
 __device__ __forceinline__ void margin_update(unsigned int *m, double d) {
   float f = (float)d;
   // non-negative floats order like their bit patterns
@@ -260,11 +248,6 @@ __device__ __forceinline__ void write_group_half(const PassArgs &a, long long *l
     uint4 *dst = reinterpret_cast<uint4 *>(a.ybuf + (j0 / C) * (unsigned long long)K);
     for (int q = 0; q < K / 4; q++) dst[q] = make_uint4(lw[4 * q], lw[4 * q + 1], lw[4 * q + 2], lw[4 * q + 3]);
   }
-}
-
-// Whole-point form for single-pass plans (M = 1): j = row.
-__device__ __forceinline__ double unpack_point(const PassArgs &a, cd v, unsigned long long j) {
-  return round_store(a, cmulc(v, omega_pow(a.roots, j)), j, 0, 0);
 }
 
 // Margin slots: a single product spreads its atomics over MARGIN_SLOTS
@@ -705,190 +688,54 @@ __attribute__((amdgpu_waves_per_eu((MODE == 1 && SplitTile<L, C>::ON && C >= 8) 
 
 // ------------------------------------------------------------- middle pass
 
-// Forward DIF of one contiguous block of L points, ending with the innermost
-// stage's outputs in registers: xr[i * R + t] for butterfly i of that stage.
-template <int L, bool PACK, int CACHE = 0>
-__device__ __forceinline__ void mid_forward(const PassArgs &a, cd *lds, const cd *__restrict__ src,
-                                            const uint32_t *__restrict__ w, unsigned long long wl,
-                                            unsigned long long blk0, cd (&xr)[Tile<L, 1>::EPT], int tid) {
-  using TC = Tile<L, 1>;
-  constexpr int RB0 = TC::FIRSTB;
-  constexpr int R0 = 1 << RB0;
-  constexpr int PER0 = TC::EPT / R0;
-  constexpr int SUB0 = L / R0;
-  // Stage 0 straight from global.
-#pragma unroll
-  for (int i = 0; i < PER0; i++) {
-    int q = tid + i * TC::T;
-    cd x[R0];
-#pragma unroll
-    for (int t = 0; t < R0; t++) {
-      unsigned long long j = blk0 + (unsigned long long)(q + t * SUB0);
-      x[t] = PACK ? packed_point(a, w, wl, j) : ld_pol<(CACHE & 1) != 0>(&src[j]);
-    }
-    dif_levels<RB0>(x, a.tl, q, 1);
-    if (TC::NST2 == 1 && !TC::THREE) {
-#pragma unroll
-      for (int t = 0; t < R0; t++) xr[i * R0 + t] = x[t];
-    } else {
-#pragma unroll
-      for (int t = 0; t < R0; t++) lds[slot_step<SUB0>(q, t)] = x[t];
-    }
-  }
-  if (TC::NST2 == 1 && !TC::THREE) return;
-  __syncthreads();
-  // Middle stages in LDS.
-  int span = L >> RB0;
-  const int last = TC::THREE ? TC::NST2 : TC::NST2 - 1;  // stages run in LDS
-  for (int s = 1; s < last; s++) {
-    int rb = stage_bits<L, 1>(s);
-    lds_stage_any<L, 1, false>(lds, rb, span, a.tl, tid);
-    __syncthreads();
-    span >>= rb;
-  }
-  if (TC::THREE) {
-    constexpr int PER = TC::EPT / 3;
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      int b3 = tid + i * TC::T;
-      cd p = lds[pad16(3 * b3)], q = lds[pad16(3 * b3 + 1)], r = lds[pad16(3 * b3 + 2)];
-      dft3<false>(p, q, r);
-      xr[3 * i] = p;
-      xr[3 * i + 1] = q;
-      xr[3 * i + 2] = r;
-    }
-  } else {
-    constexpr int RBL = TC::MAXB;  // last stage is a full MAXB stage when NST2 > 1
-    constexpr int R = 1 << RBL;
-    constexpr int PER = TC::EPT / R;
-    // span == R here: each butterfly is one contiguous block of R rows
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      int blk = tid + i * TC::T;
-      cd x[R];
-#pragma unroll
-      for (int t = 0; t < R; t++) x[t] = lds[slot<R>(blk, t)];
-      dif_levels_q0<RBL>(x);
-#pragma unroll
-      for (int t = 0; t < R; t++) xr[i * R + t] = x[t];
-    }
-  }
-}
+// Points per thread of a middle pass: a block of a power of two shares its CU
+// with enough others for sixteen to pay (2^26 points in blocks of 1024, whole
+// product: 2.50 ms against 2.54 ms with eight; equal below 2^23 points).
+constexpr int mid_points(int L) { return L % 3 != 0 && L >= 256 ? 16 : 8; }
 
-// Last forward pass of A (and B), pointwise product (or square), first inverse
-// pass on one contiguous block of L points. Ends with the outermost inverse
-// stage's outputs in registers: out[i * R0 + t] holds row q + t * (L / R0),
-// q = tid + i * T (natural order). The caller stores or unpacks them.
-template <int L, bool SQUARE, bool PACK, int CACHE = 0>
-__device__ __forceinline__ void mid_pipeline(const PassArgs &a, cd *lds, unsigned long long blk0,
-                                             cd (&xa)[Tile<L, 1>::EPT], int tid) {
-  using TC = Tile<L, 1>;
-  mid_forward<L, PACK, CACHE>(a, lds, a.data, a.wa, a.al, blk0, xa, tid);
-  if (!SQUARE) {
-    cd xb[TC::EPT];
-    __syncthreads();
-    mid_forward<L, PACK, CACHE>(a, lds, a.data_b, a.wb, a.bl, blk0, xb, tid);
-#pragma unroll
-    for (int i = 0; i < TC::EPT; i++) xa[i] = cmul(xa[i], xb[i]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < TC::EPT; i++) xa[i] = cmul(xa[i], xa[i]);
-  }
-  constexpr int RB0 = TC::FIRSTB;
-  constexpr int R0 = 1 << RB0;
-  constexpr int PER0 = TC::EPT / R0;
-  constexpr int SUB0 = L / R0;
-  if (!(TC::NST2 == 1 && !TC::THREE)) {
-    __syncthreads();  // every thread is done reading B's innermost stage from LDS
-    if (TC::THREE) {
-      constexpr int PER = TC::EPT / 3;
-#pragma unroll
-      for (int i = 0; i < PER; i++) {
-        int b3 = tid + i * TC::T;
-        cd p = xa[3 * i], q = xa[3 * i + 1], r = xa[3 * i + 2];
-        dft3<true>(p, q, r);
-        lds[pad16(3 * b3)] = p;
-        lds[pad16(3 * b3 + 1)] = q;
-        lds[pad16(3 * b3 + 2)] = r;
-      }
-    } else {
-      constexpr int RBL = TC::MAXB;
-      constexpr int R = 1 << RBL;
-      constexpr int PER = TC::EPT / R;
-#pragma unroll
-      for (int i = 0; i < PER; i++) {
-        int blk = tid + i * TC::T;
-        cd x[R];
-#pragma unroll
-        for (int t = 0; t < R; t++) x[t] = xa[i * R + t];
-        dit_levels_q0<RBL>(x);
-#pragma unroll
-        for (int t = 0; t < R; t++) lds[slot<R>(blk, t)] = x[t];
-      }
-    }
-    __syncthreads();
-    // remaining inverse stages in LDS, innermost to outermost, excluding stage 0
-    int first_lds = TC::THREE ? TC::NST2 - 1 : TC::NST2 - 2;
-    int span = TC::THREE ? 3 : 1;
-    for (int s = TC::NST2 - 1; s > first_lds; s--) span <<= stage_bits<L, 1>(s);
-    for (int s = first_lds; s >= 1; s--) {
-      int rb = stage_bits<L, 1>(s);
-      span <<= rb;
-      lds_stage_any<L, 1, true>(lds, rb, span, a.tl, tid);
-      __syncthreads();
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < PER0; i++) {
-    int q = tid + i * TC::T;
-    cd x[R0];
-    if (TC::NST2 == 1 && !TC::THREE) {
-#pragma unroll
-      for (int t = 0; t < R0; t++) x[t] = xa[i * R0 + t];
-    } else {
-#pragma unroll
-      for (int t = 0; t < R0; t++) x[t] = lds[slot_step<SUB0>(q, t)];
-    }
-    dit_levels<RB0>(x, a.tl, q, 1);
-#pragma unroll
-    for (int t = 0; t < R0; t++) xa[i * R0 + t] = x[t];
-  }
-}
-
-// Middle pass of a multi-pass plan (in place into a.data), or a whole one-pass
-// product rounded into a.coef when PACK/UNPACK. BPW contiguous blocks per
-// workgroup (each with its own LDS tile): blocks of L < 1024 (1536 for 3 2^k)
-// have fewer than 64 threads, and one block per workgroup would leave most
-// lanes of the wave idle.
-template <int L, bool SQUARE, bool PACK, bool UNPACK, int BPW = 1, int CACHE = 0>
-__global__ __launch_bounds__((Tile<L, 1>::T * BPW)) void k_mid(PassArgs a) {
-  using TC = Tile<L, 1>;
-  static_assert(BPW == 1 || !PACK, "one-pass products take one workgroup each");
+// Middle pass of a multi-pass plan (in place into a.data): last forward pass of
+// A (and B), pointwise product (or square), first inverse pass of one contiguous
+// block of L points (see Row). BPW blocks per workgroup, each with its own LDS
+// tile: short blocks have fewer threads than a wave, or a part of one left over.
+// With eight points a thread B's are loaded together with A's, so they arrive
+// under A's stages (not with 1024 threads, whose 128 registers would spill).
+// Bound by HBM where many blocks are in flight (5.4 TB/s at 2^26 points); 6144
+// points on 64 workgroups 33 -> 22 us against 24 points a thread.
+template <int L, bool SQUARE, int BPW = 1, int CACHE = 0>
+__global__ __launch_bounds__((Row<L, mid_points(L)>::T * BPW)) void k_mid(PassArgs a) {
+  constexpr int E = mid_points(L);
+  using RC = Row<L, E>;
   bind_product(a);
-  __shared__ cd lds_all[TC::LDS_ELEMS * BPW];
-  const int sub = BPW > 1 ? (int)threadIdx.x / TC::T : 0;
-  const int tid = BPW > 1 ? (int)threadIdx.x % TC::T : (int)threadIdx.x;
-  cd *lds = lds_all + sub * TC::LDS_ELEMS;
-  const unsigned long long blk0 = ((unsigned long long)blockIdx.x * BPW + sub) * L;
-  cd xa[TC::EPT];
-  mid_pipeline<L, SQUARE, PACK, CACHE>(a, lds, blk0, xa, tid);
-  constexpr int R0 = 1 << TC::FIRSTB;
-  constexpr int PER0 = TC::EPT / R0;
-  constexpr int SUB0 = L / R0;
-  double worst = 0.0;
+  __shared__ cd lds_all[RC::LDS_ELEMS * BPW];
+  const int sub = BPW > 1 ? (int)threadIdx.x / RC::T : 0;
+  const int tid = BPW > 1 ? (int)threadIdx.x % RC::T : (int)threadIdx.x;
+  cd *lds = lds_all + sub * RC::LDS_ELEMS;
+  const unsigned long long j0 = ((unsigned long long)blockIdx.x * BPW + sub) * L + tid;
+  cd x[E], xa[RC::XR];
 #pragma unroll
-  for (int i = 0; i < PER0; i++) {
-    int q = tid + i * TC::T;
+  for (int h = 0; h < E; h++) x[h] = ld_pol<(CACHE & 1) != 0>(&a.data[j0 + h * RC::T]);
+  if constexpr (!SQUARE) {
+    cd y[E], xb[RC::XR];
+    constexpr bool EARLY = E == 8 && RC::T * BPW < 1024;
+    auto load_b = [&] {
 #pragma unroll
-    for (int t = 0; t < R0; t++) {
-      unsigned long long j = blk0 + (unsigned long long)(q + t * SUB0);
-      if (UNPACK)
-        worst = fmax(worst, unpack_point(a, xa[i * R0 + t], j));
-      else
-        st_pol<(CACHE & 2) != 0>(&a.data[j], xa[i * R0 + t]);
-    }
+      for (int h = 0; h < E; h++) y[h] = ld_pol<(CACHE & 1) != 0>(&a.data_b[j0 + h * RC::T]);
+    };
+    if constexpr (EARLY) load_b();
+    row_forward<L, E>(x, xa, lds, a.tl, tid);
+    if constexpr (!EARLY) load_b();
+    __syncthreads();
+    row_forward<L, E>(y, xb, lds, a.tl, tid);
+#pragma unroll
+    for (int i = 0; i < RC::XR; i++) xa[i] = cmul(xa[i], xb[i]);
+  } else {
+    row_forward<L, E>(x, xa, lds, a.tl, tid);
+#pragma unroll
+    for (int i = 0; i < RC::XR; i++) xa[i] = cmul(xa[i], xa[i]);
   }
-  if (UNPACK) margin_reduce(a.margin, worst, a.margin_mask);
+  row_inverse<L, E>(xa, x, lds, a.tl, tid);
+#pragma unroll
+  for (int h = 0; h < E; h++) st_pol<(CACHE & 2) != 0>(&a.data[j0 + h * RC::T], x[h]);
 }
 
 // ------------------------------------------------------------ carry resolve
@@ -1616,71 +1463,138 @@ struct ClassArgs {
   Roots roots;
   const cd *tl;
   unsigned int *margins;  // per product, float bits of the worst rounding distance
-  int *next;              // work counter, zero at launch
 };
 
-// Persistent workgroups pull products of one length class from a counter and
-// run each product whole: pack, forward, pointwise, inverse, rounding and the
-// carry resolve, with the coefficients never leaving LDS.
+// Values the same in every lane, held in scalar registers.
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long v) {
+  return (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v) |
+         (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32)) << 32;
+}
+template <class T>
+__device__ __forceinline__ T *uniform_ptr(T *p) {
+  return reinterpret_cast<T *>(uniform64(reinterpret_cast<unsigned long long>(p)));
+}
+
+// A product's descriptor, the same for the whole workgroup. The compiler reads
+// it with vector loads (the kernel stores to global memory between products),
+// and a buffer resource made of vector registers costs a loop per load.
+__device__ __forceinline__ MulDesc uniform_desc(const MulDesc &m) {
+  MulDesc d;
+  d.a = uniform_ptr(m.a);
+  d.b = uniform_ptr(m.b);
+  d.c = uniform_ptr(m.c);
+  d.d = uniform_ptr(m.d);
+  d.al = uniform64(m.al);
+  d.bl = uniform64(m.bl);
+  d.cl = uniform64(m.cl);
+  d.dl = uniform64(m.dl);
+  d.bits = __builtin_amdgcn_readfirstlane(m.bits);
+  d.cbits = __builtin_amdgcn_readfirstlane(m.cbits);
+  return d;
+}
+
+// Digits tid + h T of an operand (h < 8) into lo, digits tid + h T + L into up
+// (zero beyond the operand). For 32 | T a lane's digits sit a whole number of
+// words apart, so one bit offset and one byte offset serve all sixteen, read
+// with range-checked buffer loads as in PackDigits; shorter rows go digit by
+// digit.
 template <int L>
-__global__ __launch_bounds__((Tile<L, 1>::T)) void k_mul1(ClassArgs ca) {
-  using TC = Tile<L, 1>;
-  __shared__ cd lds[TC::LDS_ELEMS];
-  __shared__ int job;
-  const int tid = threadIdx.x;
-  constexpr int R0 = 1 << TC::FIRSTB;
-  constexpr int PER0 = TC::EPT / R0;
-  constexpr int SUB0 = L / R0;
-  for (;;) {
-    if (tid == 0) job = atomicAdd(ca.next, 1);
-    __syncthreads();
-    const int idx = job;
-    __syncthreads();
-    if (idx >= ca.count) break;
-    const MulDesc d = ca.desc[idx];
-    PassArgs a;
-    a.data = nullptr;
-    a.data_b = nullptr;
-    a.wa = d.a;
-    a.wb = d.b;
-    a.al = d.al;
-    a.bl = d.bl;
-    a.coef = nullptr;
-    a.N = L;
-    a.M = 1;
-    a.S = L;
-    a.tw_mul = 4;
-    a.tl = ca.tl;
-    a.roots = ca.roots;
-    a.bits = d.bits;
-    a.ntiles = 1;
-    a.margin = nullptr;
-    a.inv_n = 1.0 / (double)L;
-    cd xa[TC::EPT];
-    if (d.a == d.b && d.al == d.bl)
-      mid_pipeline<L, true, true>(a, lds, 0, xa, tid);
-    else
-      mid_pipeline<L, false, true>(a, lds, 0, xa, tid);
-    __syncthreads();  // LDS now becomes the coefficient array
-    long long *coef = (long long *)lds;
-    double worst = 0.0;
+__device__ __forceinline__ void row_digits(const uint32_t *w, unsigned long long wl, int bits, int tid,
+                                           unsigned (&lo)[8], unsigned (&up)[8]) {
+  constexpr int T = Row<L>::T;
+  if constexpr (T % 32 == 0) {
+    const unsigned b = (unsigned)bits, bit = (unsigned)tid * b;
+    const unsigned step = (unsigned)(T / 32) * b * 4u;  // bytes between digits j and j + T
+    const unsigned off = (bit >> 5) * 4u, sh = bit & 31u;
+    const __amdgpu_buffer_rsrc_t w0 = word_rsrc(w, wl), w1 = word_rsrc(w + 1, wl - 1);
 #pragma unroll
-    for (int i = 0; i < PER0; i++) {
-      int q = tid + i * TC::T;
+    for (int h = 0; h < 8; h++) {
+      lo[h] = __builtin_amdgcn_raw_buffer_load_b32(w0, off + (unsigned)h * step, 0, 0);
+      up[h] = __builtin_amdgcn_raw_buffer_load_b32(w0, off + (unsigned)(h + 8) * step, 0, 0);
+    }
+    if ((b & (b - 1u)) == 0u) {  // b <= 32 divides 32: no digit straddles two words
 #pragma unroll
-      for (int t = 0; t < R0; t++) {
-        int j = q + t * SUB0;
-        cd f = cmulc(xa[i * R0 + t], omega_pow(a.roots, (unsigned long long)j));
-        const bool fast = d.cbits <= 51;
-        coef[j] = round_coef(f.x * a.inv_n, fast, worst);
-        coef[j + L] = round_coef(f.y * a.inv_n, fast, worst);
+      for (int h = 0; h < 8; h++) {
+        lo[h] = __builtin_amdgcn_ubfe(lo[h], sh, b);
+        up[h] = __builtin_amdgcn_ubfe(up[h], sh, b);
+      }
+    } else {
+      unsigned lo1[8], up1[8];
+#pragma unroll
+      for (int h = 0; h < 8; h++) {
+        lo1[h] = __builtin_amdgcn_raw_buffer_load_b32(w1, off + (unsigned)h * step, 0, 0);
+        up1[h] = __builtin_amdgcn_raw_buffer_load_b32(w1, off + (unsigned)(h + 8) * step, 0, 0);
+      }
+#pragma unroll
+      for (int h = 0; h < 8; h++) {
+        lo[h] = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(lo1[h], lo[h], sh), 0, b);
+        up[h] = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(up1[h], up[h], sh), 0, b);
       }
     }
-    margin_reduce(ca.margins + idx, worst);
-    __syncthreads();
-    wg_carry<TC::T>(coef, 2 * L, d.bits, d.cbits, d.c, (long long)d.cl, d.d, (long long)d.dl, tid);
-    __syncthreads();
+  } else {
+#pragma unroll
+    for (int h = 0; h < 8; h++) {
+      lo[h] = (unsigned)digit_at(w, wl, (unsigned long long)(tid + h * T), bits);
+      up[h] = (unsigned)digit_at(w, wl, (unsigned long long)(tid + h * T + L), bits);
+    }
   }
+}
+
+// One workgroup per product of a length class runs it whole: pack, forward,
+// pointwise, inverse, rounding and the carry resolve, with the coefficients
+// never leaving LDS. Row tid + h T has the right-angle weight
+// Omega^{tid} e^{2 pi i h / 32} (T = L / 8, N = L): one computed point and
+// eight constants per thread. Bound by LDS exchanges and FP64 issue, with one
+// (8192 points) to sixteen workgroups on a CU. Workgroups that loop over the
+// class's products had the loop's constants and twiddles hoisted into 50 more
+// registers; the products of a class cost the same, so the dispatcher
+// balances them as well.
+template <int L>
+__global__ __launch_bounds__((Row<L>::T)) void k_mul1(ClassArgs ca) {
+  using RC = Row<L>;
+  __shared__ cd lds[RC::LDS_ELEMS];
+  const int tid = threadIdx.x, idx = blockIdx.x;
+  const MulDesc d = uniform_desc(ca.desc[idx]);
+  cd wt = omega_direct(ca.roots, (unsigned long long)tid);
+  const bool square = d.a == d.b && d.al == d.bl;
+  cd x[8], xa[RC::XR];
+  unsigned lo[8], up[8];
+  row_digits<L>(d.a, d.al, d.bits, tid, lo, up);
+#pragma unroll
+  for (int h = 0; h < 8; h++) x[h] = cmul(make_double2((double)lo[h], (double)up[h]), cmul(wt, w64(2 * h)));
+  if (square) {
+    row_forward<L, 8>(x, xa, lds, ca.tl, tid);
+#pragma unroll
+    for (int i = 0; i < RC::XR; i++) xa[i] = cmul(xa[i], xa[i]);
+  } else {
+    cd xb[RC::XR];
+    row_digits<L>(d.b, d.bl, d.bits, tid, lo, up);  // arrive under A's stages
+    row_forward<L, 8>(x, xa, lds, ca.tl, tid);
+    asm volatile("" : "+v"(wt.x), "+v"(wt.y));
+#pragma unroll
+    for (int h = 0; h < 8; h++) x[h] = cmul(make_double2((double)lo[h], (double)up[h]), cmul(wt, w64(2 * h)));
+    __syncthreads();
+    row_forward<L, 8>(x, xb, lds, ca.tl, tid);
+#pragma unroll
+    for (int i = 0; i < RC::XR; i++) xa[i] = cmul(xa[i], xb[i]);
+  }
+  row_inverse<L, 8>(xa, x, lds, ca.tl, tid);
+  __syncthreads();  // LDS now becomes the coefficient array
+  long long *coef = (long long *)lds;
+  const double inv_n = 1.0 / (double)L;
+  double worst = 0.0;
+  const bool fast = d.cbits <= 51;
+  asm volatile("" : "+v"(wt.x), "+v"(wt.y));
+#pragma unroll
+  for (int h = 0; h < 8; h++) {
+    const int j = tid + h * RC::T;
+    const cd f = cmulc(x[h], cmul(wt, w64(2 * h)));
+    coef[j] = round_coef(f.x * inv_n, fast, worst);
+    coef[j + L] = round_coef(f.y * inv_n, fast, worst);
+  }
+  margin_reduce(ca.margins + idx, worst);
+  __syncthreads();
+wg_carry<RC::T>(coef, 2 * L, d.bits, d.cbits, d.c, (long long)d.cl, d.d, (long long)d.dl, tid);
 }
 
 }  // namespace bcg

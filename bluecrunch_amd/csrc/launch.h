@@ -9,8 +9,8 @@ namespace bcg {
 // fwd/inv: (pack-or-unpack, grid.x, grid.y, stream, args) -> 0, or nonzero
 // when the flag is not supported for that tile.
 typedef int (*fwd_fn)(bool, int, int, hipStream_t, const PassArgs &);
-// mid: (square, pack, grid.x, grid.y, stream, args)
-typedef int (*mid_fn)(bool, bool, int, int, hipStream_t, const PassArgs &);
+// mid: (square, grid.x, grid.y, stream, args)
+typedef int (*mid_fn)(bool, int, int, hipStream_t, const PassArgs &);
 typedef int (*mul1_fn)(int, hipStream_t, const ClassArgs &);
 
 // nullptr when no kernel exists for the (L, C) tile.

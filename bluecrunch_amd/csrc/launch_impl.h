@@ -7,6 +7,14 @@ namespace bcg {
 #define BCG_LAUNCH2(kern, gx, gy, block, stream, ...) \
   hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(block), 0, stream, __VA_ARGS__)
 
+// Blocks of L points one workgroup of a middle pass holds: enough to fill whole
+// waves (L / 8 threads each: eight blocks of 64 points make one wave, two of 768
+// three), a power of two because the block counts are.
+constexpr int mid_blocks(int L) {
+  const int wave = 64 * mid_points(L);
+  return L % 3 == 0 ? (L < 1536 ? 1536 / L : 1) : (L < wave ? wave / L : 1);
+}
+
 // Packing/unpacking passes are always the outermost pass, a power of two
 // (the 3 * 2^k factor sits in the innermost pass): the flag is rejected on
 // 3 * 2^k tiles.

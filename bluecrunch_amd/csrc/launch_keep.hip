@@ -26,20 +26,18 @@ int inv_keep(bool unpack, int grid, int gy, hipStream_t s, const PassArgs &a) {
 }
 
 template <int L>
-int mid_keep(bool sq, bool pack, int grid, int gy, hipStream_t s, const PassArgs &a) {
-  constexpr int T = Tile<L, 1>::T;
-  constexpr int BPW = T < 64 ? 64 / T : 1;
-  if (pack) return -2;
+int mid_keep(bool sq, int grid, int gy, hipStream_t s, const PassArgs &a) {
+  constexpr int T = Row<L, mid_points(L)>::T, BPW = mid_blocks(L);
   if (BPW > 1 && grid % BPW == 0) {
     if (sq)
-      BCG_LAUNCH2((k_mid<L, true, false, false, BPW, 3>), grid / BPW, gy, T * BPW, s, a);
+      BCG_LAUNCH2((k_mid<L, true, BPW, 3>), grid / BPW, gy, T * BPW, s, a);
     else
-      BCG_LAUNCH2((k_mid<L, false, false, false, BPW, 3>), grid / BPW, gy, T * BPW, s, a);
+      BCG_LAUNCH2((k_mid<L, false, BPW, 3>), grid / BPW, gy, T * BPW, s, a);
   } else {
     if (sq)
-      BCG_LAUNCH2((k_mid<L, true, false, false, 1, 3>), grid, gy, T, s, a);
+      BCG_LAUNCH2((k_mid<L, true, 1, 3>), grid, gy, T, s, a);
     else
-      BCG_LAUNCH2((k_mid<L, false, false, false, 1, 3>), grid, gy, T, s, a);
+      BCG_LAUNCH2((k_mid<L, false, 1, 3>), grid, gy, T, s, a);
   }
   return 0;
 }
@@ -81,7 +79,7 @@ mid_fn pick_mid_keep(int L) {
 // first launch of one of its kernels, inside a caller's first product.
 int preload_keep() {
   hipFuncAttributes fa;
-  return hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&(k_mid<1024, false, false, false, 1, 3>))) ==
+  return hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&(k_mid<1024, false, 1, 3>))) ==
                  hipSuccess
              ? 0
              : -1;

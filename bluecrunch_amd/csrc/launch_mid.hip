@@ -1,31 +1,23 @@
 // Middle pass kernels (last forward pass + pointwise product + first inverse
-// pass, or a whole one-pass product), every length class.
+// pass), every length class.
 #include "launch_impl.h"
 
 namespace bcg {
 
-// grid = number of contiguous blocks of L points (1 for a one-pass product).
-// Middle passes with blocks of fewer than 64 threads put BPW = 64 / T blocks
-// in one workgroup (one full wave) when the block count allows it.
+// grid = number of contiguous blocks of L points.
 template <int L>
-int launch_mid(bool sq, bool pack, int grid, int gy, hipStream_t s, const PassArgs &a) {
-  constexpr int T = Tile<L, 1>::T;
-  constexpr int BPW = T < 64 ? 64 / T : 1;
-  if (pack) {
+int launch_mid(bool sq, int grid, int gy, hipStream_t s, const PassArgs &a) {
+  constexpr int T = Row<L, mid_points(L)>::T, BPW = mid_blocks(L);
+  if (BPW > 1 && grid % BPW == 0) {
     if (sq)
-      BCG_LAUNCH2((k_mid<L, true, true, true>), grid, gy, T, s, a);
+      BCG_LAUNCH2((k_mid<L, true, BPW>), grid / BPW, gy, T * BPW, s, a);
     else
-      BCG_LAUNCH2((k_mid<L, false, true, true>), grid, gy, T, s, a);
-  } else if (BPW > 1 && grid % BPW == 0) {
-    if (sq)
-      BCG_LAUNCH2((k_mid<L, true, false, false, BPW>), grid / BPW, gy, T * BPW, s, a);
-    else
-      BCG_LAUNCH2((k_mid<L, false, false, false, BPW>), grid / BPW, gy, T * BPW, s, a);
+      BCG_LAUNCH2((k_mid<L, false, BPW>), grid / BPW, gy, T * BPW, s, a);
   } else {
     if (sq)
-      BCG_LAUNCH2((k_mid<L, true, false, false>), grid, gy, T, s, a);
+      BCG_LAUNCH2((k_mid<L, true>), grid, gy, T, s, a);
     else
-      BCG_LAUNCH2((k_mid<L, false, false, false>), grid, gy, T, s, a);
+      BCG_LAUNCH2((k_mid<L, false>), grid, gy, T, s, a);
   }
   return 0;
 }
@@ -55,7 +47,7 @@ mid_fn pick_mid(int L) {
 // first launch of one of its kernels, inside a caller's first product.
 int preload_mid() {
   hipFuncAttributes fa;
-  return hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&(k_mid<1024, false, false, false>))) == hipSuccess ? 0 : -1;
+  return hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&(k_mid<1024, false>))) == hipSuccess ? 0 : -1;
 }
 
 }  // namespace bcg

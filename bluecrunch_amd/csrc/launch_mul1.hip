@@ -1,11 +1,11 @@
-// One-workgroup product kernels (persistent, one length class per launch).
+// One-workgroup product kernels, one length class per launch.
 #include "launch_impl.h"
 
 namespace bcg {
 
 template <int L>
 int launch_mul1(int grid, hipStream_t s, const ClassArgs &ca) {
-  hipLaunchKernelGGL((k_mul1<L>), dim3(grid), dim3(Tile<L, 1>::T), 0, s, ca);
+  hipLaunchKernelGGL((k_mul1<L>), dim3(grid), dim3(Row<L>::T), 0, s, ca);
   return 0;
 }
 

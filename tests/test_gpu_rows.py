@@ -1,0 +1,70 @@
+"""One workgroup per contiguous block of points: every one-pass product length
+(64 to 8192 points, 2^k and 3 * 2^k) at the longest and the shortest operands
+of its class, ragged pairs, squares and operands of all ones, and every middle
+pass length in a two-pass split, each product exact."""
+import numpy as np
+import pytest
+
+from helpers import exact_product
+from bluecrunch_amd.workload import operands
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [64, 96, 128, 192, 256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192]
+
+
+def _pairs(bc, n):
+    """(al, bl) on both edges of the class of n points, balanced and 1 to 3."""
+    out = []
+    for num in (2, 4):  # bl = al, bl = al / 3
+        on = [t for t in range(100, 2 * n) if bc.plan(t - t // num, t // num)["points"] == n]
+        if on:
+            out += [(t - t // num, t // num) for t in (on[0], on[-1])]
+    return out
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_one_pass_lengths(bc, n):
+    pairs = _pairs(bc, n)
+    if not pairs:
+        pytest.skip("no product of at least 100 words has this length")
+    for al, bl in pairs:
+        a, b = operands(al * 31 + bl, al, bl)
+        c, info = bc.mul(a, b)
+        assert (info["points"], info["passes"]) == (n, 1)
+        assert np.array_equal(c, exact_product(a, b)), (al, bl)
+        s, sinfo = bc.mul(a, a)
+        assert np.array_equal(s, exact_product(a, a)), (al, sinfo)
+        ones = np.full(al, 0xFFFFFFFF, dtype=np.uint32)
+        m, _ = bc.mul(ones, b)
+        assert np.array_equal(m, exact_product(ones, b)), (al, bl)
+    out, worst = bc.mul_batch([operands(k, al, bl) for k, (al, bl) in enumerate(pairs * 3)])
+    for k, (c, (al, bl)) in enumerate(zip(out, pairs * 3)):
+        assert np.array_equal(c, exact_product(*operands(k, al, bl))), (al, bl)
+    assert worst < 0.25
+
+
+@pytest.mark.parametrize("inner", [x for x in LENGTHS if x >= 128])
+def test_middle_pass_lengths(bc, inner):
+    n = 64 * inner
+    if n < 12288:
+        pytest.skip("shorter lengths run as one pass")
+    lo, hi = 100, n
+    while hi - lo > 1:  # the longest balanced product of n points
+        mid = (lo + hi) // 2
+        lo, hi = (mid, hi) if bc.plan(mid, mid)["points"] <= n else (lo, mid)
+    assert bc.plan(lo, lo)["points"] == n
+    a, b = operands(inner, lo, lo - 7)
+    want = exact_product(a, b), exact_product(a, a)
+    cands = bc.plan_candidates(n)
+    picks = [i for i, (P, L, C) in enumerate(cands) if P == 2 and L == [64, inner]]
+    assert picks
+    try:
+        for i in picks:
+            bc.plan_force(n, i)
+            c, info = bc.mul(a, b)
+            assert info["passes"] == 2 and np.array_equal(c, want[0]), cands[i]
+            s, _ = bc.mul(a, a)
+            assert np.array_equal(s, want[1]), cands[i]
+    finally:
+        bc.plan_force(n, -1)
