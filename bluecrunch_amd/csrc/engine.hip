@@ -53,7 +53,9 @@ struct Engine {
   hipEvent_t fork_ev = nullptr, join_ev[NAUX] = {nullptr, nullptr, nullptr};
   std::map<unsigned long long, RootsDev> roots;  // keyed by N
   std::map<int, cd *> ltab;                      // e^{2 pi i t/L}, keyed by L
-  DevBuf bufA, bufB, wA, wB, wC, blk, margin, zbuf, desc, counters;
+  DevBuf bufA, bufB, wA, wB, wC, blk, margin, zbuf, counters;
+  HostResult *hres = nullptr;      // pinned: what the kernels of a product leave for the host
+  HostResult *hres_dev = nullptr;  // its device address
   bool prof = false;
   std::vector<Pending> pending;
   std::vector<hipEvent_t> free_events;
@@ -279,6 +281,8 @@ int init_locked(int device) {
   g.device = device;
   g.ready = true;
   if (int rc = ensure(g.margin, sizeof(unsigned int) * MARGIN_SLOTS * MARGIN_STRIDE)) return rc;
+  HIPCHK(hipHostMalloc((void **)&g.hres, sizeof(HostResult), hipHostMallocMapped));
+  HIPCHK(hipHostGetDevicePointer((void **)&g.hres_dev, g.hres, 0));
   // every kernel family's code object now rather than inside a first product
   // (a failure here only defers the load to the first launch)
   for (auto f : {preload_mul1, preload_fwd_pow2, preload_fwd_three, preload_inv_pow2, preload_inv_three, preload_mid,
@@ -784,10 +788,44 @@ int pass_args(const Plan &p, int i, PassArgs &a) {
   return 0;
 }
 
-// Carry resolve: coefficients -> CL words.
+// The open blocks of a carry (k_carry_ripple): always launched where the host
+// does not read the product's result right after.
+void launch_ripple(const CarryArgs &c, int count, hipStream_t s) {
+  LAUNCH2(k_carry_ripple, (unsigned)((c.nblk + RIPPLE_BLOCKS - 1) / RIPPLE_BLOCKS), (unsigned)count, RIPPLE_BLOCKS, s,
+          c);
+}
+
+// Ends a carry launched with c: without a host read-back the ripple follows on
+// the stream; with one, the host waits, and launches it only if a block asked
+// for it. *margin (with host) receives the product's margin.
+int end_carry(const CarryArgs &c, hipStream_t s, double *margin) {
+  if (!c.host) {
+    ProfScope ps(BCG_K_CARRY, s);
+    launch_ripple(c, 1, s);
+    HIPCHK(hipGetLastError());
+    return 0;
+  }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(s));
+  float f;
+  memcpy(&f, &g.hres->margin, sizeof f);
+  *margin = (double)f;
+  if (f < 0.25f && g.hres->open_carry) {
+    {
+      ProfScope ps(BCG_K_CARRY, s);
+      launch_ripple(c, 1, s);
+    }
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s));
+  }
+  return 0;
+}
+
+// Carry resolve: coefficients -> CL words. With margin the host waits for the
+// result and takes the worst slot of g.margin there.
 int run_carry(const long long *coef, unsigned long long ncoef, int bits, int cbits, uint32_t *out,
               unsigned long long CL, hipStream_t s, const uint32_t *add = nullptr, unsigned long long addl = 0,
-              unsigned cM = 0, unsigned crows = 0) {
+              unsigned cM = 0, unsigned crows = 0, double *margin = nullptr) {
   if (CL == 0) return 0;
   const unsigned long long wpb = (unsigned long long)CT * CWPT;
   unsigned long long nblk = (CL + wpb - 1) / wpb;
@@ -809,27 +847,53 @@ int run_carry(const long long *coef, unsigned long long ncoef, int bits, int cbi
   c.crows = crows;
   c.wpb = (unsigned)wpb;
   c.lds_slots = carry_slots(bits, cbits);
+  if (margin) {
+    c.host = g.hres_dev;
+    c.margin = (const unsigned int *)g.margin.p;
+    g.hres->open_carry = 0;
+  }
   {
     ProfScope ps(BCG_K_CARRY, s);
     hipLaunchKernelGGL(k_carry_local, dim3((unsigned)nblk), dim3(CT), c.lds_slots * sizeof(long long), s, c);
-    LAUNCH(k_carry_fix, 1, 1024, s, c);
-    LAUNCH(k_carry_apply, (unsigned)nblk, 256, s, c);
   }
-  HIPCHK(hipGetLastError());
-  return 0;
+  return end_carry(c, s, margin);
+}
+
+// Dynamic LDS of k_carry_groups: the group sums under one block's words and the
+// two words below, G digits of `bits` bits each, stride gks words, one pad word
+// per 32.
+size_t group_lds(int G, int bits, int gks) {
+  const size_t w = ((size_t)(32 * GCT * GWPT) / (size_t)(G * bits) + CARRY_GCOV + 4) * (size_t)gks;
+  return (w + w / 32 + 4) * 4;
+}
+
+// Group sums that cover one word: ceil(K / (G b / 32)) when group starts are
+// word-aligned, else the bound of group_words.
+int group_cover(int G, int bits, int K) {
+  const int gb = G * bits;
+  return gb % 32 == 0 ? (K + gb / 32 - 1) / (gb / 32) : (32 * K + gb - 1) / gb + 1;
+}
+
+void launch_carry_groups(const CarryArgs &c, int gcov, dim3 grid, size_t lds, hipStream_t s) {
+  if (gcov <= 2)
+    hipLaunchKernelGGL(k_carry_groups<2>, grid, dim3(GCT), lds, s, c);
+  else if (gcov == 3)
+    hipLaunchKernelGGL(k_carry_groups<3>, grid, dim3(GCT), lds, s, c);
+  else
+    hipLaunchKernelGGL(k_carry_groups<CARRY_GCOV>, grid, dim3(GCT), lds, s, c);
 }
 
 // Carry resolve of plan p's last pass output (group sums or coefficients in
-// bufB) into CL words (+ addend D).
+// bufB) into CL words (+ addend D), as run_carry.
 int group_words(const Plan &p);
 int group_stride(int K);
 bool coef_transposed(const Plan &p);
 int carry_of_plan(const Plan &p, uint32_t *out, unsigned long long CL, hipStream_t s, const uint32_t *add,
-                  unsigned long long addl) {
+                  unsigned long long addl, double *margin) {
   const int K = group_words(p);
   if (!K)
     return run_carry((const long long *)g.bufB.p, 2 * p.N, p.bits, coef_bits(p), out, CL, s, add, addl,
-                     coef_transposed(p) ? (unsigned)p.M[0] : 0u, 2u * (unsigned)p.L[0]);
+                     coef_transposed(p) ? (unsigned)p.M[0] : 0u, 2u * (unsigned)p.L[0], margin);
   if (CL == 0) return 0;
   const unsigned long long wpb = (unsigned long long)GCT * GWPT;
   unsigned long long nblk = (CL + wpb - 1) / wpb;
@@ -851,26 +915,16 @@ int carry_of_plan(const Plan &p, uint32_t *out, unsigned long long CL, hipStream
   c.ng = (long long)(c.ncoef / (unsigned long long)c.gC);
   c.gK = K;
   c.gKs = group_stride(K);
-  // LDS: the groups under one block's GCT * GWPT words
-  size_t glds = ((size_t)(32 * GCT * GWPT) / (size_t)(p.C[0] * p.bits) + CARRY_GCOV + 2) * c.gKs;
-  glds = (glds + glds / 32 + 4) * 4;  // one pad word per 32
+  if (margin) {
+    c.host = g.hres_dev;
+    c.margin = (const unsigned int *)g.margin.p;
+    g.hres->open_carry = 0;
+  }
   {
     ProfScope ps(BCG_K_CARRY, s);
-    // groups covering one word: ceil(K / (G b / 32)) when group starts are
-    // word-aligned, else the bound of group_words
-    const int gb = p.C[0] * p.bits;
-    const int gcov = gb % 32 == 0 ? (K + gb / 32 - 1) / (gb / 32) : (32 * K + gb - 1) / gb + 1;
-    if (gcov <= 2)
-      hipLaunchKernelGGL(k_carry_groups<2>, dim3((unsigned)nblk), dim3(GCT), glds, s, c);
-    else if (gcov == 3)
-      hipLaunchKernelGGL(k_carry_groups<3>, dim3((unsigned)nblk), dim3(GCT), glds, s, c);
-    else
-      hipLaunchKernelGGL(k_carry_groups<CARRY_GCOV>, dim3((unsigned)nblk), dim3(GCT), glds, s, c);
-    LAUNCH(k_carry_fix, 1, 1024, s, c);
-    LAUNCH(k_carry_apply, (unsigned)nblk, 256, s, c);
+    launch_carry_groups(c, group_cover(p.C[0], p.bits, K), dim3((unsigned)nblk), group_lds(p.C[0], p.bits, c.gKs), s);
   }
-  HIPCHK(hipGetLastError());
-  return 0;
+  return end_carry(c, s, margin);
 }
 
 int zero_margin(hipStream_t s) {
@@ -900,17 +954,14 @@ struct DeferScope {
 };
 DeferScope g_defer;
 
+// The margin of a product whose carry has not run (products in place): the
+// host waits for it.
 int read_margin(hipStream_t s, double *m) {
-  if (g_defer.in_product) {  // read with the scope's other sets later
-    *m = 0.0;
-    return 0;
-  }
-  unsigned int slots[MARGIN_SLOTS * MARGIN_STRIDE];
-  if (int rc = d2h(slots, g.margin.p, sizeof slots, s)) return rc;
-  unsigned int bits = 0;
-  for (int i = 0; i < MARGIN_SLOTS; i++) bits = slots[i * MARGIN_STRIDE] > bits ? slots[i * MARGIN_STRIDE] : bits;
+  LAUNCH(k_margin_out, 1, 64, s, (const unsigned int *)g.margin.p, g.hres_dev);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(s));
   float f;
-  memcpy(&f, &bits, sizeof f);
+  memcpy(&f, &g.hres->margin, sizeof f);
   *m = (double)f;
   return 0;
 }
@@ -1053,7 +1104,6 @@ int run_transforms(const Plan &p, const uint32_t *A, unsigned long long AL, cons
   cd *da = (cd *)g.bufA.p;
   cd *db = (cd *)g.bufB.p;
   long long *coef = (long long *)g.bufB.p;
-  if (int rc = zero_margin(s)) return rc;
   PassArgs a;
   memset(&a, 0, sizeof a);
   a.wa = A;
@@ -1209,15 +1259,11 @@ int fill_zero(uint32_t *C, size_t CL, hipStream_t s) {
   return 0;
 }
 
-// Launch the one-pass products desc[first .. first+count) of length class L
-// (descriptors and margin slots already on the device).
-int run_class(int L, const MulDesc *ddesc, int count, unsigned int *dmargins, hipStream_t s) {
-  ClassArgs ca;
-  ca.desc = ddesc;
-  ca.count = count;
+// Launch one-pass products of length class L: `count` descriptors on the device,
+// or the one product in ca.one; margins (and clear) set by the caller.
+int run_class(int L, ClassArgs &ca, int count, hipStream_t s) {
   if (int rc = get_roots((unsigned long long)L, &ca.roots)) return rc;
   if (int rc = get_ltab(L, &ca.tl)) return rc;
-  ca.margins = dmargins;
   mul1_fn f = pick_mul1(L);
   if (!f) return fail(BCG_E_ARG, "no one-pass kernel for this length");
   ProfScope ps(BCG_K_MID, s);
@@ -1226,11 +1272,16 @@ int run_class(int L, const MulDesc *ddesc, int count, unsigned int *dmargins, hi
   return 0;
 }
 
-// One product whose plan is a single pass: the whole product in one workgroup.
+// One product whose plan is a single pass: the whole product in one workgroup
+// and one launch, which carries the descriptor and leaves the margin in host
+// memory (a descriptor copy, two fill kernels and a margin copy around it were
+// 20 of 51 us at 2048 points).
 int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL,
                 hipStream_t s, double *margin, const uint32_t *D = nullptr, size_t DL = 0) {
-  if (int rc = ensure(g.desc, sizeof(MulDesc))) return rc;
-  MulDesc d;
+  const bool deferred = g_defer.in_product;
+  ClassArgs ca;
+  memset(&ca, 0, sizeof ca);
+  MulDesc &d = ca.one;
   d.a = A;
   d.b = B;
   d.c = C;
@@ -1241,10 +1292,16 @@ int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t
   d.dl = D ? DL : 0;
   d.bits = p.bits;
   d.cbits = coef_bits(p);
-  if (int rc = h2d(g.desc.p, &d, sizeof d, s)) return rc;
-  if (int rc = zero_margin(s)) return rc;
-  if (int rc = run_class(p.L[0], (const MulDesc *)g.desc.p, 1, (unsigned int *)g.margin.p, s)) return rc;
-  return read_margin(s, margin);
+  ca.margins = deferred ? (unsigned int *)g.margin.p : &g.hres_dev->margin;
+  ca.clear = deferred ? 1 : 0;
+  if (int rc = run_class(p.L[0], ca, 1, s)) return rc;
+  *margin = 0.0;
+  if (deferred) return 0;  // read with the scope's other sets later
+  HIPCHK(hipStreamSynchronize(s));
+  float f;
+  memcpy(&f, &g.hres->margin, sizeof f);
+  *margin = (double)f;
+  return 0;
 }
 
 // Batched multi-pass products of one plan (same N and pass split): every pass
@@ -1322,9 +1379,7 @@ int run_multipass_class(const Plan &p, const MulDesc *ddesc, const std::vector<M
     if (!d.gk) groups = false;
     gks = std::max(gks, group_stride(d.gk));
     bmin = std::min(bmin, d.bits);
-    const int gb = p.C[0] * d.bits;
-    const int cv = gb % 32 == 0 ? (d.gk + gb / 32 - 1) / (gb / 32) : (32 * d.gk + gb - 1) / gb + 1;
-    gcov = std::max(gcov, cv);
+    gcov = std::max(gcov, group_cover(p.C[0], d.bits, d.gk));
   }
   const unsigned long long ng = groups ? 2 * p.N / (unsigned long long)p.C[0] : 0;
   const unsigned long long ystride = ng * (unsigned long long)gks;
@@ -1382,25 +1437,14 @@ int run_multipass_class(const Plan &p, const MulDesc *ddesc, const std::vector<M
     c.ng = (long long)ng;
     c.gK = gks;  // per product from its descriptor
     c.gKs = gks;
-    // LDS: the groups under one block's GCT * GWPT words at the smallest digit size
-    size_t glds = ((size_t)(32 * GCT * GWPT) / (size_t)(p.C[0] * bmin) + CARRY_GCOV + 2) * (size_t)gks;
-    glds = (glds + glds / 32 + 4) * 4;  // one pad word per 32
     ProfScope ps(BCG_K_CARRY, s);
-    const dim3 grid((unsigned)nblk_max, (unsigned)count);
-    if (gcov <= 2)
-      hipLaunchKernelGGL(k_carry_groups<2>, grid, dim3(GCT), glds, s, c);
-    else if (gcov == 3)
-      hipLaunchKernelGGL(k_carry_groups<3>, grid, dim3(GCT), glds, s, c);
-    else
-      hipLaunchKernelGGL(k_carry_groups<CARRY_GCOV>, grid, dim3(GCT), glds, s, c);
-    LAUNCH(k_carry_fix, count, 1024, s, c);
-    LAUNCH2(k_carry_apply, (unsigned)nblk_max, (unsigned)count, 256, s, c);
+    launch_carry_groups(c, gcov, dim3((unsigned)nblk_max, (unsigned)count), group_lds(p.C[0], bmin, gks), s);
+    launch_ripple(c, count, s);
   } else {
     ProfScope ps(BCG_K_CARRY, s);
     hipLaunchKernelGGL(k_carry_local, dim3((unsigned)nblk_max, (unsigned)count), dim3(CT),
                        c.lds_slots * sizeof(long long), s, c);
-    LAUNCH(k_carry_fix, count, 1024, s, c);
-    LAUNCH2(k_carry_apply, (unsigned)nblk_max, (unsigned)count, 256, s, c);
+    launch_ripple(c, count, s);
   }
   HIPCHK(hipGetLastError());
   return 0;
@@ -1512,10 +1556,9 @@ int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
     if (alias) {
       // the carry pass overwrites the inputs: check the margin first
       if (int rc = read_margin(s, &m)) return rc;
-    }
-    if (!alias) {
-      if (int rc = carry_of_plan(p, C, CL, s, D, DL)) return rc;
-      if (int rc = read_margin(s, &m)) return rc;
+    } else {
+      // a deferred product's margin is read with its scope's other sets later
+      if (int rc = carry_of_plan(p, C, CL, s, D, DL, g_defer.in_product ? nullptr : &m)) return rc;
     }
     inf.bits = p.bits;
     inf.passes = p.P;
@@ -1540,7 +1583,7 @@ int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
       continue;
     }
     if (alias) {
-      if (int rc = carry_of_plan(p, C, CL, s, D, DL)) return rc;
+      if (int rc = carry_of_plan(p, C, CL, s, D, DL, nullptr)) return rc;
     }
     break;
   }
@@ -1820,16 +1863,15 @@ namespace {
 // Scratch of bcg_mul_dev_noalloc: the engine's per-product buffers as fixed
 // slices of one static device array, for products whose transform has at
 // most NOALLOC_MAX_POINTS points: two transform arrays (16 bytes a point),
-// the margin slots, carry block functions, one product descriptor, counters,
+// the margin slots, carry block functions, counters,
 // and the staging of an aliased output (one-pass and schoolbook products).
 constexpr unsigned long long NOALLOC_MAX_POINTS = 1ull << 20;
 constexpr size_t NA_ARR = (size_t)NOALLOC_MAX_POINTS * sizeof(cd);
 constexpr size_t NA_MARGIN = (size_t)MARGIN_SLOTS * MARGIN_STRIDE * sizeof(unsigned int);
 constexpr size_t NA_BLK = (size_t)64 << 10;
-constexpr size_t NA_DESC = 256;
 constexpr size_t NA_COUNTERS = 256;
 constexpr size_t NA_ZBUF = (size_t)64 << 10;
-constexpr size_t NA_BYTES = 2 * NA_ARR + NA_MARGIN + NA_BLK + NA_DESC + NA_COUNTERS + NA_ZBUF;
+constexpr size_t NA_BYTES = 2 * NA_ARR + NA_MARGIN + NA_BLK + NA_COUNTERS + NA_ZBUF;
 
 }  // namespace
 
@@ -1872,12 +1914,12 @@ int prepare_noalloc() {
 // The engine's buffers pointed at the scratch for one call (under the engine
 // lock), restored afterwards.
 struct ScratchScope {
-  DevBuf *bufs[7] = {&g.bufA, &g.bufB, &g.margin, &g.blk, &g.desc, &g.counters, &g.zbuf};
-  DevBuf saved[7];
+  DevBuf *bufs[6] = {&g.bufA, &g.bufB, &g.margin, &g.blk, &g.counters, &g.zbuf};
+  DevBuf saved[6];
   explicit ScratchScope(unsigned char *base) {
-    const size_t sizes[7] = {NA_ARR, NA_ARR, NA_MARGIN, NA_BLK, NA_DESC, NA_COUNTERS, NA_ZBUF};
+    const size_t sizes[6] = {NA_ARR, NA_ARR, NA_MARGIN, NA_BLK, NA_COUNTERS, NA_ZBUF};
     size_t off = 0;
-    for (int i = 0; i < 7; i++) {
+    for (int i = 0; i < 6; i++) {
       saved[i] = *bufs[i];
       bufs[i]->p = base + off;
       bufs[i]->bytes = sizes[i];
@@ -1886,7 +1928,7 @@ struct ScratchScope {
     g_fixed = true;
   }
   ~ScratchScope() {
-    for (int i = 0; i < 7; i++) *bufs[i] = saved[i];
+    for (int i = 0; i < 6; i++) *bufs[i] = saved[i];
     g_fixed = false;
   }
 };
@@ -1908,7 +1950,7 @@ int bcg_shutdown(void) {
   (void)hipStreamSynchronize(g.stream);
   g_defer.open = false;
   g_defer.n = 0;
-  for (DevBuf *b : {&g.bufA, &g.bufB, &g.wA, &g.wB, &g.wC, &g.blk, &g.margin, &g.zbuf, &g.desc, &g.counters,
+  for (DevBuf *b : {&g.bufA, &g.bufB, &g.wA, &g.wB, &g.wC, &g.blk, &g.margin, &g.zbuf, &g.counters,
                     &g_defer.sets}) {
     if (b->p) (void)hipFree(b->p);
     b->p = nullptr;
@@ -1936,6 +1978,8 @@ int bcg_shutdown(void) {
   (void)hipStreamDestroy(g.cap);
   g_bb.release();
   ep_trim();
+  if (g.hres) (void)hipHostFree(g.hres);
+  g.hres = g.hres_dev = nullptr;
   if (g_ring.p) (void)hipHostFree(g_ring.p);
   for (auto &e : g_ring.ev)
     if (e) (void)hipEventDestroy(e);
@@ -2231,7 +2275,6 @@ int batch_upload(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
 int batch_launch(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
   const size_t nm = bp.mdesc.size(), nc = bp.cdesc.size();
   unsigned int *mm = (unsigned int *)bb.margins.p, *cm = mm + nm;
-  if (nm + nc) LAUNCH(k_zero_u32, (int)((nm + nc + 255) / 256), 256, s, mm, (int)(nm + nc));
   HIPCHK(hipGetLastError());
   // one-pass length classes: independent persistent launches, spread over the
   // side streams (largest class first), beside the multi-pass groups on s, so
@@ -2264,7 +2307,11 @@ int batch_launch(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
       const int ci = order[k];
       const auto &gr = bp.cgroups[ci];
       const size_t first = gr.second.first, n = gr.second.second;
-      rc = run_class(gr.first, (const MulDesc *)bb.cdesc.p + first, (int)n, cm + first, g.aux[k % Engine::NAUX]);
+      ClassArgs ca;
+      memset(&ca, 0, sizeof ca);
+      ca.desc = (const MulDesc *)bb.cdesc.p + first;
+      ca.margins = cm + first;
+      rc = run_class(gr.first, ca, (int)n, g.aux[k % Engine::NAUX]);
     }
   }
   if (!rc && !bp.tiny.empty()) {
@@ -2479,9 +2526,8 @@ int bcg_fft_to_int_dev(const double *z, size_t length, uint32_t *A, size_t AL, i
          (unsigned int *)g.margin.p);
   HIPCHK(hipGetLastError());
   // r_k are < 2^53; bound the coefficient width by the largest possible value
-  if (int rc = run_carry((const long long *)g.zbuf.p, pts, bits, 63, A, AL, s)) return rc;
   double m = 0;
-  if (int rc = read_margin(s, &m)) return rc;
+  if (int rc = run_carry((const long long *)g.zbuf.p, pts, bits, 63, A, AL, s, nullptr, 0, 0, 0, &m)) return rc;
   if (margin) *margin = m;
   return 0;
 }

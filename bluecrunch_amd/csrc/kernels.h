@@ -33,7 +33,7 @@ struct PassArgs {
   Roots roots;
   int bits;                 // digit size
   int ntiles;
-  unsigned int *margin;     // float bits of the worst |x - round(x)| (atomic max)
+  unsigned int *margin;     // float bits of the worst |x - round(x)| (atomic max; zeroed by the packing pass)
   int margin_mask;          // single products: slot (block & mask) * MARGIN_STRIDE; batched: 0
   double inv_n;
   int fast_round;           // every coefficient < 2^51: round with the 1.5 * 2^52 addition
@@ -79,7 +79,7 @@ __device__ __forceinline__ void bind_product(PassArgs &a) {
   if (a.data_b) a.data_b += p * a.N;
   if (a.coef) a.coef += p * 2 * a.N;
   if (a.ybuf) a.ybuf += p * a.ystride;
-  if (a.margin) a.margin += p;
+  if (a.margin) a.margin += p;  // margin_mask 0: one slot (both operands' packing rows clear the same one)
 }
 
 // Tile order that keeps adjacent column tiles on one XCD at the same time:
@@ -252,8 +252,8 @@ __device__ __forceinline__ void write_group_half(const PassArgs &a, long long *l
 
 // Margin slots: a single product spreads its atomics over MARGIN_SLOTS
 // addresses MARGIN_STRIDE words apart (one 128-byte line each), so tens of
-// thousands of workgroups do not serialise on one address; the host takes the
-// maximum over the slots.
+// thousands of workgroups do not serialise on one address; the carry takes the
+// maximum over the slots (margin_of_slots) to host memory.
 constexpr int MARGIN_SLOTS = 64;
 constexpr int MARGIN_STRIDE = 32;
 
@@ -262,6 +262,34 @@ __device__ __forceinline__ void margin_reduce(unsigned int *m, double d, int mas
   float f = (float)d;
   for (int off = 32; off > 0; off >>= 1) f = fmaxf(f, __shfl_xor(f, off, 64));
   if ((threadIdx.x & 63) == 0) atomicMax(m + (blockIdx.x & mask) * MARGIN_STRIDE, __float_as_uint(f));
+}
+
+// The packing pass of a product zeroes its margin slots (the unpacking pass,
+// later on the same stream, raises them): a fill kernel of its own is a launch.
+__device__ __forceinline__ void margin_clear(const PassArgs &a) {
+  if (blockIdx.x != 0) return;
+  for (int i = threadIdx.x; i <= a.margin_mask; i += blockDim.x) a.margin[i * MARGIN_STRIDE] = 0u;
+}
+
+// First wave: the largest slot, on every lane.
+__device__ __forceinline__ unsigned margin_of_slots(const unsigned int *m) {
+  unsigned v = m[(threadIdx.x & 63) * MARGIN_STRIDE];  // non-negative floats order like their bit patterns
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned o = __shfl_xor(v, off, 64);
+    v = o > v ? o : v;
+  }
+  return v;
+}
+
+// What the host reads after a product, in host memory the kernels write: the
+// worst rounding distance (float bits) and whether a carry block's carry-in is
+// still open (see k_carry_groups).
+struct HostResult {
+  unsigned margin;
+  unsigned open_carry;
+};
+__device__ __forceinline__ void host_store(unsigned *p, unsigned v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ------------------------------------------------------------ forward pass
@@ -447,6 +475,9 @@ __global__ __launch_bounds__((Tile<L, C>::T)) void k_fwd(PassArgs a) {
   const unsigned long long m = m0 + c;
   // PACK: digit pairs (a_j, a_{j+N}) of rows r0 + h L/16 and the right-angle
   // weight Omega^{row M + m} = Omega^{r0 M + m} e^{2 pi i h / 64}
+  if constexpr (PACK) {
+    if (a.margin) margin_clear(a);
+  }
   unsigned dre[PACK ? 16 : 1], dim_[PACK ? 16 : 1];
   cd wpack = make_double2(1.0, 0.0);
   cd tb0[4];  // split tile: stage-0 level twiddles, loaded ahead of the digits
@@ -777,6 +808,8 @@ struct CarryArgs {
   long long ng;              // groups: ncoef / gC
   unsigned wpb;              // words per carry block
   unsigned long long ystride;  // batched group mode: group-sum words per product
+  HostResult *host;            // nullptr, or where block 0 leaves the margin and open blocks their flag
+  const unsigned int *margin;  // margin slots of the product (with host)
 };
 
 __device__ __forceinline__ long long coef_at(const CarryArgs &a, long long j) {
@@ -838,14 +871,14 @@ __device__ __forceinline__ void bind_carry(CarryArgs &a, unsigned long long p) {
   a.nblk = (d.cl + a.wpb - 1) / a.wpb;
 }
 
-// Coefficient window of one carry block in LDS: words [W0, W0 + CT*CWPT) need
-// coefficients j with b j in (32 (W0-1) - cbits, 32 (W0 + CT*CWPT)); the
+// Coefficient window of one carry block in LDS: words [W0 - 2, W0 + CT*CWPT) need
+// coefficients j with b j in (32 (W0-2) - cbits, 32 (W0 + CT*CWPT)); the
 // window is sized per launch (dynamic LDS) from the smallest digit size.
 // 0 (no staging: coefficients are read from global memory) when the window
 // would exceed CARRY_LDS_MAX slots (digit sizes below 4 bits).
 constexpr unsigned CARRY_LDS_MAX = 8256;
 __host__ __device__ inline unsigned carry_slots(int bits, int cbits) {
-  unsigned n = (unsigned)((32ull * CT * CWPT + (unsigned long long)cbits + 64) / (unsigned long long)bits + 4);
+  unsigned n = (unsigned)((32ull * CT * CWPT + (unsigned long long)cbits + 96) / (unsigned long long)bits + 4);
   return n <= CARRY_LDS_MAX ? n : 0u;
 }
 
@@ -887,21 +920,47 @@ __device__ __forceinline__ unsigned long long partial_rel(const long long *win, 
   return P;
 }
 
+// The carry into a block of words: v_w = lo(P_w) + hi(P_{w-1}) < 2^33 carries
+// v >> 32 out of word w = W0 - 1 whatever comes into it, unless its low word is
+// all ones (a chance of 2^-32 for ordinary digits): then the carry-in is open, the
+// block is written as for 0 and marked (bit 2 of its function) for
+// k_carry_ripple. So almost every block finishes by itself, from two words of its
+// predecessor's range; scanning all blocks' functions in a second kernel and
+// incrementing in a third cost 6 to 10 us per product.
+struct BlockCarry {
+  unsigned cin;   // carry into the block's first word (0 when open)
+  unsigned open;
+};
+__device__ __forceinline__ BlockCarry block_carry(unsigned long long Pm1, unsigned long long Pm2) {
+  const unsigned long long v = (Pm1 & 0xffffffffull) + (Pm2 >> 32);
+  BlockCarry c;
+  c.open = (unsigned)v == 0xffffffffu ? 1u : 0u;
+  c.cin = (unsigned)(v >> 32);
+  return c;
+}
+
+// A block's function and mark, and the host's flag when its carry-in is open.
+__device__ __forceinline__ void carry_publish(const CarryArgs &a, unsigned fn, const BlockCarry &c) {
+  a.blk_fn[blockIdx.x] = (unsigned char)(fn | (c.open << 2));
+  if (c.open && a.host) host_store(&a.host->open_carry, 1u);
+}
+
 // Words of one block from coefficients: P_w (< 2^37) per word, v_w = lo(P_w) +
 // hi(P_{w-1}), a wave-shuffle scan of per-thread carry functions, words
-// written for block carry-in 0 and the block's function saved for k_carry_fix.
+// written for the block's carry-in, its function and mark saved for k_carry_ripple.
 // The coefficient window is staged into LDS with eight loads in flight per
 // thread; each thread's word w-1 partial comes from its left neighbour.
 static __global__ __launch_bounds__(CT) void k_carry_local(CarryArgs a) {
   extern __shared__ long long cl[];
   __shared__ unsigned wave_fn[CT / 64];
+  __shared__ BlockCarry bc;
   const int tid = threadIdx.x;
   bind_carry(a, blockIdx.y);
   if (blockIdx.x >= a.nblk) return;
   const long long W0 = (long long)blockIdx.x * CT * CWPT;
   const long long wfirst = W0 + (long long)tid * CWPT;
   const double inv_b = 1.0 / (double)a.bits;
-  long long lo_bit = 32 * (W0 - 1) - a.cbits + 1;
+  long long lo_bit = 32 * (W0 - 2) - a.cbits + 1;
   long long jbase = lo_bit <= 0 ? 0 : div_small(lo_bit + a.bits - 1, a.bits, inv_b);
   long long jend = div_small(32 * (W0 + (long long)CT * CWPT) - 1, a.bits, inv_b);  // inclusive
   if (jend >= (long long)a.ncoef) jend = (long long)a.ncoef - 1;
@@ -923,7 +982,7 @@ static __global__ __launch_bounds__(CT) void k_carry_local(CarryArgs a) {
     }
   }
   __syncthreads();
-  unsigned long long P[CWPT + 1];
+  unsigned long long P[CWPT + 1], Pm2 = 0;  // Pm2: word W0 - 2 (thread 0)
   if (staged) {
     const int lane = tid & 63;
     const int D = (int)(32 * W0 - (long long)a.bits * jbase);
@@ -940,20 +999,27 @@ static __global__ __launch_bounds__(CT) void k_carry_local(CarryArgs a) {
       left = (wfirst >= 1 && wfirst - 1 < (long long)a.CL) ? partial_rel(cl, cnti, a.bits, a.cbits, inv_bf, x0 - 32)
                                                           : 0ull;
     P[0] = left;
+    if (tid == 0 && W0) Pm2 = partial_rel(cl, cnti, a.bits, a.cbits, inv_bf, x0 - 64);
     if (a.add) {
 #pragma unroll
       for (int k = 0; k <= CWPT; k++) {
         long long w = wfirst - 1 + k;
         if (w >= 0 && w < (long long)a.addl && w < (long long)a.CL) P[k] += a.add[w];
       }
+      if (tid == 0 && W0 && W0 - 2 < (long long)a.addl) Pm2 += a.add[W0 - 2];
     }
   } else {
+    if (tid == 0 && W0) {
+      word_partials(a, W0 - 1, P);
+      Pm2 = P[0];
+    }
     if (wfirst < (long long)a.CL)
       word_partials(a, wfirst, P);
     else
       for (int k = 0; k <= CWPT; k++) P[k] = 0;
   }
   if (wfirst == 0) P[0] = 0;
+  if (tid == 0) bc = block_carry(P[0], Pm2);
   unsigned long long v[CWPT];
 #pragma unroll
   for (int k = 0; k < CWPT; k++) v[k] = (P[k + 1] & 0xffffffffull) + (P[k] >> 32);
@@ -980,9 +1046,13 @@ static __global__ __launch_bounds__(CT) void k_carry_local(CarryArgs a) {
   if (tid == 0) {
     unsigned tot = 2u;
     for (int w = 0; w < CT / 64; w++) tot = carry_compose(tot, wave_fn[w]);
-    a.blk_fn[blockIdx.x] = (unsigned char)tot;
+    carry_publish(a, tot, bc);
   }
-  unsigned cin = carry_compose(pre, excl) & 1u;
+  if (a.host && blockIdx.x == 0 && tid < 64) {
+    const unsigned m = margin_of_slots(a.margin);
+    if (tid == 0) host_store(&a.host->margin, m);
+  }
+  unsigned cin = (carry_compose(pre, excl) >> bc.cin) & 1u;
   uint32_t o[CWPT];
 #pragma unroll
   for (int k = 0; k < CWPT; k++) {
@@ -1012,6 +1082,7 @@ template <int GCOV>  // group sums that can cover one word (<= CARRY_GCOV)
 static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
   extern __shared__ uint32_t gl_w[];
   __shared__ unsigned wave_fn[GCT / 64];
+  __shared__ BlockCarry bc;
   bind_carry(a, blockIdx.y);  // batched: product blockIdx.y
   if ((unsigned long long)blockIdx.x >= a.nblk) return;
   const int tid = threadIdx.x;
@@ -1019,7 +1090,7 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
   const int gb = a.gC * a.bits;  // bits per group, >= 32
   const double inv_gb = 1.0 / (double)gb;
   const long long ng = a.ng;
-  long long g_first = W0 == 0 ? 0 : div_small(32 * (W0 - 1) + 31, gb, inv_gb) - (CARRY_GCOV - 1);
+  long long g_first = W0 == 0 ? 0 : div_small(32 * (W0 - 2) + 31, gb, inv_gb) - (CARRY_GCOV - 1);
   if (g_first < 0) g_first = 0;
   long long g_last = div_small(32 * (W0 + (long long)GCT * GWPT - 1) + 31, gb, inv_gb);
   if (g_last >= ng) g_last = ng - 1;
@@ -1061,7 +1132,20 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
   const long long lim64 = (long long)a.CL - W0;
   const int lim = lim64 > (1 << 30) ? (1 << 30) : (int)lim64;
   const int wmin = W0 == 0 ? 0 : -1;  // word W0 - 1 exists unless W0 = 0
-  unsigned long long P[GWPT + 1];
+  unsigned long long P[GWPT + 1], Pm2 = 0;  // Pm2: word W0 - 2 (thread 0)
+  if (tid == 0 && W0) {
+    const int num = 32 * (-2 - D) + 31 - r0;
+    const int gh = num < 0 ? -1 : min((int)((unsigned)num / (unsigned)gb), ngl - 1);
+#pragma unroll
+    for (int t = 0; t < GCOV; t++) {
+      const int off = -2 - (((r0 + (gh - t) * gb) >> 5) + D);
+      if (gh - t >= 0 && off < a.gK) {
+        const unsigned i = (unsigned)((gh - t) * a.gKs + off);
+        Pm2 += gl_w[i + (i >> 5)];
+      }
+    }
+    if (a.add && W0 - 2 < (long long)a.addl) Pm2 += a.add[W0 - 2];
+  }
   if ((gb & 31) == 0) {
     // Word-aligned group starts (G b a multiple of 32, e.g. b even): group gl
     // starts at block word D + gl Q, so word wl = D + gh Q + o takes word
@@ -1133,6 +1217,7 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
     }
   }
   if (wfirst == 0) P[0] = 0;
+  if (tid == 0) bc = block_carry(P[0], Pm2);
   unsigned long long v[GWPT];
 #pragma unroll
   for (int k = 0; k < GWPT; k++) v[k] = (P[k + 1] & 0xffffffffull) + (P[k] >> 32);
@@ -1158,9 +1243,13 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
   if (tid == 0) {
     unsigned tot = 2u;
     for (int q = 0; q < GCT / 64; q++) tot = carry_compose(tot, wave_fn[q]);
-    a.blk_fn[blockIdx.x] = (unsigned char)tot;
+    carry_publish(a, tot, bc);
   }
-  unsigned cin = carry_compose(pre, excl) & 1u;
+  if (a.host && blockIdx.x == 0 && tid < 64) {
+    const unsigned m = margin_of_slots(a.margin);
+    if (tid == 0) host_store(&a.host->margin, m);
+  }
+  unsigned cin = (carry_compose(pre, excl) >> bc.cin) & 1u;
   uint32_t o[GWPT];
 #pragma unroll
   for (int k = 0; k < GWPT; k++) {
@@ -1179,108 +1268,73 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
   }
 }
 
-// One workgroup per product: scan the block carry functions, then add the
-// carry into every block whose carry-in is 1 (ripple through 0xffffffff words
-// inside the block). Thread t owns blocks [t per, t per + per) with per a
-// multiple of 16, so its function bytes arrive as 16-byte loads; the scan
-// across threads uses wave shuffles; the first words of the carried blocks
-// of a 16-block chunk are read together and take the +1 when it stops there;
-// the other carried blocks (all-ones blocks, as in products close to a power
-// of two, and +1s that run on) are marked for k_carry_apply.
-static __global__ __launch_bounds__(1024) void k_carry_fix(CarryArgs a) {
-  __shared__ unsigned wfn[16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  bind_carry(a, blockIdx.x);
-  const unsigned long long nb = a.nblk;
-  const unsigned long long per = (((nb + 1023) / 1024) + 15) & ~15ull;
-  const unsigned long long b0 = (unsigned long long)tid * per;
-  unsigned long long b1 = b0 + per;
-  if (b1 > nb) b1 = nb;
-  unsigned fn = 2u;  // identity
-  for (unsigned long long c0 = b0; c0 < b1; c0 += 16) {
-    const uint4 v = *reinterpret_cast<const uint4 *>(a.blk_fn + c0);
-    const unsigned wv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int k = 0; k < 16; k++)
-      if (c0 + k < b1) fn = carry_compose(fn, (wv[k >> 2] >> (8 * (k & 3))) & 3u);
-  }
-  unsigned inc = fn;
-  for (int off = 1; off < 64; off <<= 1) {
-    unsigned gq = __shfl_up(inc, off, 64);
-    if (lane >= off) inc = carry_compose(gq, inc);
-  }
-  unsigned excl = __shfl_up(inc, 1, 64);
-  if (lane == 0) excl = 2u;
-  if (lane == 63) wfn[wave] = inc;
-  __syncthreads();
-  unsigned pre = 2u;
-  for (int w = 0; w < wave; w++) pre = carry_compose(pre, wfn[w]);
-  unsigned c = carry_compose(pre, excl) & 1u;
-  const unsigned long long wpb = a.wpb;
-  for (unsigned long long c0 = b0; c0 < b1; c0 += 16) {
-    const uint4 v = *reinterpret_cast<const uint4 *>(a.blk_fn + c0);
-    const unsigned wv[4] = {v.x, v.y, v.z, v.w};
-    unsigned carried = 0, heavy = 0;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      if (c0 + k < b1) {
-        const unsigned f = (wv[k >> 2] >> (8 * (k & 3))) & 3u;
-        if (c) {
-          // a carried block whose function propagates holds only 0xffffffff
-          // words (it becomes zero): left to k_carry_apply
-          if (f == 2u)
-            heavy |= 1u << k;
-          else
-            carried |= 1u << k;
-        }
-        c = (f >> c) & 1u;
-      }
-    }
-    uint32_t x[16];
-#pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = ((carried >> k) & 1u) ? a.out[(c0 + k) * wpb] : 0u;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      if (!((carried >> k) & 1u)) continue;
-      if (x[k] != 0xffffffffu)
-        a.out[(c0 + k) * wpb] = x[k] + 1u;
-      else
-        heavy |= 1u << k;  // the +1 runs on through 0xffffffff words
-    }
-    if (heavy)
-      for (int k = 0; k < 16; k++)
-        if ((heavy >> k) & 1u) a.blk_fn[c0 + k] |= 4u;
-  }
-}
-
-// The carried blocks k_carry_fix marked (bit 2 of the block function): one
-// workgroup per block adds the carry with all its threads, clearing a block of
-// 0xffffffff words, or the 0xffffffff words below the first other word, which
-// takes the +1 (a block whose function does not propagate has such a word).
-static __global__ __launch_bounds__(256) void k_carry_apply(CarryArgs a) {
+// The blocks whose carry-in the block itself left open (bit 2 of its function):
+// their carry-in is what the nearest lower block that does not propagate hands
+// on. Each workgroup looks at RIPPLE_BLOCKS functions and is done when none of
+// them is marked; otherwise it walks down to the carry into its first block,
+// then up through its blocks, and adds the carry where it is 1: a block of
+// 0xffffffff words (one that propagates) is cleared, in any other the words up
+// to the first other one are cleared and that one takes the +1.
+constexpr int RIPPLE_BLOCKS = 256;
+static __global__ __launch_bounds__(RIPPLE_BLOCKS) void k_carry_ripple(CarryArgs a) {
+  __shared__ unsigned char fn[RIPPLE_BLOCKS];
+  __shared__ int near;
   __shared__ unsigned long long first;
   const int tid = threadIdx.x;
   bind_carry(a, blockIdx.y);
-  if (blockIdx.x >= a.nblk) return;
-  const unsigned f = a.blk_fn[blockIdx.x];
-  if (!(f & 4u)) return;
-  const unsigned long long w0 = (unsigned long long)blockIdx.x * a.wpb;
-  const unsigned long long w1 = w0 + a.wpb < a.CL ? w0 + a.wpb : a.CL;
-  if ((f & 3u) == 2u) {
-    for (unsigned long long w = w0 + tid; w < w1; w += 256) a.out[w] = 0u;
-    return;
-  }
-  if (tid == 0) first = w1;
-  __syncthreads();
-  for (unsigned long long w = w0 + tid; w < w1; w += 256)
-    if (a.out[w] != 0xffffffffu) {
-      atomicMin(&first, w);
+  const unsigned long long b0 = (unsigned long long)blockIdx.x * RIPPLE_BLOCKS;
+  if (b0 >= a.nblk) return;
+  const int n = (int)(a.nblk - b0 < RIPPLE_BLOCKS ? a.nblk - b0 : RIPPLE_BLOCKS);
+  const unsigned f = tid < n ? a.blk_fn[b0 + tid] : 0u;
+  fn[tid] = (unsigned char)f;
+  if (!__syncthreads_or((int)(f & 4u))) return;
+  // carry into block b0: the nearest block below whose function is constant
+  unsigned c = 0;
+  for (unsigned long long hi = b0; hi > 0;) {
+    const unsigned long long lo = hi > RIPPLE_BLOCKS ? hi - RIPPLE_BLOCKS : 0;
+    if (tid == 0) near = -1;
+    __syncthreads();
+    const unsigned g = lo + tid < hi ? a.blk_fn[lo + tid] & 3u : 2u;
+    if (g != 2u) atomicMax(&near, tid);
+    __syncthreads();
+    const int k = near;
+    __syncthreads();
+    if (k >= 0) {
+      c = a.blk_fn[lo + k] & 1u;
       break;
     }
-  __syncthreads();
-  const unsigned long long fw = first;
-  for (unsigned long long w = w0 + tid; w < fw; w += 256) a.out[w] = 0u;
-  if (tid == 0 && fw < w1) a.out[fw] += 1u;
+    hi = lo;
+  }
+  for (int k = 0; k < n; k++) {  // uniform across the workgroup
+    const unsigned g = fn[k];
+    if ((g & 4u) && c) {
+      const unsigned long long w0 = (b0 + k) * a.wpb;
+      const unsigned long long w1 = w0 + a.wpb < a.CL ? w0 + a.wpb : a.CL;
+      if ((g & 3u) == 2u) {
+        for (unsigned long long w = w0 + tid; w < w1; w += RIPPLE_BLOCKS) a.out[w] = 0u;
+      } else {
+        if (tid == 0) first = w1;
+        __syncthreads();
+        for (unsigned long long w = w0 + tid; w < w1; w += RIPPLE_BLOCKS)
+          if (a.out[w] != 0xffffffffu) {
+            atomicMin(&first, w);
+            break;
+          }
+        __syncthreads();
+        const unsigned long long fw = first;
+        for (unsigned long long w = w0 + tid; w < fw; w += RIPPLE_BLOCKS) a.out[w] = 0u;
+        if (tid == 0 && fw < w1) a.out[fw] += 1u;
+        __syncthreads();
+      }
+    }
+    c = (g >> c) & 1u;
+  }
+}
+
+// The margin of a product to the host ahead of its carry (products in place).
+static __global__ __launch_bounds__(64) void k_margin_out(const unsigned int *m, HostResult *host) {
+  const unsigned v = margin_of_slots(m);
+  if (threadIdx.x == 0) host_store(&host->margin, v);
 }
 
 // --------------------------------------------------------------- utilities
@@ -1458,11 +1512,12 @@ __device__ void wg_carry(const long long *coef, long long ncoef, int bits, int c
 
 // All products of one transform length class L (one-pass plans: N = L).
 struct ClassArgs {
-  const MulDesc *desc;
-  int count;
+  const MulDesc *desc;    // nullptr: the single product `one`
   Roots roots;
   const cd *tl;
   unsigned int *margins;  // per product, float bits of the worst rounding distance
+  int clear;              // a set of MARGIN_SLOTS slots: clear the others
+  MulDesc one;            // a single product travels in the launch itself
 };
 
 // Values the same in every lane, held in scalar registers.
@@ -1553,8 +1608,9 @@ template <int L>
 __global__ __launch_bounds__((Row<L>::T)) void k_mul1(ClassArgs ca) {
   using RC = Row<L>;
   __shared__ cd lds[RC::LDS_ELEMS];
+  __shared__ float wmax[(RC::T + 63) / 64];
   const int tid = threadIdx.x, idx = blockIdx.x;
-  const MulDesc d = uniform_desc(ca.desc[idx]);
+  const MulDesc d = ca.desc ? uniform_desc(ca.desc[idx]) : ca.one;
   cd wt = omega_direct(ca.roots, (unsigned long long)tid);
   const bool square = d.a == d.b && d.al == d.bl;
   cd x[8], xa[RC::XR];
