@@ -1648,9 +1648,17 @@ __global__ __launch_bounds__((Row<L>::T)) void k_mul1(ClassArgs ca) {
     coef[j] = round_coef(f.x * inv_n, fast, worst);
     coef[j + L] = round_coef(f.y * inv_n, fast, worst);
   }
-  margin_reduce(ca.margins + idx, worst);
+  float far = (float)worst;
+  for (int off = 32; off > 0; off >>= 1) far = fmaxf(far, __shfl_xor(far, off, 64));
+  if ((tid & 63) == 0) wmax[tid >> 6] = far;
   __syncthreads();
-wg_carry<RC::T>(coef, 2 * L, d.bits, d.cbits, d.c, (long long)d.cl, d.d, (long long)d.dl, tid);
+  if (tid == 0) {
+    for (int w = 1; w < (RC::T + 63) / 64; w++) far = fmaxf(far, wmax[w]);
+    host_store(ca.margins + idx, __float_as_uint(far));
+  }
+  if (ca.clear)
+    for (int i = 1 + tid; i < MARGIN_SLOTS; i += RC::T) ca.margins[i * MARGIN_STRIDE] = 0u;
+  wg_carry<RC::T>(coef, 2 * L, d.bits, d.cbits, d.c, (long long)d.cl, d.d, (long long)d.dl, tid);
 }
 
 }  // namespace bcg

@@ -68,3 +68,21 @@ def test_middle_pass_lengths(bc, inner):
             assert np.array_equal(s, want[1]), cands[i]
     finally:
         bc.plan_force(n, -1)
+
+
+def test_margins_are_each_products_own(bc):
+    # a margin raised by digits far above the bound must not stay in any slot:
+    # the same product reads the same margin before and after it, alone and batched
+    a, b = operands(7, 3000, 2500)
+    own = bc.mul(a, b)[1]["margin"]
+    _, batch = bc.mul_batch([(a, b), (a[:700], b[:600])])
+    bc.plan_digit_bias(6)
+    try:
+        assert bc.mul(*operands(8, 5000, 5000))[1]["retries"] >= 1
+        bc.mul_batch([operands(9, 5000, 5000), operands(10, 5000, 5000), operands(11, 40000, 40000)])
+    finally:
+        bc.plan_digit_bias(0)
+    assert bc.mul(a, b)[1]["margin"] == own
+    assert bc.mul_batch([(a, b), (a[:700], b[:600])])[1] == batch
+    small = bc.mul(a[:700], b[:600])[1]["margin"]
+    assert batch == max(own, small) and small < own
