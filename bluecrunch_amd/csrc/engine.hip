@@ -53,7 +53,8 @@ struct Engine {
   hipEvent_t fork_ev = nullptr, join_ev[NAUX] = {nullptr, nullptr, nullptr};
   std::map<unsigned long long, RootsDev> roots;  // keyed by N
   std::map<int, cd *> ltab;                      // e^{2 pi i t/L}, keyed by L
-  DevBuf bufA, bufB, wA, wB, wC, blk, margin, zbuf, counters;
+  DevBuf bufA, bufB, wA, wB, wC, blk, margin, zbuf;
+  DevBuf scan, flags, one;  // state of the scans and sums (zero between launches), the word 1
   HostResult *hres = nullptr;      // pinned: what the kernels of a product leave for the host
   HostResult *hres_dev = nullptr;  // its device address
   bool prof = false;
@@ -96,6 +97,13 @@ int fail(int code, const char *what, hipError_t e = hipSuccess) {
     hipError_t e_ = (x);                               \
     if (e_ != hipSuccess) return fail(BCG_E_HIP, #x, e_); \
   } while (0)
+
+#define LAUNCH(kern, grid, block, stream, ...) \
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, stream, __VA_ARGS__)
+
+// grid.y > 1 only for batched launches (PassArgs::desc set).
+#define LAUNCH2(kern, gx, gy, block, stream, ...) \
+  hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(block), 0, stream, __VA_ARGS__)
 
 void ep_trim(size_t keep = 0);  // idle blocks of the e pipeline's pool
 
@@ -281,6 +289,11 @@ int init_locked(int device) {
   g.device = device;
   g.ready = true;
   if (int rc = ensure(g.margin, sizeof(unsigned int) * MARGIN_SLOTS * MARGIN_STRIDE)) return rc;
+  if (int rc = ensure(g.scan, 256)) return rc;
+  if (int rc = ensure(g.one, 4)) return rc;
+  LAUNCH(k_fill_u32, 1, 64, g.stream, (uint32_t *)g.scan.p, 64ull, 0u);
+  LAUNCH(k_fill_u32, 1, 64, g.stream, (uint32_t *)g.one.p, 1ull, 1u);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipHostMalloc((void **)&g.hres, sizeof(HostResult), hipHostMallocMapped));
   HIPCHK(hipHostGetDevicePointer((void **)&g.hres_dev, g.hres, 0));
   // every kernel family's code object now rather than inside a first product
@@ -754,13 +767,6 @@ int make_plan(unsigned long long AL, unsigned long long BL, int force_bits, Plan
 
 // --------------------------------------------------------------- launching
 
-#define LAUNCH(kern, grid, block, stream, ...) \
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, stream, __VA_ARGS__)
-
-// grid.y > 1 only for batched launches (PassArgs::desc set).
-#define LAUNCH2(kern, gx, gy, block, stream, ...) \
-  hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(block), 0, stream, __VA_ARGS__)
-
 int coef_bits(const Plan &p) {
   unsigned long long m = p.dA < p.dB ? p.dA : p.dB;
   int cb = 2 * p.bits + ilog2u(m + 1) + 2;
@@ -798,13 +804,17 @@ void launch_ripple(const CarryArgs &c, int count, hipStream_t s) {
 // Ends a carry launched with c: without a host read-back the ripple follows on
 // the stream; with one, the host waits, and launches it only if a block asked
 // for it. *margin (with host) receives the product's margin.
-int end_carry(const CarryArgs &c, hipStream_t s, double *margin) {
+// top: after the carry, the search for the output's highest nonzero word as well
+// (hres->top once the host has waited).
+void launch_top(const uint32_t *x, size_t n, hipStream_t s);
+int end_carry(const CarryArgs &c, hipStream_t s, double *margin, bool top = false) {
   if (!c.host) {
     ProfScope ps(BCG_K_CARRY, s);
     launch_ripple(c, 1, s);
     HIPCHK(hipGetLastError());
     return 0;
   }
+  if (top) launch_top(c.out, (size_t)c.CL, s);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));
   float f;
@@ -815,6 +825,7 @@ int end_carry(const CarryArgs &c, hipStream_t s, double *margin) {
       ProfScope ps(BCG_K_CARRY, s);
       launch_ripple(c, 1, s);
     }
+    if (top) launch_top(c.out, (size_t)c.CL, s);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s));
   }
@@ -825,7 +836,7 @@ int end_carry(const CarryArgs &c, hipStream_t s, double *margin) {
 // result and takes the worst slot of g.margin there.
 int run_carry(const long long *coef, unsigned long long ncoef, int bits, int cbits, uint32_t *out,
               unsigned long long CL, hipStream_t s, const uint32_t *add = nullptr, unsigned long long addl = 0,
-              unsigned cM = 0, unsigned crows = 0, double *margin = nullptr) {
+              unsigned cM = 0, unsigned crows = 0, double *margin = nullptr, bool top = false) {
   if (CL == 0) return 0;
   const unsigned long long wpb = (unsigned long long)CT * CWPT;
   unsigned long long nblk = (CL + wpb - 1) / wpb;
@@ -856,7 +867,7 @@ int run_carry(const long long *coef, unsigned long long ncoef, int bits, int cbi
     ProfScope ps(BCG_K_CARRY, s);
     hipLaunchKernelGGL(k_carry_local, dim3((unsigned)nblk), dim3(CT), c.lds_slots * sizeof(long long), s, c);
   }
-  return end_carry(c, s, margin);
+  return end_carry(c, s, margin, top);
 }
 
 // Dynamic LDS of k_carry_groups: the group sums under one block's words and the
@@ -889,11 +900,11 @@ int group_words(const Plan &p);
 int group_stride(int K);
 bool coef_transposed(const Plan &p);
 int carry_of_plan(const Plan &p, uint32_t *out, unsigned long long CL, hipStream_t s, const uint32_t *add,
-                  unsigned long long addl, double *margin) {
+                  unsigned long long addl, double *margin, bool top = false) {
   const int K = group_words(p);
   if (!K)
     return run_carry((const long long *)g.bufB.p, 2 * p.N, p.bits, coef_bits(p), out, CL, s, add, addl,
-                     coef_transposed(p) ? (unsigned)p.M[0] : 0u, 2u * (unsigned)p.L[0], margin);
+                     coef_transposed(p) ? (unsigned)p.M[0] : 0u, 2u * (unsigned)p.L[0], margin, top);
   if (CL == 0) return 0;
   const unsigned long long wpb = (unsigned long long)GCT * GWPT;
   unsigned long long nblk = (CL + wpb - 1) / wpb;
@@ -924,7 +935,7 @@ int carry_of_plan(const Plan &p, uint32_t *out, unsigned long long CL, hipStream
     ProfScope ps(BCG_K_CARRY, s);
     launch_carry_groups(c, group_cover(p.C[0], p.bits, K), dim3((unsigned)nblk), group_lds(p.C[0], p.bits, c.gKs), s);
   }
-  return end_carry(c, s, margin);
+  return end_carry(c, s, margin, top);
 }
 
 int zero_margin(hipStream_t s) {
@@ -1277,7 +1288,7 @@ int run_class(int L, ClassArgs &ca, int count, hipStream_t s) {
 // memory (a descriptor copy, two fill kernels and a margin copy around it were
 // 20 of 51 us at 2048 points).
 int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL,
-                hipStream_t s, double *margin, const uint32_t *D = nullptr, size_t DL = 0) {
+                hipStream_t s, double *margin, const uint32_t *D, size_t DL, bool top) {
   const bool deferred = g_defer.in_product;
   ClassArgs ca;
   memset(&ca, 0, sizeof ca);
@@ -1297,6 +1308,8 @@ int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t
   if (int rc = run_class(p.L[0], ca, 1, s)) return rc;
   *margin = 0.0;
   if (deferred) return 0;  // read with the scope's other sets later
+  if (top) launch_top(C, CL, s);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));
   float f;
   memcpy(&f, &g.hres->margin, sizeof f);
@@ -1471,13 +1484,18 @@ int defer_flush() {
 }
 
 int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL, int force_bits,
-                 hipStream_t s, bcg_mul_info *info, const uint32_t *D, size_t DL);
+                 hipStream_t s, bcg_mul_info *info, const uint32_t *D, size_t DL, size_t *top);
+int d_top_len(const uint32_t *x, size_t n, size_t *len, hipStream_t s);
+int rest_of_top(const uint32_t *x, size_t n, size_t *len, hipStream_t s);
 
+// top (operands and output all nonempty): the output's length without its zero
+// top words, read in the same wait as the margin.
 int mul_dev_locked(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL,
-                   int force_bits, hipStream_t s, bcg_mul_info *info, const uint32_t *D = nullptr, size_t DL = 0) {
+                   int force_bits, hipStream_t s, bcg_mul_info *info, const uint32_t *D = nullptr, size_t DL = 0,
+                   size_t *top = nullptr) {
   DeferScope &d = g_defer;
   if (!d.open || d.in_product || g_fixed || std::this_thread::get_id() != d.owner || C == A || C == B)
-    return mul_dev_body(C, CL, A, AL, B, BL, force_bits, s, info, D, DL);
+    return mul_dev_body(C, CL, A, AL, B, BL, force_bits, s, info, D, DL, top);
   // a deferred product: margin slots of its own set, no read-back
   if (d.n == DEFER_SETS)
     if (int rc = defer_flush()) return rc;
@@ -1486,10 +1504,12 @@ int mul_dev_locked(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const u
   d.in_product = true;
   bcg_mul_info inf;
   memset(&inf, 0, sizeof inf);
-  const int rc = mul_dev_body(C, CL, A, AL, B, BL, force_bits, s, &inf, D, DL);
+  const int rc = mul_dev_body(C, CL, A, AL, B, BL, force_bits, s, &inf, D, DL, nullptr);
   d.in_product = false;
   g.margin.p = keep;
   if (rc) return rc;
+  if (top)
+    if (int rc2 = d_top_len(C, CL, top, s)) return rc2;
   if (inf.points) {  // an FFT product: its set holds its margin (schoolbook products have none)
     d.points[d.n] = inf.points;
     d.bits[d.n] = inf.bits;
@@ -1500,7 +1520,7 @@ int mul_dev_locked(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const u
 }
 
 int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL, int force_bits,
-                 hipStream_t s, bcg_mul_info *info, const uint32_t *D, size_t DL) {
+                 hipStream_t s, bcg_mul_info *info, const uint32_t *D, size_t DL, size_t *top) {
   bcg_mul_info inf;
   memset(&inf, 0, sizeof inf);
   bool square = (A == B && AL == BL);
@@ -1519,7 +1539,8 @@ int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
   }
   if (AL + BL < 100 && force_bits <= 0) {
     if (info) *info = inf;
-    return basecase_dev(C, CL, A, AL, B, BL, s, D, DL);
+    if (int rc = basecase_dev(C, CL, A, AL, B, BL, s, D, DL)) return rc;
+    return top ? d_top_len(C, CL, top, s) : 0;
   }
   Plan p;
   if (int rc = make_plan(AL, BL, force_bits, p)) return rc;
@@ -1534,7 +1555,7 @@ int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
         if (int rc = ensure(g.zbuf, CL * sizeof(uint32_t) + 64)) return rc;
         dst = (uint32_t *)g.zbuf.p;
       }
-      if (int rc = mul_onepass(p, dst, CL, A, AL, B, BL, s, &m, D, DL)) return rc;
+      if (int rc = mul_onepass(p, dst, CL, A, AL, B, BL, s, &m, D, DL, top != nullptr)) return rc;
       inf.bits = p.bits;
       inf.passes = 1;
       inf.points = (size_t)p.N;
@@ -1558,7 +1579,7 @@ int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
       if (int rc = read_margin(s, &m)) return rc;
     } else {
       // a deferred product's margin is read with its scope's other sets later
-      if (int rc = carry_of_plan(p, C, CL, s, D, DL, g_defer.in_product ? nullptr : &m)) return rc;
+      if (int rc = carry_of_plan(p, C, CL, s, D, DL, g_defer.in_product ? nullptr : &m, top != nullptr)) return rc;
     }
     inf.bits = p.bits;
     inf.passes = p.P;
@@ -1589,6 +1610,7 @@ int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
   }
   if (!g_defer.in_product) note_product(inf.points, inf.bits, inf.margin);  // deferred: when its set is read
   if (info) *info = inf;
+  if (top) return alias ? d_top_len(C, CL, top, s) : rest_of_top(C, CL, top, s);
   return 0;
 }
 
@@ -1863,15 +1885,13 @@ namespace {
 // Scratch of bcg_mul_dev_noalloc: the engine's per-product buffers as fixed
 // slices of one static device array, for products whose transform has at
 // most NOALLOC_MAX_POINTS points: two transform arrays (16 bytes a point),
-// the margin slots, carry block functions, counters,
-// and the staging of an aliased output (one-pass and schoolbook products).
+// the margin slots, carry block functions, and the staging of an aliased output (one-pass and schoolbook products).
 constexpr unsigned long long NOALLOC_MAX_POINTS = 1ull << 20;
 constexpr size_t NA_ARR = (size_t)NOALLOC_MAX_POINTS * sizeof(cd);
 constexpr size_t NA_MARGIN = (size_t)MARGIN_SLOTS * MARGIN_STRIDE * sizeof(unsigned int);
 constexpr size_t NA_BLK = (size_t)64 << 10;
-constexpr size_t NA_COUNTERS = 256;
 constexpr size_t NA_ZBUF = (size_t)64 << 10;
-constexpr size_t NA_BYTES = 2 * NA_ARR + NA_MARGIN + NA_BLK + NA_COUNTERS + NA_ZBUF;
+constexpr size_t NA_BYTES = 2 * NA_ARR + NA_MARGIN + NA_BLK + NA_ZBUF;
 
 }  // namespace
 
@@ -1914,12 +1934,12 @@ int prepare_noalloc() {
 // The engine's buffers pointed at the scratch for one call (under the engine
 // lock), restored afterwards.
 struct ScratchScope {
-  DevBuf *bufs[6] = {&g.bufA, &g.bufB, &g.margin, &g.blk, &g.counters, &g.zbuf};
-  DevBuf saved[6];
+  DevBuf *bufs[5] = {&g.bufA, &g.bufB, &g.margin, &g.blk, &g.zbuf};
+  DevBuf saved[5];
   explicit ScratchScope(unsigned char *base) {
-    const size_t sizes[6] = {NA_ARR, NA_ARR, NA_MARGIN, NA_BLK, NA_COUNTERS, NA_ZBUF};
+    const size_t sizes[5] = {NA_ARR, NA_ARR, NA_MARGIN, NA_BLK, NA_ZBUF};
     size_t off = 0;
-    for (int i = 0; i < 6; i++) {
+    for (int i = 0; i < 5; i++) {
       saved[i] = *bufs[i];
       bufs[i]->p = base + off;
       bufs[i]->bytes = sizes[i];
@@ -1928,7 +1948,7 @@ struct ScratchScope {
     g_fixed = true;
   }
   ~ScratchScope() {
-    for (int i = 0; i < 6; i++) *bufs[i] = saved[i];
+    for (int i = 0; i < 5; i++) *bufs[i] = saved[i];
     g_fixed = false;
   }
 };
@@ -1950,7 +1970,7 @@ int bcg_shutdown(void) {
   (void)hipStreamSynchronize(g.stream);
   g_defer.open = false;
   g_defer.n = 0;
-  for (DevBuf *b : {&g.bufA, &g.bufB, &g.wA, &g.wB, &g.wC, &g.blk, &g.margin, &g.zbuf, &g.counters,
+  for (DevBuf *b : {&g.bufA, &g.bufB, &g.wA, &g.wB, &g.wC, &g.blk, &g.margin, &g.zbuf, &g.scan, &g.flags, &g.one,
                     &g_defer.sets}) {
     if (b->p) (void)hipFree(b->p);
     b->p = nullptr;

@@ -281,12 +281,15 @@ __device__ __forceinline__ unsigned margin_of_slots(const unsigned int *m) {
   return v;
 }
 
-// What the host reads after a product, in host memory the kernels write: the
-// worst rounding distance (float bits) and whether a carry block's carry-in is
-// still open (see k_carry_groups).
+// What the host reads after a call, in host memory the kernels write: the worst
+// rounding distance (float bits), whether a carry block's carry-in is still open
+// (see k_carry_groups), 1 + the index of the highest nonzero word (see
+// k_top_nonzero, k_addsub) and the order of a difference's operands.
 struct HostResult {
   unsigned margin;
   unsigned open_carry;
+  unsigned long long top;
+  unsigned swapped;
 };
 __device__ __forceinline__ void host_store(unsigned *p, unsigned v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

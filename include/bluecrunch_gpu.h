@@ -72,7 +72,7 @@ int bcg_mul_dev_bits(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const
 /* bcg_mul_dev without any allocation: no hipMalloc, hipFree or other
  * allocating call, for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops). No counterpart in the reference. Its buffers
- * are one static device array of 33,693,952 bytes (32.1 MiB) per GPU, held
+ * are one static device array of 33,693,696 bytes (32.1 MiB) per GPU, held
  * until the process ends and set up by bcg_init (which must have run), so the
  * transform is limited to 2^20 points (operands up to about 400,000 words
  * each; bcg_plan_query gives the length) and an output that aliases an
