@@ -289,6 +289,7 @@ struct HostResult {
   unsigned margin;
   unsigned open_carry;
   unsigned long long top;
+  unsigned long long exp;      // k_rcp_small: the result's exponent (top: its length, swapped: its sign)
   unsigned swapped;
 };
 __device__ __forceinline__ void host_store(unsigned *p, unsigned v) {

@@ -155,3 +155,18 @@ def test_zero_and_argument_errors(bc):
     assert dev(bc, "mul", zero, five)[0].size == 0
     with pytest.raises(bc.GpuError):
         dev(bc, "rcp", zero, None, 3)
+
+
+@pytest.mark.parametrize("p", [0, 1, 2, 3, 6, 7, 30, 31, 128, 129, 130, 255, 256, 257, 258, 511, 512, 513])
+def test_rcp_short_precisions(bc, oracle, p):
+    # both sides of the precision up to which one workgroup runs the whole
+    # recursion: operands of one word, around p and far longer, either sign,
+    # powers of the word base (products that end in zero words) and all ones
+    rng = np.random.default_rng(19 + p)
+    cases = [rand_bf(rng, n, n, 40, zero_ok=False) for n in (1, 2, 3, 4, max(1, p - 1), p + 1, p + 2, p + 3, 3 * p + 9)]
+    for n in (1, 2, max(1, p), p + 5):
+        one = np.zeros(n, dtype=np.uint32)
+        one[-1] = 1
+        cases += [(one, -n, 1), (np.full(n, 0xFFFFFFFF, dtype=np.uint32), 7, 0)]
+    for a in cases:
+        assert same(dev(bc, "rcp", a, None, p), oracle.bigfloat_rcp(a, p)), (p, a[0].size, a[1:])
