@@ -1191,47 +1191,18 @@ int run_transforms(const Plan &p, const uint32_t *A, unsigned long long AL, cons
   return 0;
 }
 
-__global__ void k_basecase(const uint32_t *A, unsigned long long AL, const uint32_t *B, unsigned long long BL,
-                           uint32_t *C, unsigned long long CL, const uint32_t *D, unsigned long long DL) {
-  // column sums of 32x32-bit products split into low and high halves
-  extern __shared__ unsigned long long colsum[];
-  const unsigned long long W = AL + BL;
-  for (unsigned long long w = threadIdx.x; w < W; w += blockDim.x) {
-    unsigned long long lo = 0, hi = 0;
-    unsigned long long i0 = w >= BL ? w - BL + 1 : 0;
-    for (unsigned long long i = i0; i < AL && i <= w; i++) {
-      unsigned long long pr = (unsigned long long)A[i] * B[w - i];
-      lo += pr & 0xffffffffull;
-      hi += pr >> 32;
-    }
-    colsum[2 * w] = lo;
-    colsum[2 * w + 1] = hi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long carry = 0;  // < 2^40
-    for (unsigned long long w = 0; w < CL; w++) {
-      unsigned long long v = carry;
-      if (w < W) v += colsum[2 * w];
-      if (w >= 1 && w - 1 < W) v += colsum[2 * (w - 1) + 1];
-      if (D && w < DL) v += D[w];
-      C[w] = (uint32_t)v;
-      carry = v >> 32;
-    }
-  }
-}
-
 int basecase_dev(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL,
                  hipStream_t s, const uint32_t *D = nullptr, size_t DL = 0) {
   if (AL + BL > 4000) return fail(BCG_E_ARG, "basecase limited to AL + BL <= 4000 words");
-  size_t sh = (AL + BL + 1) * 2 * sizeof(unsigned long long);
-  // an output overlapping an input (in-place products) goes through a scratch;
-  // otherwise the kernel writes C directly
+  const bool stage = AL + BL <= (size_t)BASECASE_STAGE;
+  const size_t sh = (AL + BL + 1) * 2 * sizeof(unsigned long long) + (stage ? (AL + BL) * sizeof(uint32_t) : 0);
+  // an output overlapping an input the kernel reads while it writes goes through
+  // a scratch (staged operands are read before the first word is written)
   const uintptr_t c0 = (uintptr_t)C, c1 = c0 + CL * sizeof(uint32_t);
   auto overlaps = [&](const uint32_t *x, size_t n) {
     return x && n && (uintptr_t)x < c1 && c0 < (uintptr_t)(x + n);
   };
-  const bool via_scratch = overlaps(A, AL) || overlaps(B, BL) || overlaps(D, DL);
+  const bool via_scratch = (!stage && (overlaps(A, AL) || overlaps(B, BL))) || overlaps(D, DL);
   uint32_t *dst = C;
   if (via_scratch) {
     if (int rc = ensure(g.zbuf, CL * sizeof(uint32_t) + 64)) return rc;
@@ -1239,8 +1210,15 @@ int basecase_dev(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
   }
   {
     ProfScope ps(BCG_K_OTHER, s);
-    hipLaunchKernelGGL(k_basecase, dim3(1), dim3(256), sh, s, A, (unsigned long long)AL, B,
-                       (unsigned long long)BL, dst, (unsigned long long)CL, D, (unsigned long long)DL);
+    if (AL + BL <= 128)
+      hipLaunchKernelGGL((k_basecase<128, true>), dim3(1), dim3(128), sh, s, A, (int)AL, B, (int)BL, dst,
+                         (unsigned long long)CL, D, (unsigned long long)DL);
+    else if (stage)
+      hipLaunchKernelGGL((k_basecase<256, true>), dim3(1), dim3(256), sh, s, A, (int)AL, B, (int)BL, dst,
+                         (unsigned long long)CL, D, (unsigned long long)DL);
+    else
+      hipLaunchKernelGGL((k_basecase<256, false>), dim3(1), dim3(256), sh, s, A, (int)AL, B, (int)BL, dst,
+                         (unsigned long long)CL, D, (unsigned long long)DL);
   }
   HIPCHK(hipGetLastError());
   if (via_scratch) HIPCHK(hipMemcpyAsync(C, dst, CL * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));

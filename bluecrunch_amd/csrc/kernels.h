@@ -1669,20 +1669,68 @@ __global__ __launch_bounds__((Row<L>::T)) void k_mul1(ClassArgs ca) {
 
 namespace bcg {
 
-// Batched schoolbook products (CL < 100 words, AL + BL <= 128): one wave per
-// product; lane w sums column w of 32x32-bit partial products (low and high
-// halves apart), lane 0 then runs the carry chain, adding the optional addend.
-static __global__ __launch_bounds__(64) void k_basecase_batch(const MulDesc *desc, int count) {
-  __shared__ unsigned long long lo[128], hi[128];
-  const int p = blockIdx.x;
-  if (p >= count) return;
-  const MulDesc d = desc[p];
-  const int W = (int)(d.al + d.bl);
-  for (int w = threadIdx.x; w < W; w += 64) {
+// out[w] = low word of val(w) + carries for w < n (val < 2^32 + 2^31, carry-in
+// cin), each of the workgroup's T threads a run of consecutive words; returns 1 +
+// the highest nonzero index (0: none), the same in every thread. What val reads
+// may be overwritten only after the return.
+template <int T, class F>
+__device__ long long wg_carry_words(uint32_t *out, long long n, unsigned cin, F val) {
+  constexpr int W = T / 64;
+  __shared__ unsigned fn[W];
+  __shared__ long long tops[W];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long long per = (n + T - 1) / T, w0 = tid * per, w1 = w0 + per < n ? w0 + per : n;
+  unsigned c0 = 0, c1 = 1;
+  for (long long w = w0; w < w1; w++) {
+    const unsigned long long v = val(w);
+    c0 = (unsigned)((v + c0) >> 32);
+    c1 = (unsigned)((v + c1) >> 32);
+  }
+  unsigned inc = w0 < w1 ? c0 | (c1 << 1) : 2u;
+  for (int off = 1; off < 64; off <<= 1) {
+    const unsigned g1 = __shfl_up(inc, off, 64);
+    if (lane >= off) inc = carry_compose(g1, inc);
+  }
+  unsigned excl = __shfl_up(inc, 1, 64);
+  if (lane == 0) excl = 2u;
+  if (lane == 63) fn[wave] = inc;
+  __syncthreads();
+  unsigned pre = 2u;
+  for (int w = 0; w < wave; w++) pre = carry_compose(pre, fn[w]);
+  unsigned c = (carry_compose(pre, excl) >> cin) & 1u;
+  long long top = 0;
+  for (long long w = w0; w < w1; w++) {
+    const unsigned long long v = val(w) + c;
+    c = (unsigned)(v >> 32);
+    out[w] = (uint32_t)v;
+    if ((uint32_t)v) top = w + 1;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    const long long o = __shfl_xor(top, off, 64);
+    top = o > top ? o : top;
+  }
+  if (lane == 0) tops[wave] = top;
+  __syncthreads();
+  for (int w = 0; w < W; w++) top = tops[w] > top ? tops[w] : top;
+  __syncthreads();
+  return top;
+}
+
+// Schoolbook product (+ addend) of one workgroup from operands a, b (in LDS, or
+// in global memory): thread w sums column w of 32x32-bit products, low and high
+// halves apart, and the carry chain is a scan over the threads. One thread
+// walking the chain was 5 of 8 us at 43 words.
+template <int T>
+__device__ void wg_basecase(uint32_t *C, unsigned long long CL, const uint32_t *a, int al, const uint32_t *b, int bl,
+                            const uint32_t *D, unsigned long long DL, unsigned long long *lo,
+                            unsigned long long *hi) {
+  const int W = al + bl;
+  for (int w = threadIdx.x; w < W; w += T) {
+    const int i0 = w >= bl ? w - bl + 1 : 0, i1 = w < al ? w : al - 1;
     unsigned long long l = 0, h = 0;
-    int i0 = w >= (int)d.bl ? w - (int)d.bl + 1 : 0;
-    for (int i = i0; i < (int)d.al && i <= w; i++) {
-      unsigned long long pr = (unsigned long long)d.a[i] * d.b[w - i];
+#pragma unroll 4
+    for (int i = i0; i <= i1; i++) {
+      const unsigned long long pr = (unsigned long long)a[i] * b[w - i];
       l += pr & 0xffffffffull;
       h += pr >> 32;
     }
@@ -1690,21 +1738,45 @@ static __global__ __launch_bounds__(64) void k_basecase_batch(const MulDesc *des
     hi[w] = h;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long carry = 0;
-    for (unsigned long long w = 0; w < d.cl; w++) {
-      unsigned long long v = carry;
-      if (w < (unsigned long long)W) v += lo[w];
-      if (w >= 1 && w - 1 < (unsigned long long)W) v += hi[w - 1];
-      if (d.d && w < d.dl) v += d.d[w];
-      d.c[w] = (uint32_t)v;
-      carry = v >> 32;
-    }
-  }
+  auto P = [&](long long w) {
+    unsigned long long v = w >= 0 && w < W ? lo[w] : 0ull;
+    if (w >= 1 && w - 1 < W) v += hi[w - 1];
+    if (D && w >= 0 && (unsigned long long)w < DL) v += D[w];
+    return v;
+  };
+  wg_carry_words<T>(C, (long long)CL, 0u,
+                    [&](long long w) { return (P(w) & 0xffffffffull) + (P(w - 1) >> 32); });
 }
 
-}  // namespace bcg
+// Batched schoolbook products (AL + BL < 100 words): one wave per product.
+static __global__ __launch_bounds__(64) void k_basecase_batch(const MulDesc *desc, int count) {
+  __shared__ unsigned long long lo[128], hi[128];
+  __shared__ uint32_t ab[128];
+  const int p = blockIdx.x;
+  if (p >= count) return;
+  const MulDesc d = desc[p];
+  const int al = (int)d.al, bl = (int)d.bl;
+  for (int i = threadIdx.x; i < al + bl; i += 64) ab[i] = i < al ? d.a[i] : d.b[i - al];
+  __syncthreads();
+  wg_basecase<64>(d.c, d.cl, ab, al, ab + al, bl, d.d, d.dl, lo, hi);
+}
 
-namespace bcg {
+// One schoolbook product. STAGE: the operands go through LDS (al + bl <=
+// BASECASE_STAGE), so C may be A or B.
+constexpr int BASECASE_STAGE = 1024;
+template <int T, bool STAGE>
+__global__ __launch_bounds__(T) void k_basecase(const uint32_t *A, int al, const uint32_t *B, int bl, uint32_t *C,
+                                                unsigned long long CL, const uint32_t *D, unsigned long long DL) {
+  extern __shared__ unsigned long long dyn[];
+  unsigned long long *lo = dyn, *hi = dyn + (al + bl);
+  if constexpr (STAGE) {
+    uint32_t *ab = reinterpret_cast<uint32_t *>(dyn + 2 * (al + bl));
+    for (int i = threadIdx.x; i < al + bl; i += T) ab[i] = i < al ? A[i] : B[i - al];
+    __syncthreads();
+    wg_basecase<T>(C, CL, ab, al, ab + al, bl, D, DL, lo, hi);
+  } else {
+    wg_basecase<T>(C, CL, A, al, B, bl, D, DL, lo, hi);
+  }
+}
 
 }  // namespace bcg
