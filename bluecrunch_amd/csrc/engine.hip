@@ -494,12 +494,9 @@ int grid_for(unsigned long long n);
 
 // Smallest 2^k or 3*2^k >= n (fft/fft.c:22-41 length classes), at least 64.
 unsigned long long class_ceil(unsigned long long n) {
-  unsigned long long b = 32;
-  for (;;) {
-    if (2 * b >= n) return 2 * b;
-    if (3 * b >= n) return 3 * b;
-    b *= 2;
-  }
+  if (n <= 64) return 64;
+  const unsigned long long p2 = 1ull << (64 - __builtin_clzll(n - 1));  // smallest 2^k >= n
+  return p2 / 4 * 3 >= n ? p2 / 4 * 3 : p2;
 }
 
 int ilog2u(unsigned long long v) { return v ? 63 - __builtin_clzll(v) : 0; }
@@ -635,8 +632,19 @@ std::vector<Plan> factor_candidates(unsigned long long N) {
 // single products (bcg_autotune, bcg_autotune_classes) and for the products of
 // batched calls (bcg_autotune_classes), which run every pass over a whole
 // length class at once and may prefer another split.
+// plans_changed() follows every change of either.
 std::map<unsigned long long, int> g_tuned;
 std::map<unsigned long long, int> g_tuned_batch;
+unsigned g_plan_version = 1;
+void plans_changed() { g_plan_version++; }
+
+// Index of a length class: 2^k -> 2 k, 3 * 2^(k-1) -> 2 k + 1 (-1: no class).
+constexpr int CLASSES = 128;
+int class_id(unsigned long long N) {
+  const int k = ilog2u(N);
+  if (N == (1ull << k)) return 2 * k;
+  return k >= 1 && N == (3ull << (k - 1)) ? 2 * k + 1 : -1;
+}
 
 // Untuned choice, from every split timed for one product of each length on one
 // MI355X (the best and the chosen one lie within 4 % from 2^19 points up, and
@@ -695,42 +703,44 @@ int default_candidate(const std::vector<Plan> &c, bool batched = false) {
   return best < 0 ? 0 : best;
 }
 
-bool factor(unsigned long long N, Plan &p) {
-  std::vector<Plan> c = factor_candidates(N);
-  if (c.empty()) return false;
-  int idx = default_candidate(c);
-  auto it = g_tuned.find(N);
-  if (it != g_tuned.end() && it->second >= 0 && it->second < (int)c.size()) idx = it->second;
-  int bits = p.bits;
-  unsigned long long dA = p.dA, dB = p.dB;
-  p = c[idx];
-  p.bits = bits;
-  p.dA = dA;
-  p.dB = dB;
-  return true;
-}
-
 // Split cache: factor_candidates is only built once per transform length.
 std::map<unsigned long long, std::vector<Plan>> g_cands;
 
+// The split in use for N, from a table per length class that a change of the
+// tuned choices empties: batch planning asks once per product.
 bool factor_cached(unsigned long long N, Plan &p, bool batched = false) {
-  auto it = g_cands.find(N);
-  if (it == g_cands.end()) it = g_cands.emplace(N, factor_candidates(N)).first;
-  const std::vector<Plan> &c = it->second;
-  if (c.empty()) return false;
-  int idx = default_candidate(c, batched);
-  auto t = g_tuned.find(N);
-  if (t != g_tuned.end() && t->second >= 0 && t->second < (int)c.size()) idx = t->second;
-  if (batched) {
-    auto tb = g_tuned_batch.find(N);
-    if (tb != g_tuned_batch.end() && tb->second >= 0 && tb->second < (int)c.size()) idx = tb->second;
+  struct Entry {
+    unsigned version = 0;
+    Plan plan;
+  };
+  static Entry memo[2][CLASSES];
+  const int id = class_id(N);
+  Entry *e = id >= 0 ? &memo[batched ? 1 : 0][id] : nullptr;
+  Plan found;
+  if (e && e->version == g_plan_version) {
+    found = e->plan;
+  } else {
+    auto it = g_cands.find(N);
+    if (it == g_cands.end()) it = g_cands.emplace(N, factor_candidates(N)).first;
+    const std::vector<Plan> &c = it->second;
+    if (c.empty()) return false;
+    int idx = default_candidate(c, batched);
+    auto t = g_tuned.find(N);
+    if (t != g_tuned.end() && t->second >= 0 && t->second < (int)c.size()) idx = t->second;
+    if (batched) {
+      auto tb = g_tuned_batch.find(N);
+      if (tb != g_tuned_batch.end() && tb->second >= 0 && tb->second < (int)c.size()) idx = tb->second;
+    }
+    found = c[idx];
+    if (e) {
+      e->plan = found;
+      e->version = g_plan_version;
+    }
   }
-  int bits = p.bits;
-  unsigned long long dA = p.dA, dB = p.dB;
-  p = c[idx];
-  p.bits = bits;
-  p.dA = dA;
-  p.dB = dB;
+  found.bits = p.bits;
+  found.dA = p.dA;
+  found.dB = p.dB;
+  p = found;
   return true;
 }
 
@@ -1304,7 +1314,14 @@ int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t
 // addresses).
 struct BatchBufs {
   DevBuf tdesc, mdesc, cdesc, margins, tA, tB, blk;
+  // pinned: the descriptors and margins of a short plain call, which its kernels
+  // read and write in host memory (see batch_upload)
+  char *host = nullptr, *host_dev = nullptr;
+  size_t host_bytes = 0;
   void release() {
+    if (host) (void)hipHostFree(host);
+    host = host_dev = nullptr;
+    host_bytes = 0;
     for (DevBuf *b : {&tdesc, &mdesc, &cdesc, &margins, &tA, &tB, &blk}) {
       if (b->p) (void)hipFree(b->p);
       b->p = nullptr;
@@ -1661,7 +1678,7 @@ int transform_dev(double *z, size_t length, bool inverse, hipStream_t s) {
   }
   Plan p;
   p.N = length;
-  if (!factor(length, p)) return fail(BCG_E_ARG, "no transform plan for this length");
+  if (!factor_cached(length, p)) return fail(BCG_E_ARG, "no transform plan for this length");
   for (int i = 0; i < p.P; i++)
     if (i == p.P - 1) p.C[i] = 1;
   PassArgs a;
@@ -2128,20 +2145,21 @@ int bcg_basecase_host(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, cons
 namespace {
 
 // One batch call, planned on the host: tiny products (one wave each),
-// one-pass products grouped by length class (one persistent k_mul1 launch per
-// class), multi-pass products grouped by transform length (one launch per
-// pass, the product in grid.y), and the products that go alone (aliasing or
-// empty operands).
+// one-pass products grouped by length class (one k_mul1 launch per class),
+// multi-pass products grouped by transform length (one launch per pass, the
+// product in grid.y), and the products that go alone (aliasing or empty
+// operands).
 struct BatchPlan {
   std::vector<MulDesc> tiny, mdesc, cdesc;
   std::vector<std::pair<Plan, std::pair<size_t, size_t>>> mgroups;  // plan, (first, count) in mdesc
   std::vector<std::pair<int, std::pair<size_t, size_t>>> cgroups;   // L, (first, count) in cdesc
   std::vector<size_t> morder, corder, single;                        // product index of each entry
-  std::vector<Plan> plans;
+  std::vector<unsigned long long> points;                            // transform length of product i
   // the call's arguments (kept for the products re-run alone)
   uint32_t *C = nullptr;
   const uint32_t *A = nullptr, *B = nullptr, *D = nullptr;
   std::vector<size_t> c_off, cl, a_off, al, b_off, bl, d_off, dl;
+  bool host_desc = false;  // descriptors and margins in pinned host memory
 };
 
 int batch_plan(BatchPlan &bp, uint32_t *C, const uint32_t *A, const uint32_t *B, const uint32_t *D,
@@ -2166,82 +2184,129 @@ int batch_plan(BatchPlan &bp, uint32_t *C, const uint32_t *A, const uint32_t *B,
       bp.d_off[i] = d_off ? d_off[i] : 0;
     }
   }
-  bp.plans.assign(count, Plan());
-  auto desc_of = [&](size_t i, const Plan *pl) {
-    MulDesc d;
-    d.a = A + a_off[i];
-    d.b = B + b_off[i];
-    d.c = C + c_off[i];
-    d.d = bp.dl[i] ? D + bp.d_off[i] : nullptr;
-    d.al = al[i];
-    d.bl = bl[i];
-    d.cl = cl[i];
-    d.dl = bp.dl[i];
-    d.bits = pl ? pl->bits : 0;
-    d.cbits = pl ? coef_bits(*pl) : 0;
-    d.gk = (pl && pl->P >= 2) ? group_words_for(pl->C[0], d.bits, d.cbits) : 0;
-    return d;
+  bp.points.assign(count, 0);
+  // every product's descriptor in call order, then gathered by class; a length
+  // pair met again (the products of one tree level mostly share theirs) is
+  // found in a direct-mapped table instead of planned again
+  struct Known {
+    size_t al = 0, bl = 0;
+    unsigned long long N = 0;
+    int bits = 0, cbits = 0, gk = 0;
   };
-  std::map<int, std::vector<size_t>> classes;
-  std::map<unsigned long long, std::vector<size_t>> mclasses;
-  // the products of one tree level mostly share their lengths: plan each
-  // length pair once
-  std::map<std::pair<size_t, size_t>, Plan> plan_of;
+  constexpr int KNOWN = 64;
+  Known known[KNOWN];
+  std::vector<MulDesc> all(count);
+  std::vector<signed char> cls(count, -1);  // class_id of an FFT product
+  size_t in_class[CLASSES] = {0};
   for (size_t i = 0; i < count; i++) {
     const uint32_t *pa = A + a_off[i];
     const uint32_t *pb = B + b_off[i];
     uint32_t *pc = C + c_off[i];
     const uint32_t *pd = bp.dl[i] ? D + bp.d_off[i] : nullptr;
-    bool alias = (pc == pa || pc == pb);
+    const bool alias = (pc == pa || pc == pb);
     if (pd && pd == pc) return fail(BCG_E_ARG, "an addend may not alias its output");
     if (al[i] == 0 || bl[i] == 0 || cl[i] == 0) {
       bp.single.push_back(i);
       continue;
     }
+    MulDesc &d = all[i];
+    d.a = pa;
+    d.b = pb;
+    d.c = pc;
+    d.d = pd;
+    d.al = al[i];
+    d.bl = bl[i];
+    d.cl = cl[i];
+    d.dl = bp.dl[i];
+    d.bits = d.cbits = d.gk = 0;
     if (al[i] + bl[i] < 100) {
       if (alias || cl[i] > 4096)
         bp.single.push_back(i);
       else
-        bp.tiny.push_back(desc_of(i, nullptr));
+        bp.tiny.push_back(d);
       continue;
     }
-    auto pit = plan_of.find({al[i], bl[i]});
-    if (pit == plan_of.end()) {
+    Known &k = known[(al[i] * 7 + bl[i]) % KNOWN];
+    if (k.al != al[i] || k.bl != bl[i]) {
       Plan pl;
       if (int rc = make_plan(al[i], bl[i], 0, pl, true)) return rc;
-      pit = plan_of.emplace(std::make_pair(al[i], bl[i]), pl).first;
+      k.al = al[i];
+      k.bl = bl[i];
+      k.N = pl.N;
+      k.bits = pl.bits;
+      k.cbits = coef_bits(pl);
+      k.gk = pl.P >= 2 ? group_words_for(pl.C[0], k.bits, k.cbits) : 0;
     }
-    bp.plans[i] = pit->second;
-    if (alias)
+    d.bits = k.bits;
+    d.cbits = k.cbits;
+    d.gk = k.gk;
+    bp.points[i] = k.N;
+    if (alias) {
       bp.single.push_back(i);
-    else if (bp.plans[i].P == 1)
-      classes[bp.plans[i].L[0]].push_back(i);
-    else
-      mclasses[bp.plans[i].N].push_back(i);
-  }
-  for (auto &kv : mclasses) {
-    const size_t first = bp.mdesc.size();
-    for (size_t i : kv.second) {
-      bp.mdesc.push_back(desc_of(i, &bp.plans[i]));
-      bp.morder.push_back(i);
+      continue;
     }
-    bp.mgroups.push_back({bp.plans[kv.second[0]], {first, kv.second.size()}});  // same N and pass split
+    cls[i] = (signed char)class_id(k.N);
+    in_class[cls[i]]++;
   }
-  for (auto &kv : classes) {
-    const size_t first = bp.cdesc.size();
-    for (size_t i : kv.second) {
-      bp.cdesc.push_back(desc_of(i, &bp.plans[i]));
-      bp.corder.push_back(i);
+  // classes in order of length; within one, the call's order
+  size_t at[CLASSES];
+  for (int c = 0; c < CLASSES; c++) {
+    if (!in_class[c]) continue;
+    Plan pl;
+    const unsigned long long N = c & 1 ? 3ull << (c / 2 - 1) : 1ull << (c / 2);
+    if (!factor_cached(N, pl, true)) return fail(BCG_E_ARG, "no pass split for this length");
+    if (pl.P == 1) {
+      at[c] = bp.cdesc.size();
+      bp.cgroups.push_back({pl.L[0], {at[c], in_class[c]}});
+      bp.cdesc.resize(at[c] + in_class[c]);
+      bp.corder.resize(bp.cdesc.size());
+    } else {
+      at[c] = bp.mdesc.size();
+      bp.mgroups.push_back({pl, {at[c], in_class[c]}});
+      bp.mdesc.resize(at[c] + in_class[c]);
+      bp.morder.resize(bp.mdesc.size());
+      in_class[c] |= (size_t)1 << 63;  // a multi-pass class
     }
-    bp.cgroups.push_back({kv.first, {first, kv.second.size()}});
+  }
+  for (size_t i = 0; i < count; i++) {
+    if (cls[i] < 0) continue;
+    const int c = cls[i];
+    const size_t k = at[c]++;
+    if (in_class[c] >> 63) {
+      bp.mdesc[k] = all[i];
+      bp.morder[k] = i;
+    } else {
+      bp.cdesc[k] = all[i];
+      bp.corder[k] = i;
+    }
   }
   return 0;
 }
 
-// Descriptors to the device and scratch sized (no allocation afterwards).
-int batch_upload(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
-  const size_t nm = bp.mdesc.size(), nc = bp.cdesc.size();
-  if (int rc = ensure(bb.tdesc, bp.tiny.size() * sizeof(MulDesc))) return rc;
+// A plain call of one-pass and tiny products only, at most this many, reads its
+// descriptors from pinned host memory and writes its margins there: copies in
+// and out are a launch, a gap and a wait each (256 products: 30 us of the
+// call). A workgroup's read over the link is about 2 us, so longer calls, whose
+// workgroups follow each other on a CU, and replayed ones keep device copies.
+constexpr size_t HOST_DESC_MAX = 512;
+
+// Descriptors to the device (or pinned host memory) and scratch sized (no
+// allocation afterwards). keep_dev: a captured batch's descriptors stay on the device.
+int batch_upload(BatchPlan &bp, BatchBufs &bb, hipStream_t s, bool keep_dev) {
+  const size_t nt = bp.tiny.size(), nm = bp.mdesc.size(), nc = bp.cdesc.size();
+  bp.host_desc = !keep_dev && nm == 0 && nt + nc <= HOST_DESC_MAX;
+  if (bp.host_desc) {
+    const size_t want = HOST_DESC_MAX * (sizeof(MulDesc) + sizeof(unsigned int));
+    if (!bb.host) {
+      HIPCHK(hipHostMalloc((void **)&bb.host, want, hipHostMallocMapped));
+      HIPCHK(hipHostGetDevicePointer((void **)&bb.host_dev, bb.host, 0));
+      bb.host_bytes = want;
+    }
+    if (nc) memcpy(bb.host, bp.cdesc.data(), nc * sizeof(MulDesc));
+    if (nt) memcpy(bb.host + nc * sizeof(MulDesc), bp.tiny.data(), nt * sizeof(MulDesc));
+    return 0;
+  }
+  if (int rc = ensure(bb.tdesc, nt * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.mdesc, nm * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.cdesc, nc * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.margins, (nm + nc) * sizeof(unsigned int))) return rc;
@@ -2260,8 +2325,8 @@ int batch_upload(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
     if (int rc = ensure(bb.tB, arr)) return rc;
     if (int rc = ensure(bb.blk, blk)) return rc;
   }
-  if (!bp.tiny.empty())
-    if (int rc = h2d(bb.tdesc.p, bp.tiny.data(), bp.tiny.size() * sizeof(MulDesc), s)) return rc;
+  if (nt)
+    if (int rc = h2d(bb.tdesc.p, bp.tiny.data(), nt * sizeof(MulDesc), s)) return rc;
   if (nm)
     if (int rc = h2d(bb.mdesc.p, bp.mdesc.data(), nm * sizeof(MulDesc), s)) return rc;
   if (nc)
@@ -2269,22 +2334,40 @@ int batch_upload(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
   return 0;
 }
 
-// Every batched launch of the plan, kernels only (capturable).
-int batch_launch(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
+// Every batched launch of the plan, kernels only (capturable). margins: where the
+// products' margins go (multi-pass ones, then one-pass ones), device addresses.
+int batch_launch(const BatchPlan &bp, BatchBufs &bb, hipStream_t s, unsigned int *margins) {
   const size_t nm = bp.mdesc.size(), nc = bp.cdesc.size();
-  unsigned int *mm = (unsigned int *)bb.margins.p, *cm = mm + nm;
-  HIPCHK(hipGetLastError());
-  // one-pass length classes: independent persistent launches, spread over the
-  // side streams (largest class first), beside the multi-pass groups on s, so
-  // that small classes do not leave the GPU idle one after another; the tiny
-  // products go to a side stream too; joined back into s at the end. The
-  // multi-pass groups, the longest chain of dependent launches, are issued
-  // first (4096-product replay 1.27-1.28 -> 1.26 ms; issuing the largest
-  // one-pass classes ahead of them measured 1.30 ms).
-  const bool fork = !bp.cgroups.empty() || (!bp.tiny.empty() && !bp.mgroups.empty());
-  if (fork) {
+  unsigned int *mm = margins, *cm = mm + nm;
+  const MulDesc *cdesc = (const MulDesc *)(bp.host_desc ? (void *)bb.host_dev : bb.cdesc.p);
+  const MulDesc *tdesc = bp.host_desc ? cdesc + nc : (const MulDesc *)bb.tdesc.p;
+  // one-pass length classes: independent launches, spread over the side streams
+  // (largest class first), beside the multi-pass groups on s, so that small
+  // classes do not leave the GPU idle one after another; the tiny products take
+  // the next stream in turn; joined back into s at the end. The multi-pass
+  // groups, the longest chain of dependent launches, are issued first
+  // (4096-product replay 1.27-1.28 -> 1.26 ms; issuing the largest one-pass
+  // classes ahead of them measured 1.30 ms). Without them s takes the first
+  // class itself, and no more side streams are forked than there are launches
+  // for: a fork and join of all three was 15 us of a one-class call.
+  std::vector<int> order(bp.cgroups.size());
+  for (size_t k = 0; k < order.size(); k++) order[k] = (int)k;
+  std::sort(order.begin(), order.end(), [&](int x, int y) {
+    const double wx = (double)bp.cgroups[x].second.second * bp.cgroups[x].first;
+    const double wy = (double)bp.cgroups[y].second.second * bp.cgroups[y].first;
+    return wx > wy;
+  });
+  const int launches = (int)order.size() + (bp.tiny.empty() ? 0 : 1);
+  const int own = bp.mgroups.empty() ? 1 : 0;  // s is one of the streams
+  const int naux = std::max(0, std::min((int)Engine::NAUX, launches - own));
+  const int ns = naux + own;
+  auto stream_of = [&](int k) {
+    const int q = k % ns;
+    return own ? (q ? g.aux[q - 1] : s) : g.aux[q];
+  };
+  if (naux) {
     HIPCHK(hipEventRecord(g.fork_ev, s));
-    for (int i = 0; i < Engine::NAUX; i++) HIPCHK(hipStreamWaitEvent(g.aux[i], g.fork_ev, 0));
+    for (int i = 0; i < naux; i++) HIPCHK(hipStreamWaitEvent(g.aux[i], g.fork_ev, 0));
   }
   int rc = 0;
   for (auto &gr : bp.mgroups) {
@@ -2293,60 +2376,51 @@ int batch_launch(const BatchPlan &bp, BatchBufs &bb, hipStream_t s) {
     rc = run_multipass_class(gr.first, (const MulDesc *)bb.mdesc.p + first, hd, mm + first, s, bb);
     if (rc) break;
   }
-  if (!rc && fork) {
-    std::vector<int> order(bp.cgroups.size());
-    for (size_t k = 0; k < order.size(); k++) order[k] = (int)k;
-    std::sort(order.begin(), order.end(), [&](int x, int y) {
-      const double wx = (double)bp.cgroups[x].second.second * bp.cgroups[x].first;
-      const double wy = (double)bp.cgroups[y].second.second * bp.cgroups[y].first;
-      return wx > wy;
-    });
-    for (size_t k = 0; k < order.size() && !rc; k++) {
-      const int ci = order[k];
-      const auto &gr = bp.cgroups[ci];
-      const size_t first = gr.second.first, n = gr.second.second;
-      ClassArgs ca;
-      memset(&ca, 0, sizeof ca);
-      ca.desc = (const MulDesc *)bb.cdesc.p + first;
-      ca.margins = cm + first;
-      rc = run_class(gr.first, ca, (int)n, g.aux[k % Engine::NAUX]);
-    }
+  for (size_t k = 0; k < order.size() && !rc; k++) {
+    const auto &gr = bp.cgroups[order[k]];
+    const size_t first = gr.second.first, n = gr.second.second;
+    ClassArgs ca;
+    memset(&ca, 0, sizeof ca);
+    ca.desc = cdesc + first;
+    ca.margins = cm + first;
+    rc = run_class(gr.first, ca, (int)n, stream_of((int)k));
   }
   if (!rc && !bp.tiny.empty()) {
-    hipStream_t ts = fork ? g.aux[bp.cgroups.size() % Engine::NAUX] : s;
+    hipStream_t ts = stream_of((int)order.size());
     ProfScope ps(BCG_K_OTHER, ts);
-    LAUNCH(k_basecase_batch, (int)bp.tiny.size(), 64, ts, (const MulDesc *)bb.tdesc.p, (int)bp.tiny.size());
+    LAUNCH(k_basecase_batch, (int)bp.tiny.size(), 64, ts, tdesc, (int)bp.tiny.size());
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(BCG_E_HIP, "k_basecase_batch", e);
   }
-  if (fork) {  // the side streams rejoin s (also before an error returns)
-    for (int i = 0; i < Engine::NAUX; i++) {
-      HIPCHK(hipEventRecord(g.join_ev[i], g.aux[i]));
-      HIPCHK(hipStreamWaitEvent(s, g.join_ev[i], 0));
-    }
+  for (int i = 0; i < naux; i++) {  // the side streams rejoin s (also before an error returns)
+    HIPCHK(hipEventRecord(g.join_ev[i], g.aux[i]));
+    HIPCHK(hipStreamWaitEvent(s, g.join_ev[i], 0));
   }
   return rc;
 }
 
-// Margins back; products at >= 0.25 re-run alone with b - 1; the products
-// that go alone run now.
-int batch_finish(const BatchPlan &bp, BatchBufs &bb, hipStream_t s, double *worst_margin) {
+// Where the margins of a plan's launches go when nothing else is asked for.
+unsigned int *batch_margins(const BatchPlan &bp, const BatchBufs &bb) {
+  return bp.host_desc ? (unsigned int *)(bb.host_dev + HOST_DESC_MAX * sizeof(MulDesc)) : (unsigned int *)bb.margins.p;
+}
+
+// The margins mb (host copy, after the device is done) of the plan's products
+// judged: products at >= 0.25 re-run alone with b - 1; the products that go
+// alone run now.
+int batch_judge(const BatchPlan &bp, const unsigned int *mb, hipStream_t s, double *worst_margin) {
   double worst = 0;
   const size_t nm = bp.mdesc.size(), nc = bp.cdesc.size();
-  std::vector<size_t> retry;
-  if (nm + nc) {
-    std::vector<unsigned int> mb(nm + nc);
-    if (int rc = d2h(mb.data(), bb.margins.p, (nm + nc) * sizeof(unsigned int), s)) return rc;
-    for (size_t k = 0; k < nm + nc; k++) {
-      float f;
-      memcpy(&f, &mb[k], sizeof f);
-      const size_t i = k < nm ? bp.morder[k] : bp.corder[k - nm];
-      if (f >= 0.25f) {
-        retry.push_back(i);
-      } else {
-        if (f > worst) worst = f;
-        note_product(bp.plans[i].N, bp.plans[i].bits, f);
-      }
+  std::vector<std::pair<size_t, int>> retry;  // product, digit size
+  for (size_t k = 0; k < nm + nc; k++) {
+    float f;
+    memcpy(&f, &mb[k], sizeof f);
+    const size_t i = k < nm ? bp.morder[k] : bp.corder[k - nm];
+    const int bits = k < nm ? bp.mdesc[k].bits : bp.cdesc[k - nm].bits;
+    if (f >= 0.25f) {
+      retry.push_back({i, bits - 1});
+    } else {
+      if (f > worst) worst = f;
+      note_product(bp.points[i], bits, f);
     }
   }
   auto one = [&](size_t i, int force_bits) -> int {
@@ -2360,15 +2434,30 @@ int batch_finish(const BatchPlan &bp, BatchBufs &bb, hipStream_t s, double *wors
   };
   for (size_t i : bp.single)
     if (int rc = one(i, 0)) return rc;
-  for (size_t i : retry) {
-    int fb = bp.plans[i].bits - 1;
-    if (fb < 4) return fail(BCG_E_MARGIN, "rounding margin >= 0.25 at the smallest digit size");
+  for (auto &r : retry) {
+    if (r.second < 4) return fail(BCG_E_MARGIN, "rounding margin >= 0.25 at the smallest digit size");
     g_stats.retries++;
-    if (int rc = one(i, fb)) return rc;
+    if (int rc = one(r.first, r.second)) return rc;
   }
-  HIPCHK(hipStreamSynchronize(s));
+  if (!bp.single.empty() || !retry.empty()) HIPCHK(hipStreamSynchronize(s));
   if (worst_margin) *worst_margin = worst;
   return 0;
+}
+
+// Waits for the plan's launches and judges their margins.
+int batch_finish(const BatchPlan &bp, BatchBufs &bb, hipStream_t s, double *worst_margin) {
+  const size_t n = bp.mdesc.size() + bp.cdesc.size();
+  if (bp.host_desc) {
+    HIPCHK(hipStreamSynchronize(s));
+    return batch_judge(bp, (const unsigned int *)(bb.host + HOST_DESC_MAX * sizeof(MulDesc)), s, worst_margin);
+  }
+  std::vector<unsigned int> mb(n);
+  if (n) {
+    if (int rc = d2h(mb.data(), bb.margins.p, n * sizeof(unsigned int), s)) return rc;
+  } else {
+    HIPCHK(hipStreamSynchronize(s));
+  }
+  return batch_judge(bp, mb.data(), s, worst_margin);
 }
 
 }  // namespace
@@ -2390,8 +2479,11 @@ int bcg_muladd_batch_dev(uint32_t *C, const uint32_t *A, const uint32_t *B, cons
   hipStream_t s = pick(stream);
   BatchPlan bp;
   if (int rc = batch_plan(bp, C, A, B, D, c_off, cl, a_off, al, b_off, bl, d_off, dl, count)) return rc;
-  if (int rc = batch_upload(bp, g_bb, s)) return rc;
-  if (int rc = batch_launch(bp, g_bb, s)) return rc;
+  if (int rc = batch_upload(bp, g_bb, s, false)) return rc;
+  if (int rc = batch_launch(bp, g_bb, s, batch_margins(bp, g_bb))) {
+    (void)hipStreamSynchronize(s);  // nothing launched still reads the descriptors
+    return rc;
+  }
   return batch_finish(bp, g_bb, s, worst_margin);
 }
 
@@ -2405,9 +2497,9 @@ int bcg_batch_create(bcg_batch *batch, uint32_t *C, const uint32_t *A, const uin
   if (!bt) return fail(BCG_E_NOMEM, "batch handle");
   hipStream_t s = g.stream;
   int rc = batch_plan(bt->plan, C, A, B, D, c_off, cl, a_off, al, b_off, bl, d_off, dl, count);
-  if (!rc) rc = batch_upload(bt->plan, bt->bufs, s);
+  if (!rc) rc = batch_upload(bt->plan, bt->bufs, s, true);
   // one eager run: builds every table the kernels read, checks the launches
-  if (!rc) rc = batch_launch(bt->plan, bt->bufs, s);
+  if (!rc) rc = batch_launch(bt->plan, bt->bufs, s, batch_margins(bt->plan, bt->bufs));
   if (!rc) {
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess) rc = fail(BCG_E_HIP, "batch warm-up", e);
@@ -2419,7 +2511,7 @@ int bcg_batch_create(bcg_batch *batch, uint32_t *C, const uint32_t *A, const uin
     if (e != hipSuccess) {
       rc = fail(BCG_E_HIP, "begin capture", e);
     } else {
-      int lrc = batch_launch(bt->plan, bt->bufs, g.cap);
+      int lrc = batch_launch(bt->plan, bt->bufs, g.cap, batch_margins(bt->plan, bt->bufs));
       hipGraph_t graph = nullptr;
       e = hipStreamEndCapture(g.cap, &graph);
       bt->graph = graph;
@@ -2684,10 +2776,12 @@ int bcg_plan_force(size_t N, int index) {
   std::lock_guard<std::recursive_mutex> lk(g_lock);
   if (index < 0) {
     g_tuned.erase(N);
+    plans_changed();
     return 0;
   }
   if (index >= (int)factor_candidates(N).size()) return fail(BCG_E_ARG, "candidate index out of range");
   g_tuned[N] = index;
+  plans_changed();
   return 0;
 }
 
@@ -2729,6 +2823,7 @@ int bcg_autotune(size_t AL, size_t BL, int square, int reps, int *chosen, double
   auto saved = g_tuned.find(N) != g_tuned.end() ? g_tuned[N] : -1;
   for (int i = 0; i < (int)cands.size() && !rc; i++) {
     g_tuned[N] = i;
+    plans_changed();
     bcg_mul_info inf;
     rc = mul_dev_locked(dC, AL + BL, dA, AL, pB, BL, 0, s, &inf);  // warm-up (tables, buffers)
     if (rc) break;
@@ -2750,6 +2845,7 @@ int bcg_autotune(size_t AL, size_t BL, int square, int reps, int *chosen, double
   } else {
     g_tuned[N] = best;
   }
+  plans_changed();
   g.free_events.push_back(e0);
   g.free_events.push_back(e1);
   (void)hipFree(dA);
@@ -2794,13 +2890,14 @@ int time_batch(size_t w, int count, int reps, uint32_t *dA, uint32_t *dB, uint32
   if (int rc = batch_plan(bp, dC, dA, dB, nullptr, off.data(), cl.data(), ab_off.data(), len.data(), ab_off.data(),
                           len.data(), nullptr, nullptr, (size_t)count))
     return rc;
-  if (int rc = batch_upload(bp, g_bb, s)) return rc;
-  if (int rc = batch_launch(bp, g_bb, s)) return rc;  // warm-up
+  if (int rc = batch_upload(bp, g_bb, s, true)) return rc;
+  unsigned int *margins = batch_margins(bp, g_bb);
+  if (int rc = batch_launch(bp, g_bb, s, margins)) return rc;  // warm-up
   HIPCHK(hipStreamSynchronize(s));
   hipEvent_t e0 = get_event(), e1 = get_event();
   int rc = 0;
   (void)hipEventRecord(e0, s);
-  for (int r = 0; r < reps && !rc; r++) rc = batch_launch(bp, g_bb, s);
+  for (int r = 0; r < reps && !rc; r++) rc = batch_launch(bp, g_bb, s, margins);
   (void)hipEventRecord(e1, s);
   (void)hipEventSynchronize(e1);
   float t = 0;
@@ -2852,6 +2949,7 @@ int bcg_autotune_classes(size_t lo, size_t hi, int reps, int *tuned) {
     const auto saved = g_tuned_batch.find(N) != g_tuned_batch.end() ? g_tuned_batch[N] : -1;
     for (int i = 0; i < nc && !rc; i++) {
       g_tuned_batch[N] = i;
+      plans_changed();
       double ms = 0;
       rc = time_batch(words[k], counts[k], reps, dA, dB, dC, &ms);
       if (!rc && (best < 0 || ms < best_ms)) {
@@ -2866,6 +2964,7 @@ int bcg_autotune_classes(size_t lo, size_t hi, int reps, int *tuned) {
       g_tuned_batch[N] = best;
       done++;
     }
+    plans_changed();
   }
   (void)hipStreamSynchronize(g.stream);
   (void)hipFree(dA);
@@ -2880,10 +2979,12 @@ int bcg_plan_force_batch(size_t N, int index) {
   std::lock_guard<std::recursive_mutex> lk(g_lock);
   if (index < 0) {
     g_tuned_batch.erase(N);
+    plans_changed();
     return 0;
   }
   if (index >= (int)factor_candidates(N).size()) return fail(BCG_E_ARG, "candidate index out of range");
   g_tuned_batch[N] = index;
+  plans_changed();
   return 0;
 }
 

@@ -143,3 +143,29 @@ def test_batch_graph_replays(bc):
             assert np.array_equal(bc.mul(x, y)[0], exact_product(x, y))
     finally:
         batch.close()
+
+
+@pytest.mark.parametrize("count", [1, 2, 511, 512, 513])
+@pytest.mark.parametrize("bias", [0, 6])
+def test_plain_calls_around_the_host_descriptor_limit(bc, count, bias):
+    # calls of at most 512 one-pass and schoolbook products read descriptors and
+    # write margins in host memory; with a digit bias products re-run from there
+    from bluecrunch_amd.workload import operands
+    sizes = [(10, 20), (300, 200), (5000, 4500), (49, 50), (1000, 100), (3000, 3000)]
+    pairs = [operands(50 + k % 7, *sizes[(k + 2) % len(sizes)]) for k in range(count)]
+    want = {}
+    bc.plan_digit_bias(bias)
+    try:
+        bc.stats_reset()
+        out, worst = bc.mul_batch(pairs)
+        st = bc.stats()
+    finally:
+        bc.plan_digit_bias(0)
+    for k, (c, (a, b)) in enumerate(zip(out, pairs)):
+        key = (k % 7, (k + 2) % len(sizes))
+        if key not in want:
+            want[key] = exact_product(a, b)
+        assert np.array_equal(c, want[key]), k
+    assert worst < 0.25 and st["products"] == sum(len(a) + len(b) >= 100 for a, b in pairs)
+    assert bias or st["retries"] == 0
+    assert not bias or st["retries"] >= 1
