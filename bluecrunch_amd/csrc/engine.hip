@@ -2460,6 +2460,61 @@ int batch_finish(const BatchPlan &bp, BatchBufs &bb, hipStream_t s, double *wors
   return batch_judge(bp, mb.data(), s, worst_margin);
 }
 
+// Batched calls whose margins are judged together at the end (radix_convert): the
+// levels' launches follow each other on the stream without a wait. The plain
+// call's scratch serves them all in stream order; the margins have a buffer of
+// their own.
+struct RadixBatches {
+  DInt margins;
+  size_t used = 0;
+  std::vector<BatchPlan> plans;
+};
+
+int radix_batch_begin(RadixBatches **rb, size_t products) {
+  RadixBatches *b = new (std::nothrow) RadixBatches;
+  if (!b) return fail(BCG_E_NOMEM, "radix batches");
+  if (int rc = dalloc(b->margins, products)) {
+    delete b;
+    return rc;
+  }
+  *rb = b;
+  return 0;
+}
+
+int radix_batch_run(RadixBatches *rb, uint32_t *C, const uint32_t *A, const uint32_t *B, const size_t *c_off,
+                    const size_t *cl, const size_t *a_off, const size_t *al, const size_t *b_off, const size_t *bl,
+                    size_t count, hipStream_t s) {
+  rb->plans.emplace_back();
+  BatchPlan &bp = rb->plans.back();
+  if (int rc = batch_plan(bp, C, A, B, nullptr, c_off, cl, a_off, al, b_off, bl, nullptr, nullptr, count)) return rc;
+  if (!bp.single.empty()) return fail(BCG_E_ARG, "radix products go through a batch");
+  if (int rc = batch_upload(bp, g_bb, s, true)) return rc;
+  unsigned int *m = (unsigned int *)rb->margins.p + rb->used;
+  rb->used += bp.mdesc.size() + bp.cdesc.size();
+  return batch_launch(bp, g_bb, s, m);
+}
+
+// Waits for the launches; *ok is false when a margin reached 0.25.
+int radix_batch_end(RadixBatches *rb, bool *ok, hipStream_t s) {
+  std::vector<unsigned int> mb(rb->used);
+  int rc = rb->used ? d2h(mb.data(), rb->margins.p, rb->used * sizeof(unsigned int), s) : 0;
+  if (!rc) {
+    for (unsigned int b : mb) {
+      float f;
+      memcpy(&f, &b, sizeof f);
+      if (f >= 0.25f) *ok = false;
+    }
+    const unsigned int *m = mb.data();
+    for (const BatchPlan &bp : rb->plans) {
+      if (*ok) rc = rc ? rc : batch_judge(bp, m, s, nullptr);
+      m += bp.mdesc.size() + bp.cdesc.size();
+    }
+  }
+  dfree(rb->margins);
+  delete rb;
+  return rc;
+}
+
 }  // namespace
 
 // A batch captured once and replayed (see include/bluecrunch_gpu.h).
