@@ -871,6 +871,7 @@ int run_carry(const long long *coef, unsigned long long ncoef, int bits, int cbi
   if (margin) {
     c.host = g.hres_dev;
     c.margin = (const unsigned int *)g.margin.p;
+    c.margin_mask = MARGIN_SLOTS - 1;
     g.hres->open_carry = 0;
   }
   {
@@ -939,6 +940,7 @@ int carry_of_plan(const Plan &p, uint32_t *out, unsigned long long CL, hipStream
   if (margin) {
     c.host = g.hres_dev;
     c.margin = (const unsigned int *)g.margin.p;
+    c.margin_mask = MARGIN_SLOTS - 1;
     g.hres->open_carry = 0;
   }
   {
@@ -962,6 +964,7 @@ int zero_margin(hipStream_t s) {
 // whose output aliases an input, and all products of other threads, check
 // at once as usual.
 constexpr int DEFER_SETS = 64;
+static_assert(DEFER_SETS <= (int)(sizeof(HostResult::set_margin) / sizeof(unsigned)), "a margin per set");
 constexpr size_t MARGIN_SET_BYTES = sizeof(unsigned int) * MARGIN_SLOTS * MARGIN_STRIDE;
 struct DeferScope {
   bool open = false;
@@ -978,7 +981,7 @@ DeferScope g_defer;
 // The margin of a product whose carry has not run (products in place): the
 // host waits for it.
 int read_margin(hipStream_t s, double *m) {
-  LAUNCH(k_margin_out, 1, 64, s, (const unsigned int *)g.margin.p, g.hres_dev);
+  LAUNCH(k_margin_out, 1, 64, s, (const unsigned int *)g.margin.p, &g.hres_dev->margin);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));
   float f;
@@ -1313,7 +1316,7 @@ int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t
 // uses the engine's set; a captured batch owns one (its graph keeps the
 // addresses).
 struct BatchBufs {
-  DevBuf tdesc, mdesc, cdesc, margins, tA, tB, blk;
+  DevBuf tdesc, mdesc, cdesc, margins, slots, tA, tB, blk;
   // pinned: the descriptors and margins of a short plain call, which its kernels
   // read and write in host memory (see batch_upload)
   char *host = nullptr, *host_dev = nullptr;
@@ -1322,7 +1325,7 @@ struct BatchBufs {
     if (host) (void)hipHostFree(host);
     host = host_dev = nullptr;
     host_bytes = 0;
-    for (DevBuf *b : {&tdesc, &mdesc, &cdesc, &margins, &tA, &tB, &blk}) {
+    for (DevBuf *b : {&tdesc, &mdesc, &cdesc, &margins, &slots, &tA, &tB, &blk}) {
       if (b->p) (void)hipFree(b->p);
       b->p = nullptr;
       b->bytes = 0;
@@ -1332,18 +1335,33 @@ struct BatchBufs {
 
 BatchBufs g_bb;  // scratch of the plain batch call
 
+// Margin slots per product of a batched class: one for every four workgroups of
+// its unpacking pass.
+int batch_slots(const Plan &p) {
+  const unsigned long long tiles = p.N / ((unsigned long long)p.L[0] * (unsigned long long)inv_cols(p, 0));
+  int n = 1;
+  while (n < MARGIN_SLOTS && 4ull * (unsigned long long)n < tiles) n *= 2;
+  return n;
+}
+
+size_t batch_slot_bytes(const Plan &p, size_t count) {
+  return count * (size_t)batch_slots(p) * MARGIN_STRIDE * sizeof(unsigned int);
+}
+
 int run_multipass_class(const Plan &p, const MulDesc *ddesc, const std::vector<MulDesc> &hdesc,
                         unsigned int *dmargins, hipStream_t s, BatchBufs &bb) {
   const int count = (int)hdesc.size();
   const size_t arr = (size_t)p.N * sizeof(cd) * (size_t)count;
   if (int rc = ensure(bb.tA, arr)) return rc;
   if (int rc = ensure(bb.tB, arr)) return rc;
+  if (int rc = ensure(bb.slots, batch_slot_bytes(p, (size_t)count))) return rc;
   cd *da = (cd *)bb.tA.p;
   cd *db = (cd *)bb.tB.p;
   PassArgs a;
   memset(&a, 0, sizeof a);
   a.desc = ddesc;
-  a.margin = dmargins;
+  a.margin = (unsigned int *)bb.slots.p;
+  a.margin_mask = batch_slots(p) - 1;
   int fast = 1;  // every product of the class has coefficients below 2^51
   for (const MulDesc &d : hdesc) fast = fast && d.cbits <= 51;
   // both operands' forward passes in one launch each (grid.y = 2 count) while
@@ -1423,6 +1441,9 @@ int run_multipass_class(const Plan &p, const MulDesc *ddesc, const std::vector<M
   CarryArgs c;
   memset(&c, 0, sizeof c);
   c.desc = ddesc;
+  c.margin = a.margin;
+  c.margin_mask = a.margin_mask;
+  c.margin_out = dmargins;
   c.coef_stride = 2 * p.N;
   c.coef = (const long long *)db;
   c.ncoef = 2 * p.N;
@@ -1459,18 +1480,19 @@ int run_multipass_class(const Plan &p, const MulDesc *ddesc, const std::vector<M
 }
 
 // Reads the margin sets of the open deferral scope (after the device is
-// idle), records their products in the statistics and frees the sets.
+// idle), records their products in the statistics and frees the sets. Their
+// maxima are taken on the device: the slots themselves, 8 KiB a set, are a
+// pageable copy of 100 us.
 int defer_flush() {
   DeferScope &d = g_defer;
   if (!d.n) return 0;
   HIPCHK(hipDeviceSynchronize());
-  std::vector<unsigned int> w((size_t)d.n * MARGIN_SLOTS * MARGIN_STRIDE);
-  HIPCHK(hipMemcpy(w.data(), d.sets.p, w.size() * sizeof(unsigned int), hipMemcpyDeviceToHost));
+  LAUNCH(k_margin_out, d.n, 64, g.stream, (const unsigned int *)d.sets.p, g.hres_dev->set_margin);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(g.stream));
   for (int i = 0; i < d.n; i++) {
-    unsigned int b = 0;
-    for (int k = 0; k < MARGIN_SLOTS; k++) b = std::max(b, w[((size_t)i * MARGIN_SLOTS + k) * MARGIN_STRIDE]);
     float f;
-    memcpy(&f, &b, sizeof f);
+    memcpy(&f, &g.hres->set_margin[i], sizeof f);
     d.worst = std::max(d.worst, (double)f);
     note_product(d.points[i], d.bits[i], (double)f);
   }
@@ -2310,10 +2332,11 @@ int batch_upload(BatchPlan &bp, BatchBufs &bb, hipStream_t s, bool keep_dev) {
   if (int rc = ensure(bb.mdesc, nm * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.cdesc, nc * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.margins, (nm + nc) * sizeof(unsigned int))) return rc;
-  size_t arr = 0, blk = 16;
+  size_t arr = 0, blk = 16, slots = 0;
   for (auto &gr : bp.mgroups) {
     const Plan &p = gr.first;
     arr = std::max(arr, (size_t)p.N * sizeof(cd) * gr.second.second);
+    slots = std::max(slots, batch_slot_bytes(p, gr.second.second));
     const unsigned long long wpb = (unsigned long long)CT * CWPT;
     unsigned long long nb = 1;
     for (size_t k = 0; k < gr.second.second; k++)
@@ -2324,6 +2347,7 @@ int batch_upload(BatchPlan &bp, BatchBufs &bb, hipStream_t s, bool keep_dev) {
     if (int rc = ensure(bb.tA, arr)) return rc;
     if (int rc = ensure(bb.tB, arr)) return rc;
     if (int rc = ensure(bb.blk, blk)) return rc;
+    if (int rc = ensure(bb.slots, slots)) return rc;
   }
   if (nt)
     if (int rc = h2d(bb.tdesc.p, bp.tiny.data(), nt * sizeof(MulDesc), s)) return rc;

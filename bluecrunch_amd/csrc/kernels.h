@@ -34,7 +34,7 @@ struct PassArgs {
   int bits;                 // digit size
   int ntiles;
   unsigned int *margin;     // float bits of the worst |x - round(x)| (atomic max; zeroed by the packing pass)
-  int margin_mask;          // single products: slot (block & mask) * MARGIN_STRIDE; batched: 0
+  int margin_mask;          // slot (block & mask) * MARGIN_STRIDE; batched: mask + 1 slots per product
   double inv_n;
   int fast_round;           // every coefficient < 2^51: round with the 1.5 * 2^52 addition
   const MulDesc *desc;      // batched launch: product blockIdx.y, else nullptr
@@ -47,6 +47,15 @@ struct PassArgs {
   int lower;                // packing pass of single products: every operand leaves the upper half empty
   unsigned long long ystride;  // batched group mode: group-sum words per product in ybuf
 };
+
+// Margin slots: a product spreads its atomics over up to MARGIN_SLOTS
+// addresses MARGIN_STRIDE words apart (one 128-byte line each), so that its
+// workgroups, which mostly end together, do not serialise on one address: with
+// one word per product the atomics of 2048 waves on two products took longer
+// than their unpacking pass (37 us against 19 us). The carry takes the
+// maximum over the slots (margin_of_slots) to where the host reads it.
+constexpr int MARGIN_SLOTS = 64;
+constexpr int MARGIN_STRIDE = 32;
 
 // Batched launches (desc != nullptr): product p = blockIdx.y owns the arrays
 // data + p*N, data_b + p*N, coef + p*2N and margin slot p.
@@ -79,7 +88,8 @@ __device__ __forceinline__ void bind_product(PassArgs &a) {
   if (a.data_b) a.data_b += p * a.N;
   if (a.coef) a.coef += p * 2 * a.N;
   if (a.ybuf) a.ybuf += p * a.ystride;
-  if (a.margin) a.margin += p;  // margin_mask 0: one slot (both operands' packing rows clear the same one)
+  // both operands' packing rows clear the same slots
+  if (a.margin) a.margin += p * (unsigned long long)(a.margin_mask + 1) * MARGIN_STRIDE;
 }
 
 // Tile order that keeps adjacent column tiles on one XCD at the same time:
@@ -250,13 +260,6 @@ __device__ __forceinline__ void write_group_half(const PassArgs &a, long long *l
   }
 }
 
-// Margin slots: a single product spreads its atomics over MARGIN_SLOTS
-// addresses MARGIN_STRIDE words apart (one 128-byte line each), so tens of
-// thousands of workgroups do not serialise on one address; the carry takes the
-// maximum over the slots (margin_of_slots) to host memory.
-constexpr int MARGIN_SLOTS = 64;
-constexpr int MARGIN_STRIDE = 32;
-
 // Wave-level max then one atomic per wave, into slot (blockIdx.x & mask).
 __device__ __forceinline__ void margin_reduce(unsigned int *m, double d, int mask = 0) {
   float f = (float)d;
@@ -271,9 +274,9 @@ __device__ __forceinline__ void margin_clear(const PassArgs &a) {
   for (int i = threadIdx.x; i <= a.margin_mask; i += blockDim.x) a.margin[i * MARGIN_STRIDE] = 0u;
 }
 
-// First wave: the largest slot, on every lane.
-__device__ __forceinline__ unsigned margin_of_slots(const unsigned int *m) {
-  unsigned v = m[(threadIdx.x & 63) * MARGIN_STRIDE];  // non-negative floats order like their bit patterns
+// First wave: the largest of the mask + 1 slots, on every lane.
+__device__ __forceinline__ unsigned margin_of_slots(const unsigned int *m, int mask = MARGIN_SLOTS - 1) {
+  unsigned v = m[(threadIdx.x & mask) * MARGIN_STRIDE];  // non-negative floats order like their bit patterns
   for (int off = 32; off > 0; off >>= 1) {
     const unsigned o = __shfl_xor(v, off, 64);
     v = o > v ? o : v;
@@ -291,6 +294,7 @@ struct HostResult {
   unsigned long long top;
   unsigned long long exp;      // k_rcp_small: the result's exponent (top: its length, swapped: its sign)
   unsigned swapped;
+  unsigned set_margin[64];     // k_margin_out: of a deferral scope's products
 };
 __device__ __forceinline__ void host_store(unsigned *p, unsigned v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -813,7 +817,9 @@ struct CarryArgs {
   unsigned wpb;              // words per carry block
   unsigned long long ystride;  // batched group mode: group-sum words per product
   HostResult *host;            // nullptr, or where block 0 leaves the margin and open blocks their flag
-  const unsigned int *margin;  // margin slots of the product (with host)
+  const unsigned int *margin;  // margin slots of the product (with host or margin_out)
+  int margin_mask;             // one less than their number
+  unsigned int *margin_out;    // batched: product p's margin goes to margin_out[p]
 };
 
 __device__ __forceinline__ long long coef_at(const CarryArgs &a, long long j) {
@@ -871,6 +877,8 @@ __device__ __forceinline__ void bind_carry(CarryArgs &a, unsigned long long p) {
   a.CL = d.cl;
   a.add = d.d;
   a.addl = d.dl;
+  if (a.margin) a.margin += p * (unsigned long long)(a.margin_mask + 1) * MARGIN_STRIDE;
+  if (a.margin_out) a.margin_out += p;
   a.blk_fn += p * a.nblk;
   a.nblk = (d.cl + a.wpb - 1) / a.wpb;
 }
@@ -947,6 +955,15 @@ __device__ __forceinline__ BlockCarry block_carry(unsigned long long Pm1, unsign
 __device__ __forceinline__ void carry_publish(const CarryArgs &a, unsigned fn, const BlockCarry &c) {
   a.blk_fn[blockIdx.x] = (unsigned char)(fn | (c.open << 2));
   if (c.open && a.host) host_store(&a.host->open_carry, 1u);
+}
+
+// First wave of a product's block 0: its margin to where the host reads it.
+__device__ __forceinline__ void carry_margin(const CarryArgs &a) {
+  if (!a.host && !a.margin_out) return;
+  const unsigned m = margin_of_slots(a.margin, a.margin_mask);
+  if (threadIdx.x != 0) return;
+  if (a.host) host_store(&a.host->margin, m);
+  else *a.margin_out = m;
 }
 
 // Words of one block from coefficients: P_w (< 2^37) per word, v_w = lo(P_w) +
@@ -1052,10 +1069,7 @@ static __global__ __launch_bounds__(CT) void k_carry_local(CarryArgs a) {
     for (int w = 0; w < CT / 64; w++) tot = carry_compose(tot, wave_fn[w]);
     carry_publish(a, tot, bc);
   }
-  if (a.host && blockIdx.x == 0 && tid < 64) {
-    const unsigned m = margin_of_slots(a.margin);
-    if (tid == 0) host_store(&a.host->margin, m);
-  }
+  if (blockIdx.x == 0 && tid < 64) carry_margin(a);
   unsigned cin = (carry_compose(pre, excl) >> bc.cin) & 1u;
   uint32_t o[CWPT];
 #pragma unroll
@@ -1249,10 +1263,7 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
     for (int q = 0; q < GCT / 64; q++) tot = carry_compose(tot, wave_fn[q]);
     carry_publish(a, tot, bc);
   }
-  if (a.host && blockIdx.x == 0 && tid < 64) {
-    const unsigned m = margin_of_slots(a.margin);
-    if (tid == 0) host_store(&a.host->margin, m);
-  }
+  if (blockIdx.x == 0 && tid < 64) carry_margin(a);
   unsigned cin = (carry_compose(pre, excl) >> bc.cin) & 1u;
   uint32_t o[GWPT];
 #pragma unroll
@@ -1335,10 +1346,11 @@ static __global__ __launch_bounds__(RIPPLE_BLOCKS) void k_carry_ripple(CarryArgs
   }
 }
 
-// The margin of a product to the host ahead of its carry (products in place).
-static __global__ __launch_bounds__(64) void k_margin_out(const unsigned int *m, HostResult *host) {
-  const unsigned v = margin_of_slots(m);
-  if (threadIdx.x == 0) host_store(&host->margin, v);
+// Margins of whole slot sets to the host, one per workgroup: of a product ahead
+// of its carry (products in place), of the products of a deferral scope.
+static __global__ __launch_bounds__(64) void k_margin_out(const unsigned int *m, unsigned *host) {
+  const unsigned v = margin_of_slots(m + (size_t)blockIdx.x * MARGIN_SLOTS * MARGIN_STRIDE);
+  if (threadIdx.x == 0) host_store(host + blockIdx.x, v);
 }
 
 // --------------------------------------------------------------- utilities

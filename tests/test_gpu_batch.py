@@ -169,3 +169,16 @@ def test_plain_calls_around_the_host_descriptor_limit(bc, count, bias):
     assert worst < 0.25 and st["products"] == sum(len(a) + len(b) >= 100 for a, b in pairs)
     assert bias or st["retries"] == 0
     assert not bias or st["retries"] >= 1
+
+
+@pytest.mark.parametrize("n", [5000, 20000, 60000, 300000])
+def test_margins_of_a_batch_are_its_products(bc, n):
+    # multi-pass products of one plan, whose margins are spread over 1 to 64
+    # slots each: the batch's worst is the worst of its products'
+    pairs = [(operand(SplitMix64(n + k), n), operand(SplitMix64(n - k - 1), n - 7)) for k in range(3)]
+    alone = [bc.mul_batch([p])[1] for p in pairs]
+    assert min(alone) > 0
+    for order in ((0, 1, 2), (2, 0, 1)):
+        out, worst = bc.mul_batch([pairs[k] for k in order])
+        assert worst == max(alone)
+    assert np.array_equal(out[1], bc.mul(*pairs[0])[0])

@@ -170,3 +170,20 @@ def test_e_text_equals_the_oracle_for_small_digit_counts(bc, oracle):
     for D in list(range(1, 60)) + [99, 100, 101, 997, 2000]:
         txt, _ = bc.e_digits(D)
         assert txt.encode() == oracle.e_digits(D)[0], D
+
+
+@pytest.mark.parametrize("n", [3000, 40000])
+def test_radix_re_runs_where_a_margin_is_too_large(bc, n):
+    # digits far above the bound: the margins judged at the end fail, and the
+    # conversion runs again with every product checked (and re-run smaller);
+    # 3000 words stay within the bound at the largest digit size, 20 bits
+    F = np.random.default_rng(n).integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32)
+    want = bc.radix(F, n)
+    bc.plan_digit_bias(6)
+    try:
+        bc.stats_reset()
+        got = bc.radix(F, n)
+        assert (bc.stats()["retries"] >= 1) == (n > 3000)
+    finally:
+        bc.plan_digit_bias(0)
+    assert np.array_equal(got, want)
