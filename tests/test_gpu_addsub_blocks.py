@@ -55,3 +55,9 @@ def test_target_is_an_operand(bc, n):
     assert _value(x.triple()) == words_to_int(a) - words_to_int(b)
     bc.bf_op("add", y, x, y, 0)
     assert _value(y.triple()) == words_to_int(a)
+
+
+@pytest.mark.parametrize("n", [8192 * 17 - 1, 8192 * 64 + 1, 8192 * 66 + 5])
+def test_runs_in_long_blocks(bc, n):
+    # above 2^17 words a workgroup takes 8192 of them
+    test_carry_and_borrow_runs(bc, n)
