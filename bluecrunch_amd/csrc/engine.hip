@@ -663,9 +663,13 @@ int class_id(unsigned long long N) {
 //    workgroups' LDS on a CU (so not with 512 rows), else 8: 8 against 16 columns
 //    is 75 us against 79 us at 2^20 points, 107 us against 100 us at 2^21 and
 //    8.6 ms against 9.2 ms in the 512-row pass at 3 * 2^26.
-// The products of a batched class fill the GPU together, so its short lengths
-// keep the longest inner pass and 16 columns (4096 products of 16 to 16384
-// words: 1.10 ms against 1.16 ms with the split of single products).
+// Batched products take the same splits from 2^15 points up (64 products of 2^15: 90 us
+// with 256 x 128 against 99 us with 64 x 512, of 2^17 233 us with 256 x 512 against 252
+// with 64 x 2048), except an inner pass of 384, which gives way to 64 rows (64 of 98304
+// points: 180 us against 194 us). Shorter ones, which come by the hundred, keep 64
+// rows (4096 products of 16 to 16384 words: 670 us against 678 us), and 64 rows take
+// 16 columns, whose tiles are half a wave otherwise (400 of 12288 points: 199 us
+// against 223 us).
 int default_candidate(const std::vector<Plan> &c, bool batched = false) {
   const unsigned long long N = c[0].N;
   auto find = [&](int P, unsigned long long l0, unsigned long long l1, int c0) {
@@ -676,15 +680,13 @@ int default_candidate(const std::vector<Plan> &c, bool batched = false) {
     return -1;
   };
   if (c[0].P == 1) return 0;
-  if (batched && N <= (1ull << 17))
-    for (size_t i = 0; i < c.size(); i++)
-      if (c[i].P == 2 && c[i].C[0] >= 8) return (int)i;
   const unsigned long long max_in = is_three(N) ? 6144 : 8192;
   if (N <= (1ull << 23)) {
     unsigned long long rows = 256;
     while (N / rows > max_in) rows *= 2;
     while (rows > 64 && N / rows < 128) rows /= 2;
-    const int cols = rows <= 256 && N / rows >= 16 * 384 ? 16 : 8;
+    if (batched && (N <= 24576 || N / rows == 384)) rows = 64;
+    const int cols = (rows <= 256 && N / rows >= 16 * 384) || (batched && rows == 64) ? 16 : 8;
     const int i = find(2, rows, 0, cols);
     if (i >= 0) return i;
   } else {
