@@ -29,13 +29,6 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
-struct RootsDev {
-  cd *lo = nullptr;
-  cd *hi = nullptr;
-  int sh = 0;
-  unsigned long long four_n = 0;
-};
-
 struct Pending {
   int kind;
   hipEvent_t a, b;
@@ -51,7 +44,7 @@ struct Engine {
   static constexpr int NAUX = 3;
   hipStream_t aux[NAUX] = {nullptr, nullptr, nullptr};
   hipEvent_t fork_ev = nullptr, join_ev[NAUX] = {nullptr, nullptr, nullptr};
-  std::map<unsigned long long, RootsDev> roots;  // keyed by N
+  std::set<unsigned long long> lengths;          // transform lengths met so far
   std::map<int, cd *> ltab;                      // e^{2 pi i t/L}, keyed by L
   DevBuf bufA, bufB, wA, wB, wC, blk, margin, zbuf;
   DevBuf scan, flags, one;  // state of the scans and sums (zero between launches), the word 1
@@ -298,8 +291,7 @@ int init_locked(int device) {
   HIPCHK(hipHostGetDevicePointer((void **)&g.hres_dev, g.hres, 0));
   // every kernel family's code object now rather than inside a first product
   // (a failure here only defers the load to the first launch)
-  for (auto f : {preload_mul1, preload_fwd_pow2, preload_fwd_three, preload_inv_pow2, preload_inv_three, preload_mid,
-                 preload_keep})
+  for (auto f : {preload_mul1, preload_fwd, preload_inv, preload_mid, preload_row, preload_keep})
     if (f()) (void)hipGetLastError();
   return prepare_noalloc();
 }
@@ -398,76 +390,17 @@ int upload(cd **dst, const std::vector<double> &host) {
   return 0;
 }
 
-// Table-free fields of Roots for 4N = four_n: 4N = 8 q8, q8 = 2^qa or 3 * 2^qa.
-void roots_direct(unsigned long long four_n, Roots *r) {
-  r->four_n = four_n;
-  r->q8 = (four_n % 8 == 0) ? four_n / 8 : 0;
-  r->q3 = (r->q8 && r->q8 % 3 == 0) ? 1 : 0;
-  unsigned long long q = r->q3 ? r->q8 / 3 : r->q8;
-  r->qa = 0;
-  while (q > 1) {
-    q >>= 1;
-    r->qa++;
-  }
+// Roots for transform length N: 4N = 8 q8, q8 = 2^qa or 3 * 2^qa. The
+// allocation-free entry point takes only lengths met before it runs.
+int get_roots(unsigned long long N, Roots *r) {
+  if (g_fixed && !g.lengths.count(N)) return fail(BCG_E_ARG, "transform length not prepared at initialisation");
+  g.lengths.insert(N);
+  r->q8 = N / 2;
+  r->q3 = r->q8 % 3 == 0 ? 1 : 0;
+  const unsigned long long q = r->q3 ? r->q8 / 3 : r->q8;
+  r->qa = 63 - __builtin_clzll(q);
   const long double quarter_pi = 0.785398163397448309615660845819875721L;
-  r->step = r->q8 ? (double)(quarter_pi / (long double)r->q8) : 0.0;
-}
-
-// lo[u] = Omega^u (u < nlo), hi[u] = Omega^{u 2^sh} (u < nhi), from omega_direct.
-__global__ void k_fill_roots(Roots r, cd *lo, unsigned long long nlo, cd *hi, unsigned long long nhi) {
-  const unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nlo)
-    lo[i] = omega_direct(r, i);
-  else if (i < nlo + nhi)
-    hi[i - nlo] = omega_direct(r, (i - nlo) << r.sh);
-}
-
-// Root tables for transform length N, built once on the device (N even, so
-// omega_direct's octant split applies; the tables agree with correctly rounded
-// values within its 1.8e-16).
-int get_roots(unsigned long long N, Roots *out) {
-  auto it = g.roots.find(N);
-  if (it == g.roots.end() && g_fixed) return fail(BCG_E_ARG, "root table not prepared at initialisation");
-  if (it == g.roots.end()) {
-    RootsDev r;
-    r.four_n = 4 * N;
-    int lg = 0;
-    while ((1ull << lg) < r.four_n) lg++;
-    r.sh = (lg + 1) / 2;
-    const unsigned long long nlo = 1ull << r.sh;
-    const unsigned long long nhi = (r.four_n + nlo - 1) >> r.sh;
-    Roots d;
-    memset(&d, 0, sizeof d);
-    roots_direct(r.four_n, &d);
-    d.sh = r.sh;
-    if (N % 2 || !d.q8) {  // (no such length class) host tables, long double
-      std::vector<double> lo(2 * nlo), hi(2 * nhi);
-      for (unsigned long long u = 0; u < nlo; u++) root_ld(u, r.four_n, &lo[2 * u], &lo[2 * u + 1]);
-      for (unsigned long long u = 0; u < nhi; u++) root_ld(u << r.sh, r.four_n, &hi[2 * u], &hi[2 * u + 1]);
-      if (int rc = upload(&r.lo, lo)) return rc;
-      if (int rc = upload(&r.hi, hi)) return rc;
-    } else {
-      void *plo = nullptr, *phi = nullptr;
-      hipError_t e = hipMalloc(&plo, nlo * sizeof(cd));
-      if (e == hipSuccess) e = hipMalloc(&phi, nhi * sizeof(cd));
-      if (e != hipSuccess) {
-        if (plo) (void)hipFree(plo);
-        return fail(BCG_E_NOMEM, "table allocation failed", e);
-      }
-      r.lo = (cd *)plo;
-      r.hi = (cd *)phi;
-      const unsigned long long n = nlo + nhi;
-      hipLaunchKernelGGL(k_fill_roots, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, g.stream, d, r.lo, nlo, r.hi,
-                         nhi);
-      HIPCHK(hipGetLastError());
-      HIPCHK(hipStreamSynchronize(g.stream));  // ready before any stream uses them
-    }
-    it = g.roots.emplace(N, r).first;
-  }
-  out->lo = it->second.lo;
-  out->hi = it->second.hi;
-  out->sh = it->second.sh;
-  roots_direct(it->second.four_n, out);
+  r->step = (double)(quarter_pi / (long double)r->q8);
   return 0;
 }
 
@@ -1703,32 +1636,23 @@ int transform_dev(double *z, size_t length, bool inverse, hipStream_t s) {
   Plan p;
   p.N = length;
   if (!factor_cached(length, p)) return fail(BCG_E_ARG, "no transform plan for this length");
-  for (int i = 0; i < p.P; i++)
-    if (i == p.P - 1) p.C[i] = 1;
-  PassArgs a;
-  memset(&a, 0, sizeof a);
-  if (!inverse) {
-    for (int i = 0; i < p.P; i++) {
-      PassArgs b = a;
-      if (int rc = pass_args(p, i, b)) return rc;
-      b.data = (cd *)z;
-      fwd_fn f = pick_fwd(p.L[i], p.C[i]);
-      if (!f) return fail(BCG_E_ARG, "no forward kernel for this tile");
-      ProfScope ps(BCG_K_FWD, s);
-      if (f(false, b.ntiles, 1, s, b)) return fail(BCG_E_ARG, "kernel rejected this pass");
-      HIPCHK(hipGetLastError());
+  for (int k = 0; k < p.P; k++) {
+    const int i = inverse ? p.P - 1 - k : k;
+    PassArgs a;
+    memset(&a, 0, sizeof a);
+    if (int rc = pass_args(p, i, a)) return rc;
+    a.data = (cd *)z;
+    ProfScope ps(inverse ? BCG_K_INV : BCG_K_FWD, s);
+    if (i == p.P - 1) {
+      row_fn f = pick_row(p.L[i]);
+      if (!f) return fail(BCG_E_ARG, "no kernel for this innermost pass");
+      f(inverse, (int)(p.N / (unsigned long long)p.L[i]), s, a);
+    } else {
+      fwd_fn f = inverse ? pick_inv(p.L[i], p.C[i]) : pick_fwd(p.L[i], p.C[i]);
+      if (!f) return fail(BCG_E_ARG, inverse ? "no inverse kernel for this tile" : "no forward kernel for this tile");
+      if (f(false, a.ntiles, 1, s, a)) return fail(BCG_E_ARG, "kernel rejected this pass");
     }
-  } else {
-    for (int i = p.P - 1; i >= 0; i--) {
-      PassArgs b = a;
-      if (int rc = pass_args(p, i, b)) return rc;
-      b.data = (cd *)z;
-      fwd_fn f = pick_inv(p.L[i], p.C[i]);
-      if (!f) return fail(BCG_E_ARG, "no inverse kernel for this tile");
-      ProfScope ps(BCG_K_INV, s);
-      if (f(false, b.ntiles, 1, s, b)) return fail(BCG_E_ARG, "kernel rejected this pass");
-      HIPCHK(hipGetLastError());
-    }
+    HIPCHK(hipGetLastError());
   }
   return 0;
 }
@@ -1925,7 +1849,7 @@ unsigned char *g_scratch_ptr[NA_MAX_DEVICES] = {nullptr};
 
 // At initialisation, with the device current: the scratch's address, and
 // every table and pass split a product up to NOALLOC_MAX_POINTS points can
-// use (root tables per length class, per-pass tables per pass length), so that
+// use (length classes, per-pass tables per pass length), so that
 // the allocation-free entry point finds them built.
 int prepare_noalloc() {
   if (g.device < 0 || g.device >= NA_MAX_DEVICES) return fail(BCG_E_ARG, "device index beyond the scratch table");
@@ -1995,11 +1919,7 @@ int bcg_shutdown(void) {
     b->p = nullptr;
     b->bytes = 0;
   }
-  for (auto &r : g.roots) {
-    (void)hipFree(r.second.lo);
-    (void)hipFree(r.second.hi);
-  }
-  g.roots.clear();
+  g.lengths.clear();
   for (auto &t : g.ltab) (void)hipFree(t.second);
   g.ltab.clear();
   prof_collect();

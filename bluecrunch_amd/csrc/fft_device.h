@@ -93,16 +93,15 @@ struct Len {
 template <int L, int C>
 struct Tile {
   static constexpr int E = L * C;
-  static constexpr bool THREE = Len<L>::THREE;
-  static constexpr int LOG = Len<L>::LOG;
-  static constexpr int EPT = THREE ? 24 : 16;
+  static constexpr int LOG = ilog2c(L);
+  static constexpr int EPT = 16;
   static constexpr int T = E / EPT;
-  static constexpr int MAXB = THREE ? 3 : 4;
+  static constexpr int MAXB = 4;
   static constexpr int NST2 = (LOG + MAXB - 1) / MAXB;  // radix-2^b stages
   static constexpr int FIRSTB = LOG - MAXB * (NST2 - 1);
   // LDS index with one pad element every 16 to spread power-of-two strides.
   static constexpr int LDS_ELEMS = E + E / 16;
-  static_assert(E % EPT == 0, "tile must split evenly");
+  static_assert(L % 3 != 0 && E % EPT == 0, "strided passes are powers of two, split evenly");
   static_assert(T >= 1 && T <= 1024, "bad thread count");
 };
 
@@ -128,33 +127,16 @@ __device__ __forceinline__ unsigned brev(unsigned v, int bits) {
   return bits ? (__builtin_bitreverse32(v) >> (32 - bits)) : 0u;
 }
 
-// Frequency index held at row r after an in-place DIF of length L
-// (bit-reversed 2-part, radix-3 digit innermost).
-template <int L>
-__device__ __forceinline__ unsigned freq_of_row(unsigned r) {
-  if (Len<L>::THREE) return brev(r / 3u, Len<L>::LOG) + (r % 3u) * (unsigned)Len<L>::P2;
-  return brev(r, Len<L>::LOG);
-}
-
-// Root-of-unity tables for one transform length N: Omega = e^{2 pi i / 4N}.
-//   Omega^u = hi[u >> sh] * lo[u & (2^sh - 1)],  u in [0, 4N)
-//   tl_L[t] = e^{2 pi i t / L} for t < L/2, one table per pass length L.
-//   Without tables (omega_direct): 4N = 8 q8 with q8 = 2^qa or 3 * 2^qa and
-//   step = (pi/4) / q8 rounded to double.
+// Roots of unity of one transform length N: Omega = e^{2 pi i / 4N}, computed in
+// registers (omega_direct) from 4N = 8 q8 with q8 = 2^qa or 3 * 2^qa and
+// step = (pi/4) / q8 rounded to double. The stages of a pass of length L read
+// tl_L[t] = e^{2 pi i t / L}, t < L/2, one table per pass length.
 struct Roots {
-  const cd *lo;
-  const cd *hi;
-  int sh;
-  unsigned long long four_n;
   unsigned long long q8;
   int qa;
   int q3;
   double step;
 };
-
-__device__ __forceinline__ cd omega_pow(const Roots &r, unsigned long long u) {
-  return cmul(r.hi[u >> r.sh], r.lo[u & ((1ull << r.sh) - 1)]);
-}
 
 // Omega^u for 0 <= u < 4N, computed in registers. The octant o = floor(u / q8)
 // is split off exactly in integers; the rest is an angle y in [0, pi/4]
@@ -644,24 +626,6 @@ __device__ __forceinline__ void lds_stage(cd *lds, int span, const cd *__restric
   }
 }
 
-template <int L, int C, bool INV>
-__device__ __forceinline__ void lds_radix3(cd *lds, int tid) {
-  using TC = Tile<L, C>;
-  constexpr int PER = TC::EPT / 3;
-#pragma unroll
-  for (int i = 0; i < PER; i++) {
-    int bf = tid + i * TC::T;
-    int c = bf % C;
-    int blk = bf / C;
-    const int r3 = blk * 3;
-    cd a = lds[slot<C>(r3, c)], b = lds[slot<C>(r3 + 1, c)], d = lds[slot<C>(r3 + 2, c)];
-    dft3<INV>(a, b, d);
-    lds[slot<C>(r3, c)] = a;
-    lds[slot<C>(r3 + 1, c)] = b;
-    lds[slot<C>(r3 + 2, c)] = d;
-  }
-}
-
 // Runtime dispatch on the radix bits of a stage (1..4).
 template <int L, int C, bool INV>
 __device__ __forceinline__ void lds_stage_any(cd *lds, int rb, int span, const cd *__restrict__ tl, int tid) {
@@ -679,8 +643,8 @@ __device__ __forceinline__ int stage_bits(int s) {
   return s == 0 ? Tile<L, C>::FIRSTB : Tile<L, C>::MAXB;
 }
 
-// Forward stages 1..NST2-1 entirely in LDS (stage 0 has been done already),
-// then the radix-3 stage when L = 3*2^k. Ends with a barrier.
+// Forward stages 1..NST2-1 entirely in LDS (stage 0 has been done already).
+// Ends with a barrier.
 template <int L, int C>
 __device__ __forceinline__ void forward_rest(cd *lds, const cd *__restrict__ tl, int tid) {
   using TC = Tile<L, C>;
@@ -691,21 +655,13 @@ __device__ __forceinline__ void forward_rest(cd *lds, const cd *__restrict__ tl,
     __syncthreads();
     span >>= rb;
   }
-  if (TC::THREE) {
-    lds_radix3<L, C, false>(lds, tid);
-    __syncthreads();
-  }
 }
 
 // Inverse stages from the innermost up to (not including) stage 0.
 template <int L, int C>
 __device__ __forceinline__ void inverse_front(cd *lds, const cd *__restrict__ tl, int tid) {
   using TC = Tile<L, C>;
-  if (TC::THREE) {
-    lds_radix3<L, C, true>(lds, tid);
-    __syncthreads();
-  }
-  int span = TC::THREE ? 3 : 1;
+  int span = 1;
   for (int s = TC::NST2 - 1; s >= 1; s--) {
     int rb = stage_bits<L, C>(s);
     span <<= rb;

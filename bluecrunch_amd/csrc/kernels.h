@@ -311,7 +311,7 @@ __device__ __forceinline__ void host_store(unsigned *p, unsigned v) {
 // many waves fit on a CU.
 template <int L, int C>
 struct SplitTile {
-  static constexpr bool ON = !Tile<L, C>::THREE && Tile<L, C>::NST2 == 2 && Tile<L, C>::FIRSTB == 4;
+  static constexpr bool ON = Tile<L, C>::NST2 == 2 && Tile<L, C>::FIRSTB == 4;
   static constexpr int BYTES = Tile<L, C>::LDS_ELEMS * (ON ? 8 : 16);
 };
 
@@ -475,7 +475,6 @@ __global__ __launch_bounds__((Tile<L, C>::T)) void k_fwd(PassArgs a) {
   constexpr int R0 = 1 << RB0;
   constexpr int PER0 = TC::EPT / R0;
   constexpr int SUB0 = L / R0;
-  static_assert(!PACK || !TC::THREE, "packing pass is a power of two");
   // Thread tid owns column c = tid % C and rows r0 + h * L/16, r0 = tid / C,
   // h = 0..15 (T = L*C/16): row r0 + h*L/16 has frequency 16 brev(r0) + brev4(h).
   const int c = tid % C;
@@ -552,28 +551,15 @@ __global__ __launch_bounds__((Tile<L, C>::T)) void k_fwd(PassArgs a) {
   }
   __syncthreads();
   forward_rest<L, C>(lds, a.tl, tid);
-  if constexpr (TC::THREE) {
-    for (int e = tid; e < TC::E; e += TC::T) {
-      int row = e / C, cc = e % C;
-      unsigned long long mm = m0 + cc;
-      cd v = lds[pad16(e)];
-      if (a.M > 1) {
-        unsigned long long k = freq_of_row<L>((unsigned)row);
-        v = cmul(v, omega_pow(a.roots, mm * k * a.tw_mul));
-      }
-      base[(unsigned long long)row * a.M + mm] = v;
-    }
-  } else {
-    // pass twiddle e^{2 pi i m k / S} = Omega^{tw_mul m k}
-    Walk16 w;
-    if (a.M > 1) w.template init_shared<C>(a.roots, a.tw_mul * m * 16ull * brev((unsigned)r0, TC::LOG - 4), a.tw_mul * m);
+  // pass twiddle e^{2 pi i m k / S} = Omega^{tw_mul m k}
+  Walk16 w;
+  if (a.M > 1) w.template init_shared<C>(a.roots, a.tw_mul * m * 16ull * brev((unsigned)r0, TC::LOG - 4), a.tw_mul * m);
 #pragma unroll
-    for (int h = 0; h < 16; h++) {
-      const int row = r0 + h * (L / 16);
-      cd v = lds[slot<C>(row, c)];
-      if (a.M > 1) v = cmul(v, w.at(h));
-      st_pol<(CACHE & 2) != 0>(&base[(unsigned long long)row * a.M + m], v);
-    }
+  for (int h = 0; h < 16; h++) {
+    const int row = r0 + h * (L / 16);
+    cd v = lds[slot<C>(row, c)];
+    if (a.M > 1) v = cmul(v, w.at(h));
+    st_pol<(CACHE & 2) != 0>(&base[(unsigned long long)row * a.M + m], v);
   }
 }
 
@@ -602,7 +588,6 @@ __attribute__((amdgpu_waves_per_eu((MODE == 1 && SplitTile<L, C>::ON && C >= 8) 
   const unsigned long long ob = (unsigned)tile / (unsigned)tpb;  // tpb < 2^31
   const unsigned long long m0 = ((unsigned)tile % (unsigned)tpb) * (unsigned long long)C;
   cd *base = a.data + ob * a.S;
-  static_assert(!UNPACK || !TC::THREE, "unpacking pass is a power of two");
   const int c = tid % C;
   const int r0 = tid / C;
   const unsigned long long m = m0 + c;
@@ -655,29 +640,16 @@ __attribute__((amdgpu_waves_per_eu((MODE == 1 && SplitTile<L, C>::ON && C >= 8) 
     }
     return;
   }
-  if constexpr (TC::THREE) {
-    for (int e = tid; e < TC::E; e += TC::T) {
-      int row = e / C, cc = e % C;
-      unsigned long long mm = m0 + cc;
-      cd v = base[(unsigned long long)row * a.M + mm];
-      if (a.M > 1) {
-        unsigned long long k = freq_of_row<L>((unsigned)row);
-        v = cmulc(v, omega_pow(a.roots, mm * k * a.tw_mul));
-      }
-      lds[pad16(e)] = v;
-    }
-  } else {
-    // all sixteen loads in flight first, then the conjugate pass twiddle
-    // (rows r0 + h * L/16 as in k_fwd) on the way into LDS
-    cd xs[16];
-    load_rows16<1, L / 16, (CACHE & 1) != 0>(base, xs, r0, c, m0, a.M);
-    Walk16 w;
-    if (a.M > 1) w.template init_shared<C>(a.roots, a.tw_mul * m * 16ull * brev((unsigned)r0, TC::LOG - 4), a.tw_mul * m);
+  // all sixteen loads in flight first, then the conjugate pass twiddle
+  // (rows r0 + h * L/16 as in k_fwd) on the way into LDS
+  cd xs[16];
+  load_rows16<1, L / 16, (CACHE & 1) != 0>(base, xs, r0, c, m0, a.M);
+  Walk16 w;
+  if (a.M > 1) w.template init_shared<C>(a.roots, a.tw_mul * m * 16ull * brev((unsigned)r0, TC::LOG - 4), a.tw_mul * m);
 #pragma unroll
-    for (int h = 0; h < 16; h++) {
-      const int row = r0 + h * (L / 16);
-      lds[slot<C>(row, c)] = (a.M > 1) ? cmulc(xs[h], w.at(h)) : xs[h];
-    }
+  for (int h = 0; h < 16; h++) {
+    const int row = r0 + h * (L / 16);
+    lds[slot<C>(row, c)] = (a.M > 1) ? cmulc(xs[h], w.at(h)) : xs[h];
   }
   __syncthreads();
   inverse_front<L, C>(lds, a.tl, tid);
@@ -775,6 +747,50 @@ __global__ __launch_bounds__((Row<L, mid_points(L)>::T * BPW)) void k_mid(PassAr
   row_inverse<L, E>(xa, x, lds, a.tl, tid);
 #pragma unroll
   for (int h = 0; h < E; h++) st_pol<(CACHE & 2) != 0>(&a.data[j0 + h * RC::T], x[h]);
+}
+
+// Innermost pass of a transform that stands alone: one contiguous block of L points
+// in place, forward or inverse, BPW blocks per workgroup as in k_mid. The
+// innermost stage holds neighbouring points per thread, so global memory is reached
+// through one more turn in LDS, at points tid + h T. Bound by the chain of one
+// workgroup where each CU has one: 256 blocks of 4096 points 13 us (14 us with sixteen
+// points a thread; 6.5 us at the rate of a copy).
+template <int L, bool INV, int BPW = 1>
+__global__ __launch_bounds__((Row<L, 8>::T * BPW)) void k_row(PassArgs a) {
+  constexpr int E = 8;
+  using RC = Row<L, E>;
+  __shared__ cd lds_all[RC::LDS_ELEMS * BPW];
+  const int sub = BPW > 1 ? (int)threadIdx.x / RC::T : 0;
+  const int tid = BPW > 1 ? (int)threadIdx.x % RC::T : (int)threadIdx.x;
+  cd *lds = lds_all + sub * RC::LDS_ELEMS;
+  cd *base = a.data + ((unsigned long long)blockIdx.x * BPW + sub) * L + tid;
+  cd x[E], xr[RC::XR];
+#pragma unroll
+  for (int h = 0; h < E; h++) x[h] = ld_nt(&base[h * RC::T]);
+  // xr[i] in row_forward's layout
+  auto at = [&](int i) {
+    if constexpr (RC::THREE) return RC::pad(3 * (tid + i / 3 * RC::T) + i % 3);
+    else return RC::template slot<1>(E * tid, i);
+  };
+  auto there = [&](int i) { return !RC::THREE || i < 6 || tid + 2 * RC::T < L / 3; };
+  if constexpr (INV) {
+#pragma unroll
+    for (int h = 0; h < E; h++) lds[RC::template slot<RC::T>(tid, h)] = x[h];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RC::XR; i++) xr[i] = there(i) ? lds[at(i)] : make_double2(0.0, 0.0);
+    row_inverse<L, E>(xr, x, lds, a.tl, tid);
+  } else {
+    row_forward<L, E>(x, xr, lds, a.tl, tid);
+#pragma unroll
+    for (int i = 0; i < RC::XR; i++)
+      if (there(i)) lds[at(i)] = xr[i];
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < E; h++) x[h] = lds[RC::template slot<RC::T>(tid, h)];
+  }
+#pragma unroll
+  for (int h = 0; h < E; h++) base[h * RC::T] = x[h];
 }
 
 // ------------------------------------------------------------ carry resolve

@@ -11,14 +11,15 @@ namespace bcg {
 typedef int (*fwd_fn)(bool, int, int, hipStream_t, const PassArgs &);
 // mid: (square, grid.x, grid.y, stream, args)
 typedef int (*mid_fn)(bool, int, int, hipStream_t, const PassArgs &);
+// row: (inverse, grid, stream, args)
+typedef int (*row_fn)(bool, int, hipStream_t, const PassArgs &);
 typedef int (*mul1_fn)(int, hipStream_t, const ClassArgs &);
 
 // nullptr when no kernel exists for the (L, C) tile.
-fwd_fn pick_fwd_pow2(int L, int C);
-fwd_fn pick_fwd_three(int L, int C);
-fwd_fn pick_inv_pow2(int L, int C);
-fwd_fn pick_inv_three(int L, int C);
+fwd_fn pick_fwd(int L, int C);
+fwd_fn pick_inv(int L, int C);
 mid_fn pick_mid(int L);
+row_fn pick_row(int L);
 mul1_fn pick_mul1(int L);
 // Cache-keeping variants for the chunked middle passes of three-pass
 // products (forward pass with ordinary stores, middle pass with ordinary
@@ -30,14 +31,10 @@ mid_fn pick_mid_keep(int L);
 
 // Code-object preloads, one per launch_*.hip unit (called at initialisation).
 int preload_mul1();
-int preload_fwd_pow2();
-int preload_fwd_three();
-int preload_inv_pow2();
-int preload_inv_three();
+int preload_fwd();
+int preload_inv();
 int preload_mid();
+int preload_row();
 int preload_keep();
-
-inline fwd_fn pick_fwd(int L, int C) { return (L % 3 == 0) ? pick_fwd_three(L, C) : pick_fwd_pow2(L, C); }
-inline fwd_fn pick_inv(int L, int C) { return (L % 3 == 0) ? pick_inv_three(L, C) : pick_inv_pow2(L, C); }
 
 }  // namespace bcg

@@ -1,8 +1,8 @@
-// Forward pass kernels, power-of-two tiles.
+// Forward pass kernels.
 #include "launch_impl.h"
 
 namespace bcg {
-fwd_fn pick_fwd_pow2(int L, int C) {
+fwd_fn pick_fwd(int L, int C) {
   switch (L) {
     case 64: return ByC<64, FwdL>::pick(C);
     case 128: return ByC<128, FwdL>::pick(C);
@@ -17,7 +17,7 @@ fwd_fn pick_fwd_pow2(int L, int C) {
 }
 // Loads this unit's code object now; the runtime otherwise loads it at the
 // first launch of one of its kernels, inside a caller's first product.
-int preload_fwd_pow2() {
+int preload_fwd() {
   hipFuncAttributes fa;
   return hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&(k_fwd<256, 16, false>))) == hipSuccess ? 0 : -1;
 }

@@ -15,42 +15,30 @@ constexpr int mid_blocks(int L) {
   return L % 3 == 0 ? (L < 1536 ? 1536 / L : 1) : (L < wave ? wave / L : 1);
 }
 
-// Packing/unpacking passes are always the outermost pass, a power of two
-// (the 3 * 2^k factor sits in the innermost pass): the flag is rejected on
-// 3 * 2^k tiles.
+// Strided passes are powers of two (the 3 * 2^k factor sits in the innermost pass).
 template <int L, int C>
 int launch_fwd(bool pack, int grid, int gy, hipStream_t s, const PassArgs &a) {
-  if constexpr (Len<L>::THREE) {
-    if (pack) return -2;
+  if (pack && a.lower)
+    BCG_LAUNCH2((k_fwd<L, C, true, 0, true>), grid, gy, (Tile<L, C>::T), s, a);
+  else if (pack)
+    BCG_LAUNCH2((k_fwd<L, C, true>), grid, gy, (Tile<L, C>::T), s, a);
+  else
     BCG_LAUNCH2((k_fwd<L, C, false>), grid, gy, (Tile<L, C>::T), s, a);
-  } else {
-    if (pack && a.lower)
-      BCG_LAUNCH2((k_fwd<L, C, true, 0, true>), grid, gy, (Tile<L, C>::T), s, a);
-    else if (pack)
-      BCG_LAUNCH2((k_fwd<L, C, true>), grid, gy, (Tile<L, C>::T), s, a);
-    else
-      BCG_LAUNCH2((k_fwd<L, C, false>), grid, gy, (Tile<L, C>::T), s, a);
-  }
   return 0;
 }
 
 // Unpacking into group sums (a.ybuf) exists for 8- and 16-column tiles.
 template <int L, int C>
 int launch_inv(bool unpack, int grid, int gy, hipStream_t s, const PassArgs &a) {
-  if constexpr (Len<L>::THREE) {
-    if (unpack) return -2;
-    BCG_LAUNCH2((k_inv<L, C, 0>), grid, gy, (Tile<L, C>::T), s, a);
+  if (unpack && a.ybuf) {
+    if constexpr (C == 8 || C == 16)
+      BCG_LAUNCH2((k_inv<L, C, 2>), grid, gy, (Tile<L, C>::T), s, a);
+    else
+      return -2;
+  } else if (unpack) {
+    BCG_LAUNCH2((k_inv<L, C, 1>), grid, gy, (Tile<L, C>::T), s, a);
   } else {
-    if (unpack && a.ybuf) {
-      if constexpr (C == 8 || C == 16)
-        BCG_LAUNCH2((k_inv<L, C, 2>), grid, gy, (Tile<L, C>::T), s, a);
-      else
-        return -2;
-    } else if (unpack) {
-      BCG_LAUNCH2((k_inv<L, C, 1>), grid, gy, (Tile<L, C>::T), s, a);
-    } else {
-      BCG_LAUNCH2((k_inv<L, C, 0>), grid, gy, (Tile<L, C>::T), s, a);
-    }
+    BCG_LAUNCH2((k_inv<L, C, 0>), grid, gy, (Tile<L, C>::T), s, a);
   }
   return 0;
 }

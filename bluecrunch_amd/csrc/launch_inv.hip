@@ -1,8 +1,8 @@
-// Inverse pass kernels, power-of-two tiles.
+// Inverse pass kernels.
 #include "launch_impl.h"
 
 namespace bcg {
-fwd_fn pick_inv_pow2(int L, int C) {
+fwd_fn pick_inv(int L, int C) {
   switch (L) {
     case 64: return ByC<64, InvL>::pick(C);
     case 128: return ByC<128, InvL>::pick(C);
@@ -17,7 +17,7 @@ fwd_fn pick_inv_pow2(int L, int C) {
 }
 // Loads this unit's code object now; the runtime otherwise loads it at the
 // first launch of one of its kernels, inside a caller's first product.
-int preload_inv_pow2() {
+int preload_inv() {
   hipFuncAttributes fa;
   return hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&(k_inv<256, 16, 0>))) == hipSuccess ? 0 : -1;
 }

@@ -5,7 +5,7 @@ pass length in a two-pass split, each product exact."""
 import numpy as np
 import pytest
 
-from helpers import exact_product
+from helpers import exact_product, reference_order
 from bluecrunch_amd.workload import operands
 
 pytestmark = pytest.mark.gpu
@@ -86,3 +86,24 @@ def test_margins_are_each_products_own(bc):
     assert bc.mul_batch([(a, b), (a[:700], b[:600])])[1] == batch
     small = bc.mul(a[:700], b[:600])[1]["margin"]
     assert batch == max(own, small) and small < own
+
+
+@pytest.mark.parametrize("inner", LENGTHS)
+def test_innermost_pass_of_transforms(bc, inner):
+    # alone (one block), and under 128 rows (several blocks per workgroup)
+    for n in (inner, 128 * inner):
+        rng = np.random.default_rng(n)
+        x = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+        want = (np.fft.ifft(x) * n)[reference_order(n)]
+        picks = [i for i, (P, L, C) in enumerate(bc.plan_candidates(n)) if n == inner or L == [128, inner]][:1]
+        try:
+            for i in picks:
+                bc.plan_force(n, i)
+                z = x.copy()
+                bc.fft_forward(z)
+                assert np.abs(z - want).max() <= 1e-13 * np.abs(want).max() * np.log2(n)
+                back = want.copy()
+                bc.fft_inverse(back)
+                assert np.abs(back / n - x).max() <= 1e-13 * np.abs(x).max() * np.log2(n)
+        finally:
+            bc.plan_force(n, -1)
