@@ -50,6 +50,7 @@ struct Engine {
   DevBuf scan, flags, one;  // state of the scans and sums (zero between launches), the word 1
   HostResult *hres = nullptr;      // pinned: what the kernels of a product leave for the host
   HostResult *hres_dev = nullptr;  // its device address
+  unsigned seq = 0;                // launches that announce their results (host_wait)
   bool prof = false;
   std::vector<Pending> pending;
   std::vector<hipEvent_t> free_events;
@@ -386,6 +387,23 @@ int init_locked(int device) {
   } while (0)
 
 hipStream_t pick(void *s) { return s ? (hipStream_t)s : g.stream; }
+
+// Waits for what the last announcing launch left in *g.hres. soft: for the
+// announcement alone, which the host sees 5.5 us after a launch instead of 11 us: for
+// steps inside a call, which only queue more work on the same stream. A call returns on
+// a full wait: other streams may read its results. Past a millisecond, or should
+// the announcement not come, the full wait decides.
+int host_wait(hipStream_t s, bool soft) {
+  if (soft) {
+    const auto t0 = std::chrono::steady_clock::now();
+    do {
+      for (int k = 0; k < 64; k++)
+        if (__atomic_load_n(&g.hres->seq, __ATOMIC_ACQUIRE) == g.seq) return 0;
+    } while (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(1));
+  }
+  HIPCHK(hipStreamSynchronize(s));
+  return 0;
+}
 
 // ----------------------------------------------------------------- timing
 
@@ -834,8 +852,9 @@ void launch_ripple(const CarryArgs &c, int count, hipStream_t s) {
 // ends & END_TOP: after the carry, the search for the output's highest nonzero word as well
 // (hres->top once the host has waited). ends & END_RUNS: the caller expects whole blocks
 // of ones (a product close to a power of 2^32), so the ripple goes ahead of the wait (4 us in
-// place of a second wait and search, some 30 us).
-constexpr int END_TOP = 1, END_RUNS = 2;
+// place of a second wait and search, some 30 us). ends & END_SOFT (with END_TOP): a step
+// inside a call, see host_wait.
+constexpr int END_TOP = 1, END_RUNS = 2, END_SOFT = 4;
 void launch_top(const uint32_t *x, size_t n, hipStream_t s);
 int end_carry(const CarryArgs &c, hipStream_t s, double *margin, int ends = 0) {
   if (!c.host) {
@@ -845,13 +864,14 @@ int end_carry(const CarryArgs &c, hipStream_t s, double *margin, int ends = 0) {
     return 0;
   }
   const bool top = (ends & END_TOP) != 0, runs = (ends & END_RUNS) != 0;
+  const bool soft = top && (ends & END_SOFT) != 0;
   if (runs) {
     ProfScope ps(BCG_K_CARRY, s);
     launch_ripple(c, 1, s);
   }
   if (top) launch_top(c.out, (size_t)c.CL, s);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(s));
+  if (int rc = host_wait(s, soft)) return rc;
   float f;
   memcpy(&f, &g.hres->margin, sizeof f);
   *margin = (double)f;
@@ -862,7 +882,7 @@ int end_carry(const CarryArgs &c, hipStream_t s, double *margin, int ends = 0) {
     }
     if (top) launch_top(c.out, (size_t)c.CL, s);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(s));
+    if (int rc = host_wait(s, soft)) return rc;
   }
   return 0;
 }
@@ -1304,7 +1324,7 @@ int run_class(int L, ClassArgs &ca, int count, hipStream_t s) {
 // memory (a descriptor copy, two fill kernels and a margin copy around it were
 // 20 of 51 us at 2048 points).
 int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL,
-                hipStream_t s, double *margin, const uint32_t *D, size_t DL, bool top) {
+                hipStream_t s, double *margin, const uint32_t *D, size_t DL, int ends) {
   const bool deferred = g_defer.in_product;
   ClassArgs ca;
   memset(&ca, 0, sizeof ca);
@@ -1324,9 +1344,10 @@ int mul_onepass(const Plan &p, uint32_t *C, size_t CL, const uint32_t *A, size_t
   if (int rc = run_class(p.L[0], ca, 1, s)) return rc;
   *margin = 0.0;
   if (deferred) return 0;  // read with the scope's other sets later
+  const bool top = (ends & END_TOP) != 0;
   if (top) launch_top(C, CL, s);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(s));
+  if (int rc = host_wait(s, top && (ends & END_SOFT) != 0)) return rc;
   float f;
   memcpy(&f, &g.hres->margin, sizeof f);
   *margin = (double)f;
@@ -1531,7 +1552,7 @@ int d_top_len(const uint32_t *x, size_t n, size_t *len, hipStream_t s);
 int rest_of_top(const uint32_t *x, size_t n, size_t *len, hipStream_t s);
 
 // top (operands and output all nonempty): the output's length without its zero
-// top words, read in the same wait as the margin. ends: END_RUNS or 0 (see end_carry).
+// top words, read in the same wait as the margin. ends: END_RUNS, END_SOFT (see end_carry).
 int mul_dev_locked(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uint32_t *B, size_t BL,
                    int force_bits, hipStream_t s, bcg_mul_info *info, const uint32_t *D = nullptr, size_t DL = 0,
                    size_t *top = nullptr, int ends = 0) {
@@ -1597,7 +1618,7 @@ int mul_dev_body(uint32_t *C, size_t CL, const uint32_t *A, size_t AL, const uin
         if (int rc = ensure(g.zbuf, CL * sizeof(uint32_t) + 64)) return rc;
         dst = (uint32_t *)g.zbuf.p;
       }
-      if (int rc = mul_onepass(p, dst, CL, A, AL, B, BL, s, &m, D, DL, top != nullptr)) return rc;
+      if (int rc = mul_onepass(p, dst, CL, A, AL, B, BL, s, &m, D, DL, ends | (top ? END_TOP : 0))) return rc;
       inf.bits = p.bits;
       inf.passes = 1;
       inf.points = (size_t)p.N;

@@ -295,9 +295,17 @@ struct HostResult {
   unsigned long long exp;      // k_rcp_small: the result's exponent (top: its length, swapped: its sign)
   unsigned swapped;
   unsigned set_margin[64];     // k_margin_out: of a deferral scope's products
+  unsigned seq;                // number of the last launch whose results are in (host_done)
 };
 __device__ __forceinline__ void host_store(unsigned *p, unsigned v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Everything this thread left for the host, and what earlier launches on the
+// stream left, is in host memory (host_wait).
+__device__ __forceinline__ void host_done(HostResult *h, unsigned seq) {
+  __threadfence_system();
+  host_store(&h->seq, seq);
 }
 
 // ------------------------------------------------------------ forward pass
