@@ -212,12 +212,11 @@ __device__ __forceinline__ int group_pos0(const PassArgs &a, unsigned long long 
 // little-endian words (ygK a multiple of 4, zero padded) at ybuf[(j0 / C)
 // ygK ...]: the words from word floor(j0 b / 32) up. One thread per row; the
 // words are assembled in the row's own LDS slots and leave as 16-byte stores.
-template <int L, int C>
+template <int L, int C, int T = Tile<L, C>::T>
 __device__ __forceinline__ void write_group_sums(const PassArgs &a, cd *lds, unsigned long long m0, int tid) {
-  using TC = Tile<L, C>;
   const int b = a.bits;
   const int K = a.ygK;
-  for (int t = tid; t < L; t += TC::T) {
+  for (int t = tid; t < L; t += T) {
     const int s0 = slot<C>(t, 0);  // the row's C slots are contiguous
     unsigned long long re[C], im[C];
 #pragma unroll
@@ -367,12 +366,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t word_rsrc(const uint32_t *p, u
 struct PackDigits {
   __amdgpu_buffer_rsrc_t w0, w1, u0, u1;
   unsigned off;   // byte offset of the lane's word in row r0
-  unsigned step;  // bytes between rows r0 + h L/16 and r0 + (h + 1) L/16
+  unsigned step;  // bytes between rows r0 + h L/E and r0 + (h + 1) L/E
   unsigned sh, bits;
   bool upper;     // the upper half (digits N ..) holds words
   bool one;       // b divides 32: a digit never straddles two words
 
-  template <int L>
+  template <int L, int E = 16>
   __device__ __forceinline__ void init(const PassArgs &a, int r0, unsigned long long m) {
     bits = (unsigned)a.bits;
     const unsigned long long row_w = (a.M * bits) >> 5, half_w = (a.N * bits) >> 5, mb = m * bits;
@@ -385,53 +384,55 @@ struct PackDigits {
     u0 = word_rsrc(upper ? a.wa + half_w : a.wa, upper ? al - half_w : 0);
     u1 = word_rsrc(upper ? a.wa + half_w + 1 : a.wa, upper ? al - half_w - 1 : 0);
     off = (unsigned)(((unsigned long long)r0 * row_w + (mb >> 5)) * 4ull);
-    step = (unsigned)(row_w * (unsigned long long)(L / 16) * 4ull);
+    step = (unsigned)(row_w * (unsigned long long)(L / E) * 4ull);
     sh = (unsigned)(mb & 31ull);
     one = (bits & (bits - 1u)) == 0u;  // b <= 32 divides 32
   }
 
   // Lower-half digits only (launches whose operands all leave the upper half
   // empty).
-  __device__ __forceinline__ void load_lower(unsigned (&d)[16]) const {
-    unsigned lo[16];
+  template <int E>
+  __device__ __forceinline__ void load_lower(unsigned (&d)[E]) const {
+    unsigned lo[E];
 #pragma unroll
-    for (int h = 0; h < 16; h++) lo[h] = __builtin_amdgcn_raw_buffer_load_b32(w0, off + (unsigned)h * step, 0, 0);
+    for (int h = 0; h < E; h++) lo[h] = __builtin_amdgcn_raw_buffer_load_b32(w0, off + (unsigned)h * step, 0, 0);
     if (one) {
 #pragma unroll
-      for (int h = 0; h < 16; h++) d[h] = __builtin_amdgcn_ubfe(lo[h], sh, bits);
+      for (int h = 0; h < E; h++) d[h] = __builtin_amdgcn_ubfe(lo[h], sh, bits);
     } else {
-      unsigned hi[16];
+      unsigned hi[E];
 #pragma unroll
-      for (int h = 0; h < 16; h++) hi[h] = __builtin_amdgcn_raw_buffer_load_b32(w1, off + (unsigned)h * step, 0, 0);
+      for (int h = 0; h < E; h++) hi[h] = __builtin_amdgcn_raw_buffer_load_b32(w1, off + (unsigned)h * step, 0, 0);
 #pragma unroll
-      for (int h = 0; h < 16; h++) d[h] = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(hi[h], lo[h], sh), 0, bits);
+      for (int h = 0; h < E; h++) d[h] = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(hi[h], lo[h], sh), 0, bits);
     }
   }
 
   // Lower-half digits into d, upper-half digits into e (0 when empty); every
   // load is issued before the first is used.
-  __device__ __forceinline__ void load(unsigned (&d)[16], unsigned (&e)[16]) const {
-    unsigned lo[16], ulo[16];
+  template <int E>
+  __device__ __forceinline__ void load(unsigned (&d)[E], unsigned (&e)[E]) const {
+    unsigned lo[E], ulo[E];
 #pragma unroll
-    for (int h = 0; h < 16; h++) {
+    for (int h = 0; h < E; h++) {
       lo[h] = __builtin_amdgcn_raw_buffer_load_b32(w0, off + (unsigned)h * step, 0, 0);
       ulo[h] = __builtin_amdgcn_raw_buffer_load_b32(u0, off + (unsigned)h * step, 0, 0);
     }
     if (one) {
 #pragma unroll
-      for (int h = 0; h < 16; h++) {
+      for (int h = 0; h < E; h++) {
         d[h] = __builtin_amdgcn_ubfe(lo[h], sh, bits);
         e[h] = __builtin_amdgcn_ubfe(ulo[h], sh, bits);
       }
     } else {
-      unsigned hi[16], uhi[16];
+      unsigned hi[E], uhi[E];
 #pragma unroll
-      for (int h = 0; h < 16; h++) {
+      for (int h = 0; h < E; h++) {
         hi[h] = __builtin_amdgcn_raw_buffer_load_b32(w1, off + (unsigned)h * step, 0, 0);
         uhi[h] = __builtin_amdgcn_raw_buffer_load_b32(u1, off + (unsigned)h * step, 0, 0);
       }
 #pragma unroll
-      for (int h = 0; h < 16; h++) {
+      for (int h = 0; h < E; h++) {
         d[h] = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(hi[h], lo[h], sh), 0, bits);
         e[h] = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(uhi[h], ulo[h], sh), 0, bits);
       }
@@ -703,6 +704,132 @@ __attribute__((amdgpu_waves_per_eu((MODE == 1 && SplitTile<L, C>::ON && C >= 8) 
     }
     margin_reduce(a.margin, worst, a.margin_mask);
   }
+}
+
+// ------------------------------------- packing and unpacking, few tiles
+//
+// The packing pass of k_fwd and the unpacking pass of k_inv with eight columns and
+// eight points per thread on the row stages, a column's L points in LDS of its
+// own: the same tiles in twice the waves. For launches that leave SIMDs idle, which
+// are bound by a workgroup's chain of loads and instructions (see launch_impl.h);
+// where the waves are enough, sixteen points per thread spend fewer instructions on
+// twiddles.
+template <int L>
+struct Strip {
+  using RC = Row<L, 8>;
+  static constexpr int C = 8;
+  // neighbouring columns' points half the banks apart, neighbouring rows one after
+  // the other: eight rows of eight columns, a wave, meet each bank equally often
+  static constexpr int COL = RC::LDS_ELEMS + (24 - RC::LDS_ELEMS % 16) % 16;
+  static_assert(COL * C >= L * C + L * C / 16, "the coefficients of the tile fit");
+};
+
+// Walk16 for the eight rows 8 r0 + t: Omega^{u0 + brev3(t) du}.
+struct Walk8 {
+  cd base, g1, g2, g4, p2, p1;
+  template <int C>
+  __device__ __forceinline__ void init_shared(const Roots &r, unsigned long long u0, unsigned long long du) {
+    static_assert(4 * C <= 64, "four lanes of a wave share a column");
+    const int lane = threadIdx.x & 63;
+    const int src0 = (lane % C) + (lane / (4 * C)) * (4 * C);
+    base = omega_direct(r, u0);
+    const cd mine = omega_direct(r, du << ((lane / C) & 3));
+    g1 = make_double2(__shfl(mine.x, src0, 64), __shfl(mine.y, src0, 64));
+    g2 = make_double2(__shfl(mine.x, src0 + C, 64), __shfl(mine.y, src0 + C, 64));
+    g4 = make_double2(__shfl(mine.x, src0 + 2 * C, 64), __shfl(mine.y, src0 + 2 * C, 64));
+  }
+  // i = 0..7 in increasing order
+  __device__ __forceinline__ cd at(int i) {
+    if ((i & 3) == 0) p2 = (i & 4) ? cmul(base, g1) : base;
+    if ((i & 1) == 0) p1 = (i & 2) ? cmul(p2, g2) : p2;
+    return (i & 1) ? cmul(p1, g4) : p1;
+  }
+};
+
+template <int L, bool LOWER>
+__global__ __launch_bounds__(L) void k_fwd8(PassArgs a) {
+  using SC = Strip<L>;
+  constexpr int C = SC::C, E = 8, LOG = SC::RC::LOG;
+  bind_product(a);
+  __shared__ cd lds[SC::COL * C];
+  const int tid = threadIdx.x;
+  const int tile = tile_of_block(a.ntiles);
+  const unsigned long long tpb = a.M / C;
+  const unsigned long long ob = (unsigned)tile / (unsigned)tpb;  // tpb < 2^31
+  const int c = tid % C, r0 = tid / C;
+  const unsigned long long m = ((unsigned)tile % (unsigned)tpb) * (unsigned long long)C + c;
+  cd *base = a.data + ob * a.S + m;
+  cd x[E], y[E];
+  if (a.margin) margin_clear(a);
+  unsigned dre[E], dim_[E];
+  PackDigits pd;
+  pd.template init<L, E>(a, r0, m);
+  if constexpr (LOWER)
+    pd.load_lower(dre);
+  else
+    pd.load(dre, dim_);
+  // right-angle weight of row r0 + h L/8: Omega^{r0 M + m} e^{2 pi i h / 32}
+  const cd wpack = omega_direct(a.roots, (unsigned long long)r0 * a.M + m);
+#pragma unroll
+  for (int h = 0; h < E; h++) {
+    const cd w = cmul(wpack, w64(2 * h));
+    if constexpr (LOWER)
+      x[h] = make_double2((double)dre[h] * w.x, (double)dre[h] * w.y);
+    else
+      x[h] = cmul(make_double2((double)dre[h], (double)dim_[h]), w);
+  }
+  row_forward<L, E>(x, y, lds + c * SC::COL, a.tl, r0);
+  // row 8 r0 + t has frequency (L / 8) brev3(t) + brev(r0)
+  Walk8 w;
+  w.template init_shared<C>(a.roots, a.tw_mul * m * brev((unsigned)r0, LOG - 3), a.tw_mul * m * (L / E));
+#pragma unroll
+  for (int t = 0; t < E; t++) st_pol<false>(&base[(unsigned long long)(E * r0 + t) * a.M], cmul(y[t], w.at(t)));
+}
+
+// GROUPS: group sums (k_inv's MODE 2), else coefficients.
+template <int L, bool GROUPS>
+__global__ __launch_bounds__(L) void k_inv8(PassArgs a) {
+  using SC = Strip<L>;
+  constexpr int C = SC::C, E = 8, LOG = SC::RC::LOG;
+  bind_product(a);
+  __shared__ cd lds[SC::COL * C];
+  const int tid = threadIdx.x;
+  const int tile = tile_of_block(a.ntiles);
+  const unsigned long long tpb = a.M / C;
+  const unsigned long long ob = (unsigned)tile / (unsigned)tpb;  // tpb < 2^31
+  const unsigned long long m0 = ((unsigned)tile % (unsigned)tpb) * (unsigned long long)C;
+  const int c = tid % C, r0 = tid / C;
+  const unsigned long long m = m0 + c;
+  cd *base = a.data + ob * a.S + m;
+  cd x[E], y[E];
+#pragma unroll
+  for (int t = 0; t < E; t++) y[t] = ld_nt(&base[(unsigned long long)(E * r0 + t) * a.M]);
+  Walk8 w;
+  w.template init_shared<C>(a.roots, a.tw_mul * m * brev((unsigned)r0, LOG - 3), a.tw_mul * m * (L / E));
+#pragma unroll
+  for (int t = 0; t < E; t++) y[t] = cmulc(y[t], w.at(t));
+  row_inverse<L, E>(y, x, lds + c * SC::COL, a.tl, r0);
+  double worst = 0.0;
+  const cd wun = omega_direct(a.roots, (unsigned long long)r0 * a.M + m);
+  if constexpr (GROUPS) __syncthreads();  // the points are read: the tile takes the coefficients
+#pragma unroll
+  for (int h = 0; h < E; h++) {
+    const int row = r0 + h * (L / E);
+    const cd f = cmulc(x[h], cmul(wun, w64(2 * h)));
+    if constexpr (GROUPS) {
+      // group mode implies coefficients below 2^51
+      const long long cr = round_coef(f.x * a.inv_n, true, worst);
+      const long long ci = round_coef(f.y * a.inv_n, true, worst);
+      reinterpret_cast<longlong2 *>(lds)[slot<C>(row, c)] = make_longlong2(cr, ci);
+    } else {
+      worst = fmax(worst, round_store(a, f, (unsigned long long)row, m, L));
+    }
+  }
+  if constexpr (GROUPS) {
+    __syncthreads();
+    write_group_sums<L, C, L>(a, lds, m0, tid);
+  }
+  margin_reduce(a.margin, worst, a.margin_mask);
 }
 
 // ------------------------------------------------------------- middle pass

@@ -15,9 +15,30 @@ constexpr int mid_blocks(int L) {
   return L % 3 == 0 ? (L < 1536 ? 1536 / L : 1) : (L < wave ? wave / L : 1);
 }
 
+// The packing and unpacking passes of single products take eight points per thread
+// (k_fwd8, k_inv8) up to this many tiles of eight columns in a launch, two a CU: 12000
+// by 12000 words 38.3 -> 35.1 us, 2^17 by 2^17 49.6 -> 48.8 us; twice as many make no
+// difference. Strided passes between points of transforms are slower so (2^20 points
+// through the transform calls 123 -> 125 us), and a batched product keeps its class's
+// kernel however many share the launch.
+constexpr int STRIP_TILES = 512;
+template <int L, int C>
+constexpr bool has_strip() {
+  return C == 8 && (L == 64 || L == 128 || L == 256);
+}
+
 // Strided passes are powers of two (the 3 * 2^k factor sits in the innermost pass).
 template <int L, int C>
 int launch_fwd(bool pack, int grid, int gy, hipStream_t s, const PassArgs &a) {
+  if constexpr (has_strip<L, C>()) {
+    if (pack && !a.desc && grid * gy <= STRIP_TILES) {
+      if (a.lower)
+        BCG_LAUNCH2((k_fwd8<L, true>), grid, gy, L, s, a);
+      else
+        BCG_LAUNCH2((k_fwd8<L, false>), grid, gy, L, s, a);
+      return 0;
+    }
+  }
   if (pack && a.lower)
     BCG_LAUNCH2((k_fwd<L, C, true, 0, true>), grid, gy, (Tile<L, C>::T), s, a);
   else if (pack)
@@ -30,6 +51,15 @@ int launch_fwd(bool pack, int grid, int gy, hipStream_t s, const PassArgs &a) {
 // Unpacking into group sums (a.ybuf) exists for 8- and 16-column tiles.
 template <int L, int C>
 int launch_inv(bool unpack, int grid, int gy, hipStream_t s, const PassArgs &a) {
+  if constexpr (has_strip<L, C>()) {
+    if (unpack && !a.desc && grid * gy <= STRIP_TILES) {
+      if (a.ybuf)
+        BCG_LAUNCH2((k_inv8<L, true>), grid, gy, L, s, a);
+      else
+        BCG_LAUNCH2((k_inv8<L, false>), grid, gy, L, s, a);
+      return 0;
+    }
+  }
   if (unpack && a.ybuf) {
     if constexpr (C == 8 || C == 16)
       BCG_LAUNCH2((k_inv<L, C, 2>), grid, gy, (Tile<L, C>::T), s, a);

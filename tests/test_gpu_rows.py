@@ -107,3 +107,28 @@ def test_innermost_pass_of_transforms(bc, inner):
                 assert np.abs(back / n - x).max() <= 1e-13 * np.abs(x).max() * np.log2(n)
         finally:
             bc.plan_force(n, -1)
+
+
+@pytest.mark.parametrize("rows", [64, 128, 256])
+@pytest.mark.parametrize("inner", [192, 256])
+def test_packing_and_unpacking_of_few_tiles(bc, rows, inner):
+    # eight columns: balanced, and with words in the upper digit half (4 to 1)
+    n = rows * inner
+    if n < 12288:
+        pytest.skip("shorter lengths run as one pass")
+    total = max(t for t in range(2, 2 * n, 2) if bc.plan(t // 2, t // 2)["points"] <= n)
+    picks = [i for i, (P, L, C) in enumerate(bc.plan_candidates(n)) if P == 2 and L == [rows, inner] and C[0] == 8]
+    assert picks
+    try:
+        bc.plan_force(n, picks[0])
+        for al in (total // 2, total * 4 // 5):
+            bl = total - al
+            a, b = operands(rows + al, al, bl)
+            c, info = bc.mul(a, b)
+            assert info["passes"] == 2
+            assert np.array_equal(c, exact_product(a, b)), (al, bl)
+            ones = np.full(al, 0xFFFFFFFF, dtype=np.uint32)
+            c, _ = bc.mul(ones, b)
+            assert np.array_equal(c, exact_product(ones, b)), (al, bl)
+    finally:
+        bc.plan_force(n, -1)
