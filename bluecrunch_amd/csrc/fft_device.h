@@ -458,6 +458,19 @@ struct Row {
   static_assert(NST2 >= 2 && L % E == 0, "length too short for the row stages");
 };
 
+// Where value i of row_forward's result (row_inverse's operand) of thread tid belongs
+// among the L points, and whether there is one.
+template <int L, int E>
+__device__ __forceinline__ int row_at(int tid, int i) {
+  using RC = Row<L, E>;
+  if constexpr (RC::THREE) return RC::pad(3 * (tid + i / 3 * RC::T) + i % 3);
+  else return RC::template slot<1>(E * tid, i);
+}
+template <int L, int E>
+__device__ __forceinline__ bool row_has(int tid, int i) {
+  return !Row<L, E>::THREE || i < 6 || tid + 2 * Row<L, E>::T < L / 3;
+}
+
 // A thread index the compiler cannot see through: the level twiddles of A's, B's
 // and the inverse transform are the same values, and keeping them all from one
 // transform to the next takes about 100 registers, and with them half the waves;

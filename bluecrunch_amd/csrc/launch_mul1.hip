@@ -5,6 +5,12 @@ namespace bcg {
 
 template <int L>
 int launch_mul1(int grid, hipStream_t s, const ClassArgs &ca) {
+  if constexpr (has_mul2<L>()) {
+    if (!ca.desc) {  // a product alone
+      hipLaunchKernelGGL((k_mul2<L>), dim3(1), dim3(2 * Row<L>::T), 0, s, ca);
+      return 0;
+    }
+  }
   hipLaunchKernelGGL((k_mul1<L>), dim3(grid), dim3(Row<L>::T), 0, s, ca);
   return 0;
 }
