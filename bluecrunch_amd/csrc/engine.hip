@@ -696,13 +696,12 @@ int class_id(unsigned long long N) {
 //    workgroups' LDS on a CU (so not with 512 rows), else 8: 8 against 16 columns
 //    is 75 us against 79 us at 2^20 points, 107 us against 100 us at 2^21 and
 //    8.6 ms against 9.2 ms in the 512-row pass at 3 * 2^26.
-// Batched products take the same splits from 2^15 points up (64 products of 2^15: 90 us
-// with 256 x 128 against 99 us with 64 x 512, of 2^17 233 us with 256 x 512 against 252
-// with 64 x 2048), except an inner pass of 384, which gives way to 64 rows (64 of 98304
-// points: 180 us against 194 us). Shorter ones, which come by the hundred, keep 64
-// rows (4096 products of 16 to 16384 words: 670 us against 678 us), and 64 rows take
-// 16 columns, whose tiles are half a wave otherwise (400 of 12288 points: 199 us
-// against 223 us).
+// Batched products take the same splits, but
+//  * 16 columns up to 2^16 points and with 64 rows: half the group sums, and tiles of
+//    whole waves (200 of 2^15 points: 206 us against 219 us with eight columns, of
+//    49152 291 us against 319 us, of 12288 120 us against 133 us);
+//  * 64 rows in place of an inner pass of 384 (64 of 98304 points: 180 us against
+//    194 us).
 int default_candidate(const std::vector<Plan> &c, bool batched = false) {
   const unsigned long long N = c[0].N;
   auto find = [&](int P, unsigned long long l0, unsigned long long l1, int c0) {
@@ -718,8 +717,8 @@ int default_candidate(const std::vector<Plan> &c, bool batched = false) {
     unsigned long long rows = 256;
     while (N / rows > max_in) rows *= 2;
     while (rows > 64 && N / rows < 128) rows /= 2;
-    if (batched && (N <= 24576 || N / rows == 384)) rows = 64;
-    const int cols = (rows <= 256 && N / rows >= 16 * 384) || (batched && rows == 64) ? 16 : 8;
+    if (batched && N / rows == 384) rows = 64;
+    const int cols = (rows <= 256 && N / rows >= 16 * 384) || (batched && (N <= 65536 || rows == 64)) ? 16 : 8;
     const int i = find(2, rows, 0, cols);
     if (i >= 0) return i;
   } else {
@@ -1040,6 +1039,10 @@ int read_margin(hipStream_t s, double *m) {
 // sum_i c_i 2^{b i} as K words instead of C 64-bit coefficients (about a
 // quarter of the bytes), and the carry reads those sums. Returns K, or 0 when
 // the plan keeps plain coefficients; group_stride rounds K up to 4 words.
+// At most 12 words: 16 digits of 16 bits take 10, and 48 bytes of sums in place of 128
+// of coefficients are worth their carry (400 batched products of 24576 points, 303 us
+// against 333 us; with eight-word sums only they kept coefficients).
+constexpr int GROUP_STRIDE_MAX = 12;
 int group_stride(int K) { return (K + 3) & ~3; }
 // Words per exact group sum of G digits of b bits (coefficients below 2^cb),
 // 0 when the group-sum carry does not cover that shape.
@@ -1053,7 +1056,7 @@ int group_words_for(int G, int b, int cb) {
   const int K = (off_max + b * (G - 1) + cb + 31) / 32;
   // groups covering one word: at most ceil(32 K / (G b)) + 1
   const int cover = (32 * K + G * b - 1) / (G * b) + 1;
-  if (cover > CARRY_GCOV || group_stride(K) > 8) return 0;
+  if (cover > CARRY_GCOV || group_stride(K) > GROUP_STRIDE_MAX) return 0;
   return K;
 }
 

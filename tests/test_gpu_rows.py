@@ -132,3 +132,25 @@ def test_packing_and_unpacking_of_few_tiles(bc, rows, inner):
             assert np.array_equal(c, exact_product(ones, b)), (al, bl)
     finally:
         bc.plan_force(n, -1)
+
+
+@pytest.mark.parametrize("n", [12288, 16384, 24576, 32768, 49152])
+def test_group_sums_of_nine_to_twelve_words(bc, n):
+    # sixteen columns with 15- and 16-bit digits: the longest operands of the class,
+    # random and all ones (the largest coefficients), odd lengths below them
+    total = max(t for t in range(2, 2 * n, 2) if bc.plan(t // 2, t // 2)["points"] <= n)
+    picks = [i for i, (P, L, C) in enumerate(bc.plan_candidates(n)) if P == 2 and C[0] == 16][:2]
+    assert picks
+    try:
+        for i in picks:
+            bc.plan_force(n, i)
+            for al, bl in ((total // 2, total // 2), (total // 2 - 5, total // 2 - 26)):
+                a, b = operands(n + al, al, bl)
+                c, info = bc.mul(a, b)
+                assert (info["group_digits"], info["group_stride"]) == (16, 12), info
+                assert np.array_equal(c, exact_product(a, b))
+                ones = np.full(al, 0xFFFFFFFF, dtype=np.uint32)
+                c, _ = bc.mul(ones, np.full(bl, 0xFFFFFFFF, dtype=np.uint32))
+                assert np.array_equal(c, exact_product(ones, ones[:bl]))
+    finally:
+        bc.plan_force(n, -1)
