@@ -2349,6 +2349,28 @@ int batch_plan(BatchPlan &bp, uint32_t *C, const uint32_t *A, const uint32_t *B,
 // workgroups follow each other on a CU, and replayed ones keep device copies.
 constexpr size_t HOST_DESC_MAX = 512;
 
+// Scratch of a plan's multi-pass groups (one after the other on one stream).
+int batch_scratch(const BatchPlan &bp, BatchBufs &bb) {
+  size_t arr = 0, blk = 16, slots = 0;
+  for (auto &gr : bp.mgroups) {
+    const Plan &p = gr.first;
+    arr = std::max(arr, (size_t)p.N * sizeof(cd) * gr.second.second);
+    slots = std::max(slots, batch_slot_bytes(p, gr.second.second));
+    const unsigned long long wpb = (unsigned long long)CT * CWPT;
+    unsigned long long nb = 1;
+    for (size_t k = 0; k < gr.second.second; k++)
+      nb = std::max(nb, (unsigned long long)((bp.mdesc[gr.second.first + k].cl + wpb - 1) / wpb));
+    blk = std::max(blk, (size_t)((nb + 15) & ~15ull) * gr.second.second);
+  }
+  if (arr) {
+    if (int rc = ensure(bb.tA, arr)) return rc;
+    if (int rc = ensure(bb.tB, arr)) return rc;
+    if (int rc = ensure(bb.blk, blk)) return rc;
+    if (int rc = ensure(bb.slots, slots)) return rc;
+  }
+  return 0;
+}
+
 // Descriptors to the device (or pinned host memory) and scratch sized (no
 // allocation afterwards). keep_dev: a captured batch's descriptors stay on the device.
 int batch_upload(BatchPlan &bp, BatchBufs &bb, hipStream_t s, bool keep_dev) {
@@ -2369,23 +2391,7 @@ int batch_upload(BatchPlan &bp, BatchBufs &bb, hipStream_t s, bool keep_dev) {
   if (int rc = ensure(bb.mdesc, nm * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.cdesc, nc * sizeof(MulDesc))) return rc;
   if (int rc = ensure(bb.margins, (nm + nc) * sizeof(unsigned int))) return rc;
-  size_t arr = 0, blk = 16, slots = 0;
-  for (auto &gr : bp.mgroups) {
-    const Plan &p = gr.first;
-    arr = std::max(arr, (size_t)p.N * sizeof(cd) * gr.second.second);
-    slots = std::max(slots, batch_slot_bytes(p, gr.second.second));
-    const unsigned long long wpb = (unsigned long long)CT * CWPT;
-    unsigned long long nb = 1;
-    for (size_t k = 0; k < gr.second.second; k++)
-      nb = std::max(nb, (unsigned long long)((bp.mdesc[gr.second.first + k].cl + wpb - 1) / wpb));
-    blk = std::max(blk, (size_t)((nb + 15) & ~15ull) * gr.second.second);
-  }
-  if (arr) {
-    if (int rc = ensure(bb.tA, arr)) return rc;
-    if (int rc = ensure(bb.tB, arr)) return rc;
-    if (int rc = ensure(bb.blk, blk)) return rc;
-    if (int rc = ensure(bb.slots, slots)) return rc;
-  }
+  if (int rc = batch_scratch(bp, bb)) return rc;
   if (nt)
     if (int rc = h2d(bb.tdesc.p, bp.tiny.data(), nt * sizeof(MulDesc), s)) return rc;
   if (nm)
@@ -2523,12 +2529,13 @@ int batch_finish(const BatchPlan &bp, BatchBufs &bb, hipStream_t s, double *wors
 
 // Batched calls whose margins are judged together at the end (radix_convert): the
 // levels' launches follow each other on the stream without a wait. The plain
-// call's scratch serves them all in stream order; the margins have a buffer of
-// their own.
+// call's scratch serves them all in stream order; descriptors and margins have
+// buffers of their own.
 struct RadixBatches {
-  DInt margins;
-  size_t used = 0;
+  DInt margins, desc;
   std::vector<BatchPlan> plans;
+  std::vector<size_t> first;  // of each plan: its first descriptor (tiny, multi-pass, one-pass ones)
+  std::vector<size_t> margin;  // and its first margin
 };
 
 int radix_batch_begin(RadixBatches **rb, size_t products) {
@@ -2542,24 +2549,50 @@ int radix_batch_begin(RadixBatches **rb, size_t products) {
   return 0;
 }
 
-int radix_batch_run(RadixBatches *rb, uint32_t *C, const uint32_t *A, const uint32_t *B, const size_t *c_off,
+int radix_batch_add(RadixBatches *rb, uint32_t *C, const uint32_t *A, const uint32_t *B, const size_t *c_off,
                     const size_t *cl, const size_t *a_off, const size_t *al, const size_t *b_off, const size_t *bl,
-                    size_t count, hipStream_t s) {
+                    size_t count) {
   rb->plans.emplace_back();
   BatchPlan &bp = rb->plans.back();
   if (int rc = batch_plan(bp, C, A, B, nullptr, c_off, cl, a_off, al, b_off, bl, nullptr, nullptr, count)) return rc;
   if (!bp.single.empty()) return fail(BCG_E_ARG, "radix products go through a batch");
-  if (int rc = batch_upload(bp, g_bb, s, true)) return rc;
-  unsigned int *m = (unsigned int *)rb->margins.p + rb->used;
-  rb->used += bp.mdesc.size() + bp.cdesc.size();
-  return batch_launch(bp, g_bb, s, m);
+  return batch_scratch(bp, g_bb);
 }
 
-// Waits for the launches; *ok is false when a margin reached 0.25.
-int radix_batch_end(RadixBatches *rb, bool *ok, hipStream_t s) {
-  std::vector<unsigned int> mb(rb->used);
-  int rc = rb->used ? d2h(mb.data(), rb->margins.p, rb->used * sizeof(unsigned int), s) : 0;
-  if (!rc) {
+int radix_batch_upload(RadixBatches *rb, hipStream_t s) {
+  std::vector<MulDesc> all;
+  size_t margins = 0;
+  for (const BatchPlan &bp : rb->plans) {
+    rb->first.push_back(all.size());
+    rb->margin.push_back(margins);
+    all.insert(all.end(), bp.tiny.begin(), bp.tiny.end());
+    all.insert(all.end(), bp.mdesc.begin(), bp.mdesc.end());
+    all.insert(all.end(), bp.cdesc.begin(), bp.cdesc.end());
+    margins += bp.mdesc.size() + bp.cdesc.size();
+  }
+  if (all.empty()) return 0;
+  if (int rc = dalloc(rb->desc, all.size() * (sizeof(MulDesc) / sizeof(uint32_t)))) return rc;
+  return h2d(rb->desc.p, all.data(), all.size() * sizeof(MulDesc), s);
+}
+
+int radix_batch_launch(RadixBatches *rb, size_t i, hipStream_t s) {
+  const BatchPlan &bp = rb->plans[i];
+  MulDesc *d = (MulDesc *)rb->desc.p + rb->first[i];
+  BatchBufs view = g_bb;  // sized for every plan
+  view.tdesc.p = d;
+  view.mdesc.p = d + bp.tiny.size();
+  view.cdesc.p = d + bp.tiny.size() + bp.mdesc.size();
+  return batch_launch(bp, view, s, (unsigned int *)rb->margins.p + rb->margin[i]);
+}
+
+// launched: waits for the batches, of which every one was launched; *ok is false when a
+// margin reached 0.25. The batches end either way.
+int radix_batch_end(RadixBatches *rb, bool launched, bool *ok, hipStream_t s) {
+  size_t n = 0;
+  for (const BatchPlan &bp : rb->plans) n += bp.mdesc.size() + bp.cdesc.size();
+  std::vector<unsigned int> mb(n);
+  int rc = launched && n ? d2h(mb.data(), rb->margins.p, n * sizeof(unsigned int), s) : 0;
+  if (launched && !rc) {
     for (unsigned int b : mb) {
       float f;
       memcpy(&f, &b, sizeof f);
@@ -2572,6 +2605,7 @@ int radix_batch_end(RadixBatches *rb, bool *ok, hipStream_t s) {
     }
   }
   dfree(rb->margins);
+  dfree(rb->desc);
   delete rb;
   return rc;
 }
