@@ -2532,10 +2532,12 @@ int batch_finish(const BatchPlan &bp, BatchBufs &bb, hipStream_t s, double *wors
 // call's scratch serves them all in stream order; descriptors and margins have
 // buffers of their own.
 struct RadixBatches {
-  DInt margins, desc;
+  DInt margins;
+  size_t margins_used = 0;
   std::vector<BatchPlan> plans;
-  std::vector<size_t> first;  // of each plan: its first descriptor (tiny, multi-pass, one-pass ones)
-  std::vector<size_t> margin;  // and its first margin
+  std::vector<DInt> desc;                 // one array per upload
+  std::vector<const MulDesc *> first;     // of each uploaded plan: its descriptors (tiny, multi-pass, one-pass ones)
+  std::vector<unsigned int *> margin;     // and its margins
 };
 
 int radix_batch_begin(RadixBatches **rb, size_t products) {
@@ -2559,37 +2561,41 @@ int radix_batch_add(RadixBatches *rb, uint32_t *C, const uint32_t *A, const uint
   return batch_scratch(bp, g_bb);
 }
 
+// The descriptors of the plans added since the last upload.
 int radix_batch_upload(RadixBatches *rb, hipStream_t s) {
   std::vector<MulDesc> all;
-  size_t margins = 0;
-  for (const BatchPlan &bp : rb->plans) {
-    rb->first.push_back(all.size());
-    rb->margin.push_back(margins);
-    all.insert(all.end(), bp.tiny.begin(), bp.tiny.end());
-    all.insert(all.end(), bp.mdesc.begin(), bp.mdesc.end());
-    all.insert(all.end(), bp.cdesc.begin(), bp.cdesc.end());
-    margins += bp.mdesc.size() + bp.cdesc.size();
-  }
+  const size_t from = rb->first.size();
+  for (size_t i = from; i < rb->plans.size(); i++)
+    for (const auto *v : {&rb->plans[i].tiny, &rb->plans[i].mdesc, &rb->plans[i].cdesc})
+      all.insert(all.end(), v->begin(), v->end());
   if (all.empty()) return 0;
-  if (int rc = dalloc(rb->desc, all.size() * (sizeof(MulDesc) / sizeof(uint32_t)))) return rc;
-  return h2d(rb->desc.p, all.data(), all.size() * sizeof(MulDesc), s);
+  rb->desc.emplace_back();
+  if (int rc = dalloc(rb->desc.back(), all.size() * (sizeof(MulDesc) / sizeof(uint32_t)))) return rc;
+  const MulDesc *d = (const MulDesc *)rb->desc.back().p;
+  for (size_t i = from; i < rb->plans.size(); i++) {
+    const BatchPlan &bp = rb->plans[i];
+    rb->first.push_back(d);
+    rb->margin.push_back((unsigned int *)rb->margins.p + rb->margins_used);
+    d += bp.tiny.size() + bp.mdesc.size() + bp.cdesc.size();
+    rb->margins_used += bp.mdesc.size() + bp.cdesc.size();
+  }
+  return h2d(rb->desc.back().p, all.data(), all.size() * sizeof(MulDesc), s);
 }
 
 int radix_batch_launch(RadixBatches *rb, size_t i, hipStream_t s) {
   const BatchPlan &bp = rb->plans[i];
-  MulDesc *d = (MulDesc *)rb->desc.p + rb->first[i];
-  BatchBufs view = g_bb;  // sized for every plan
+  MulDesc *d = const_cast<MulDesc *>(rb->first[i]);
+  BatchBufs view = g_bb;  // sized for the plans so far
   view.tdesc.p = d;
   view.mdesc.p = d + bp.tiny.size();
   view.cdesc.p = d + bp.tiny.size() + bp.mdesc.size();
-  return batch_launch(bp, view, s, (unsigned int *)rb->margins.p + rb->margin[i]);
+  return batch_launch(bp, view, s, rb->margin[i]);
 }
 
 // launched: waits for the batches, of which every one was launched; *ok is false when a
 // margin reached 0.25. The batches end either way.
 int radix_batch_end(RadixBatches *rb, bool launched, bool *ok, hipStream_t s) {
-  size_t n = 0;
-  for (const BatchPlan &bp : rb->plans) n += bp.mdesc.size() + bp.cdesc.size();
+  const size_t n = rb->margins_used;
   std::vector<unsigned int> mb(n);
   int rc = launched && n ? d2h(mb.data(), rb->margins.p, n * sizeof(unsigned int), s) : 0;
   if (launched && !rc) {
@@ -2605,7 +2611,7 @@ int radix_batch_end(RadixBatches *rb, bool launched, bool *ok, hipStream_t s) {
     }
   }
   dfree(rb->margins);
-  dfree(rb->desc);
+  for (DInt &x : rb->desc) dfree(x);
   delete rb;
   return rc;
 }
