@@ -1320,9 +1320,12 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
     // Word-aligned group starts (G b a multiple of 32, e.g. b even): group gl
     // starts at block word D + gl Q, so word wl = D + gh Q + o takes word
     // o + t Q of group gh - t, at LDS index ih - t (gKs - Q), ih = gh gKs + o;
-    // all advance by one per word. o < Q < K, so term 0 only needs gh >= 0,
-    // and gh < ngl for every word of the block.
+    // all advance by one per word. A term counts where its group is staged:
+    // none below the first, and none past the last group of the product, which an
+    // output longer than the digits (AL + BL + 1 words at a full class, a long
+    // addend) goes beyond. o < Q < K, so term 0 needs no more than that.
     const int Q = gb >> 5, dg = a.gKs - Q;
+    const unsigned staged = ngl > 0 ? (unsigned)ngl : 0u;
     int wl = tid * GWPT - 1;
     const int x0 = wl - D;  // >= -1
     int gh = x0 < 0 ? -1 : (int)((unsigned)x0 / (unsigned)Q);
@@ -1336,11 +1339,10 @@ static __global__ __launch_bounds__(GCT) void k_carry_groups(CarryArgs a) {
         gh += wrap ? 1 : 0;
         ih += wrap ? 1 + dg : 1;
       }
-      const unsigned i0 = gh >= 0 ? (unsigned)ih : 0u;
-      unsigned long long p = gh >= 0 ? gl_w[i0 + (i0 >> 5)] : 0u;
+      unsigned long long p = 0;
 #pragma unroll
-      for (int t = 1; t < GCOV; t++) {
-        const bool ok = gh >= t && o + t * Q < a.gK;
+      for (int t = 0; t < GCOV; t++) {
+        const bool ok = (unsigned)(gh - t) < staged && (t == 0 || o + t * Q < a.gK);
         const unsigned i = ok ? (unsigned)(ih - t * dg) : 0u;
         const unsigned x = gl_w[i + (i >> 5)];
         p += ok ? x : 0u;
