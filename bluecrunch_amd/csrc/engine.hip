@@ -874,7 +874,9 @@ int end_carry(const CarryArgs &c, hipStream_t s, double *margin, int ends = 0) {
   float f;
   memcpy(&f, &g.hres->margin, sizeof f);
   *margin = (double)f;
-  if (f < 0.25f && g.hres->open_carry && !runs) {
+  // whatever the margin: fft_to_int returns the words it rounded, and a product that is
+  // run again from 0.25 on has an open block too seldom to be told apart
+  if (g.hres->open_carry && !runs) {
     {
       ProfScope ps(BCG_K_CARRY, s);
       launch_ripple(c, 1, s);

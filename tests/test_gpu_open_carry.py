@@ -57,3 +57,21 @@ def test_open_block_of_fft_to_int(bc, start, length):
         got = bc.fft_to_int(z, 2 * words, words, 16)
         want = ((1 << (32 * length)) - 1 + carry) << (32 * first)
         assert np.array_equal(got, int_to_words(want, words))
+
+
+@pytest.mark.parametrize("off", [0.3, 0.45, -0.45])
+@pytest.mark.parametrize("carry", [0, 1])
+def test_open_block_of_fft_to_int_between_whole_numbers(bc, oracle, off, carry):
+    # the points are rounded whatever their distance; the carry through words of
+    # ones runs on all the same
+    words = 3 * 1024 + 13
+    digits = np.full(2 * words, 65535.0)
+    digits[0] += carry
+    length = 8192
+    z = np.zeros(length, dtype=np.complex128)
+    z[:2 * words] = (digits + off) * length
+    want, margin = oracle.fft_to_int(z, length, words, 16)
+    got = bc.fft_to_int(z, length, words, 16)
+    assert margin > 0.25
+    assert np.array_equal(want, np.zeros(words) if carry else np.full(words, 0xFFFFFFFF, dtype=np.uint32))
+    assert np.array_equal(got, want)
