@@ -346,10 +346,12 @@ int d2h(void *dst, const void *src, size_t bytes, hipStream_t s) {
   return 0;
 }
 
-int prepare_noalloc();  // tables and the scratch address of bcg_mul_dev_noalloc
+int prepare_noalloc();     // tables and the scratch address of bcg_mul_dev_noalloc
+void release_resources();  // everything the engine holds
 
-int init_locked(int device) {
-  if (g.ready) return 0;
+// What a call needs besides tables: device, streams, events, and the memory that
+// every product or sum uses.
+int init_resources(int device) {
   int n = 0;
   hipError_t e = hipGetDeviceCount(&n);
   if (e != hipSuccess || n <= 0) return fail(BCG_E_NODEV, "no HIP device", e);
@@ -363,7 +365,6 @@ int init_locked(int device) {
   }
   HIPCHK(hipEventCreateWithFlags(&g.fork_ev, hipEventDisableTiming));
   g.device = device;
-  g.ready = true;
   if (int rc = ensure(g.margin, sizeof(unsigned int) * MARGIN_SLOTS * MARGIN_STRIDE)) return rc;
   if (int rc = ensure(g.scan, 256)) return rc;
   if (int rc = ensure(g.one, 4)) return rc;
@@ -371,7 +372,20 @@ int init_locked(int device) {
   LAUNCH(k_fill_u32, 1, 64, g.stream, (uint32_t *)g.one.p, 1ull, 1u);
   HIPCHK(hipGetLastError());
   HIPCHK(hipHostMalloc((void **)&g.hres, sizeof(HostResult), hipHostMallocMapped));
+  memset(g.hres, 0, sizeof(HostResult));
+  g.hres->seq = g.seq;  // nothing announced since
   HIPCHK(hipHostGetDevicePointer((void **)&g.hres_dev, g.hres, 0));
+  return 0;
+}
+
+// All or nothing: after a failure the next call starts over.
+int init_locked(int device) {
+  if (g.ready) return 0;
+  if (int rc = init_resources(device)) {
+    release_resources();
+    return rc;
+  }
+  g.ready = true;
   // every kernel family's code object now rather than inside a first product
   // (a failure here only defers the load to the first launch)
   for (auto f : {preload_mul1, preload_fwd, preload_inv, preload_mid, preload_row, preload_keep})
@@ -2013,21 +2027,8 @@ struct ScratchScope {
   }
 };
 
-}  // namespace
-
-// =================================================================== C ABI
-
-extern "C" {
-
-int bcg_init(int device) {
-  std::lock_guard<std::recursive_mutex> lk(g_lock);
-  return init_locked(device);
-}
-
-int bcg_shutdown(void) {
-  std::lock_guard<std::recursive_mutex> lk(g_lock);
-  if (!g.ready) return 0;
-  (void)hipStreamSynchronize(g.stream);
+void release_resources() {
+  if (g.stream) (void)hipStreamSynchronize(g.stream);
   g_defer.open = false;
   g_defer.n = 0;
   for (DevBuf *b : {&g.bufA, &g.bufB, &g.wA, &g.wB, &g.wC, &g.blk, &g.margin, &g.zbuf, &g.scan, &g.flags, &g.one,
@@ -2050,8 +2051,8 @@ int bcg_shutdown(void) {
   }
   if (g.fork_ev) (void)hipEventDestroy(g.fork_ev);
   g.fork_ev = nullptr;
-  (void)hipStreamDestroy(g.stream);
-  (void)hipStreamDestroy(g.cap);
+  if (g.stream) (void)hipStreamDestroy(g.stream);
+  if (g.cap) (void)hipStreamDestroy(g.cap);
   g_bb.release();
   ep_trim();
   if (g.hres) (void)hipHostFree(g.hres);
@@ -2063,6 +2064,22 @@ int bcg_shutdown(void) {
   g.stream = nullptr;
   g.cap = nullptr;
   g.ready = false;
+}
+
+}  // namespace
+
+// =================================================================== C ABI
+
+extern "C" {
+
+int bcg_init(int device) {
+  std::lock_guard<std::recursive_mutex> lk(g_lock);
+  return init_locked(device);
+}
+
+int bcg_shutdown(void) {
+  std::lock_guard<std::recursive_mutex> lk(g_lock);
+  if (g.ready) release_resources();
   return 0;
 }
 

@@ -47,6 +47,33 @@ def _run(fake, body):
     return r.stdout
 
 
+def test_failed_initialisation(fake):
+    out = _run(fake, """
+failed = 0
+for nth in range(1, 400):
+    fake.fake_fail(nth)
+    rc = L.bcg_init(0)
+    reached = fake.fake_armed() == 0
+    fake.fake_fail(0)
+    assert rc == 0 or reached, nth
+    failed += rc != 0
+    # whatever is left: a product of several passes and a difference
+    a = bc.DeviceWords.from_host(np.arange(1, 20001, dtype=np.uint32))
+    c = bc.DeviceWords(40000)
+    bc.mul_dev(c.ptr, 40000, a.ptr, 20000, a.ptr, 20000)
+    x, y, t = operands()
+    bc.bf_op("sub", t, x, y, 0)
+    del a, c, x, y, t
+    bc.check(L.bcg_shutdown(), "shutdown")
+    assert fake.fake_live() == 0, (nth, fake.fake_live())
+    if not reached:
+        break
+assert failed >= 10 and not reached
+print("done", failed)
+""")
+    assert out.startswith("done")
+
+
 def test_failed_difference_leaves_no_order_behind(fake):
     # the search for the word that decides the order leaves it to the difference behind
     # it, which clears it: the search must not run if the difference cannot
