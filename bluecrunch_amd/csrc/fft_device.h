@@ -243,14 +243,15 @@ struct Walk16 {
 // the strided passes of transforms, whose points a caller sees (a product's are rounded to
 // whole numbers, and its passes keep Walk16): error against 80-bit sums at 49152 points
 // 2.87e-16 forward and 2.90e-16 inverse, with Walk16 2.92e-16 and 2.99e-16; a convolution
-// of 2^20 points through the transform calls 123.7-127.7 us, with Walk16 125.0-125.4 us.
+// of 2^20 points through the transform calls 121.5-124.9 us (124.2-127.0 us with a pointer
+// to the roots, which put the arguments of every kernel using it into private memory).
 struct Walk16Fine {
-  const Roots *r;
+  Roots r;
   unsigned long long u0, du;
   cd g4, g8, g12, p;
   template <int C>
   __device__ __forceinline__ void init_shared(const Roots &roots, unsigned long long u, unsigned long long d) {
-    r = &roots;
+    r = roots;
     u0 = u;
     du = d;
     if constexpr (4 * C > 64) {
@@ -267,7 +268,7 @@ struct Walk16Fine {
     }
   }
   __device__ __forceinline__ cd at(int i) {
-    if ((i & 3) == 0) p = omega_direct(*r, u0 + ((i >> 3 & 1) | (i >> 1 & 2)) * du);
+    if ((i & 3) == 0) p = omega_direct(r, u0 + ((i >> 3 & 1) | (i >> 1 & 2)) * du);
     switch (i & 3) {
       case 1: return cmul(p, g8);
       case 2: return cmul(p, g4);
