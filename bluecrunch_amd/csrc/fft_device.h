@@ -240,11 +240,13 @@ struct Walk16 {
 
 // The same sixteen with one product each at most: base, base g, base g^2 and base g^3 from
 // omega_direct as they come up, g^4, g^8 and g^12 shared by lanes as in init_shared. For
-// the strided passes of transforms, whose points a caller sees (a product's are rounded to
-// whole numbers, and its passes keep Walk16): error against 80-bit sums at 49152 points
-// 2.87e-16 forward and 2.90e-16 inverse, with Walk16 2.92e-16 and 2.99e-16; a convolution
-// of 2^20 points through the transform calls 121.5-124.9 us (124.2-127.0 us with a pointer
-// to the roots, which put the arguments of every kernel using it into private memory).
+// the strided passes between points of transforms, which a caller sees, and of products
+// whose middle passes run whole: error against 80-bit sums at 49152 points
+// 2.87e-16 forward and 2.90e-16 inverse, with Walk16 2.92e-16 and 2.99e-16. The other
+// passes of products keep Walk16: their rounding distances are the same with either. A
+// convolution of 2^20 points through the transform calls 121.5-124.9 us (124.2-127.0 us
+// with a pointer to the roots, which put the arguments of every kernel using it into
+// private memory).
 struct Walk16Fine {
   Roots r;
   unsigned long long u0, du;
@@ -459,6 +461,50 @@ __device__ __forceinline__ void levels3_fine(cd (&x)[8], const cd (&tb)[3], cd t
         x[t + half] = INV ? csub(a, c) : cmul(csub(a, c), w);
       }
     }
+  }
+}
+
+// The same for four levels: t1[j - 1] = tl[(q + j span/16) tstride], j = 1..3, and
+// u1 = tl[2 (q + span/16) tstride]. With products the 256-row stage made the splits of 256
+// rows less exact than those of 64, which have no product in it: root mean square rounding
+// distance of products of 5,000,000 words (2^24 points) 1.044 of that of 64 x 64 x 4096,
+// now 0.994; transforms of 2^20 points 0.933 of 128 x 8192, now 0.905. Four loads of cached
+// twiddles more per thread: 2^24 words 2.478 -> 2.492 ms.
+template <bool INV>
+__device__ __forceinline__ void levels4_fine(cd (&x)[16], const cd (&tb)[4], const cd (&t1)[3], cd u1) {
+  const cd w0[4] = {tb[0], t1[0], t1[1], t1[2]};
+#pragma unroll
+  for (int n = 0; n < 4; n++) {
+    const int l = INV ? 3 - n : n, half = 8 >> l;
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+      if ((t & (2 * half - 1)) < half) {
+        const int j = t & (half - 1);
+        cd w = l == 0 ? w0[j & 3] : l == 1 ? (j & 1 ? u1 : tb[1]) : l == 2 ? tb[2] : tb[3];
+        if (j >= half / 2 && half > 1) w = times_i(w);
+        const cd a = x[t], b = x[t + half], c = INV ? cmulc(b, w) : b;
+        x[t] = cadd(a, c);
+        x[t + half] = INV ? csub(a, c) : cmul(csub(a, c), w);
+      }
+    }
+  }
+}
+
+// The outermost stage of a tile of L rows, rows q + t (L / 2^RB) in x: no twiddle a
+// product for two to four levels (of two none is one anyway).
+template <int L, int RB, bool INV>
+__device__ __forceinline__ void first_stage(cd (&x)[1 << RB], const cd *__restrict__ tl, int q) {
+  cd tb[RB];
+  level_bases<RB>(tl, q, 1, tb);
+  if constexpr (RB == 4) {
+    const cd t1[3] = {tl[q + L / 16], tl[q + L / 8], tl[q + 3 * L / 16]};
+    levels4_fine<INV>(x, tb, t1, tl[2 * (q + L / 16)]);
+  } else if constexpr (RB == 3) {
+    levels3_fine<INV>(x, tb, tl[q + L / 8]);
+  } else if constexpr (INV) {
+    dit_levels<RB>(x, tb);
+  } else {
+    dif_levels<RB>(x, tb);
   }
 }
 

@@ -464,9 +464,11 @@ __device__ __forceinline__ void store_rows16(cd *base, const cd (&v)[16], int r0
 }
 
 // LOWER (packing pass): every operand of the launch leaves the upper digit
-// half empty, so a_{j+N} = 0 and the weighted point is a_j w exactly.
+// half empty, so a_{j+N} = 0 and the weighted point is a_j w exactly. The packing of
+// split 8-column tiles is held to the 128 registers of four waves (130 without, no spill).
 template <int L, int C, bool PACK, int CACHE = 0, bool LOWER = false>
-__global__ __launch_bounds__((Tile<L, C>::T)) void k_fwd(PassArgs a) {
+__global__ __launch_bounds__((Tile<L, C>::T))
+__attribute__((amdgpu_waves_per_eu((PACK && !LOWER && C == 8 && SplitTile<L, C>::ON) ? 4 : 1, 8))) void k_fwd(PassArgs a) {
   using TC = Tile<L, C>;
   using ST = SplitTile<L, C>;
   using Walk = std::conditional_t<!PACK && CACHE == 0, Walk16Fine, Walk16>;
@@ -526,7 +528,8 @@ __global__ __launch_bounds__((Tile<L, C>::T)) void k_fwd(PassArgs a) {
         x[t] = ld_nt(&base[(unsigned long long)(r0 + 16 * t) * a.M + m]);
       }
     }
-    dif_levels<4>(x, tb0);
+    const cd t1[3] = {a.tl[r0 + 16], a.tl[r0 + 32], a.tl[r0 + 48]};
+    levels4_fine<false>(x, tb0, t1, a.tl[2 * (r0 + 16)]);
     split_transpose<C>(reinterpret_cast<double *>(lds_raw), x, y, r0, c, false);
     dif_levels_q0<4>(y);
     // row 16 r0 + t has frequency 16 brev4(t) + brev4(r0)
@@ -557,7 +560,7 @@ __global__ __launch_bounds__((Tile<L, C>::T)) void k_fwd(PassArgs a) {
         x[t] = ld_pol<(CACHE & 1) != 0>(&base[row * a.M + m]);
       }
     }
-    dif_levels<RB0>(x, a.tl, q, 1);
+    first_stage<L, RB0, false>(x, a.tl, q);
 #pragma unroll
     for (int t = 0; t < R0; t++) lds[slot<C>(q + t * SUB0, c)] = x[t];
   }
@@ -620,7 +623,12 @@ __attribute__((amdgpu_waves_per_eu((MODE == 1 && SplitTile<L, C>::ON && C >= 8) 
     level_bases<4>(a.tl, r0, 1, tb0);
     double *ld = reinterpret_cast<double *>(lds_raw);
     split_transpose<C>(ld, y, x, r0, c, true);
-    dit_levels<4>(x, tb0);
+    if constexpr (MODE != 1) {  // storing coefficients leaves no registers for them
+      const cd t1[3] = {a.tl[r0 + 16], a.tl[r0 + 32], a.tl[r0 + 48]};
+      levels4_fine<true>(x, tb0, t1, a.tl[2 * (r0 + 16)]);
+    } else {
+      dit_levels<4>(x, tb0);
+    }
     if constexpr (!UNPACK) {
       store_rows16<1, 16, (CACHE & 2) != 0>(base, x, r0, c, m0, a.M);
     } else {
@@ -680,7 +688,7 @@ __attribute__((amdgpu_waves_per_eu((MODE == 1 && SplitTile<L, C>::ON && C >= 8) 
     cd x[R0];
 #pragma unroll
     for (int t = 0; t < R0; t++) x[t] = lds[slot<C>(q + t * SUB0, c)];
-    dit_levels<RB0>(x, a.tl, q, 1);
+    first_stage<L, RB0, true>(x, a.tl, q);
 #pragma unroll
     for (int t = 0; t < R0; t++) {
       unsigned long long row = (unsigned long long)(q + t * SUB0);
@@ -728,25 +736,36 @@ struct Strip {
   static_assert(COL * C >= L * C + L * C / 16, "the coefficients of the tile fit");
 };
 
-// Walk16 for the eight rows 8 r0 + t: Omega^{u0 + brev3(t) du}.
+// Walk16Fine for the eight rows 8 r0 + t: Omega^{u0 + brev3(t) du}. With it and stages
+// without twiddle products the rounding distances of 300007 by 41003 words are 0.996 of
+// those of the sixteen-point kernels (root mean square), 1.039 with Walk16's products;
+// 53.5 -> 53.7 us.
 struct Walk8 {
-  cd base, g1, g2, g4, p2, p1;
+  Roots r;
+  unsigned long long u0, du;
+  cd g2, g4, g6, p;
   template <int C>
-  __device__ __forceinline__ void init_shared(const Roots &r, unsigned long long u0, unsigned long long du) {
+  __device__ __forceinline__ void init_shared(const Roots &roots, unsigned long long u, unsigned long long d) {
     static_assert(4 * C <= 64, "four lanes of a wave share a column");
+    r = roots;
+    u0 = u;
+    du = d;
     const int lane = threadIdx.x & 63;
     const int src0 = (lane % C) + (lane / (4 * C)) * (4 * C);
-    base = omega_direct(r, u0);
-    const cd mine = omega_direct(r, du << ((lane / C) & 3));
-    g1 = make_double2(__shfl(mine.x, src0, 64), __shfl(mine.y, src0, 64));
+    const cd mine = omega_direct(roots, d * (2 * ((lane / C) & 3)));
     g2 = make_double2(__shfl(mine.x, src0 + C, 64), __shfl(mine.y, src0 + C, 64));
     g4 = make_double2(__shfl(mine.x, src0 + 2 * C, 64), __shfl(mine.y, src0 + 2 * C, 64));
+    g6 = make_double2(__shfl(mine.x, src0 + 3 * C, 64), __shfl(mine.y, src0 + 3 * C, 64));
   }
-  // i = 0..7 in increasing order
+  // i = 0..7 in increasing order; brev3(i): 0 4 2 6 1 5 3 7
   __device__ __forceinline__ cd at(int i) {
-    if ((i & 3) == 0) p2 = (i & 4) ? cmul(base, g1) : base;
-    if ((i & 1) == 0) p1 = (i & 2) ? cmul(p2, g2) : p2;
-    return (i & 1) ? cmul(p1, g4) : p1;
+    if ((i & 3) == 0) p = omega_direct(r, u0 + (i >> 2) * du);
+    switch (i & 3) {
+      case 1: return cmul(p, g4);
+      case 2: return cmul(p, g2);
+      case 3: return cmul(p, g6);
+      default: return p;
+    }
   }
 };
 
@@ -782,7 +801,7 @@ __global__ __launch_bounds__(L) void k_fwd8(PassArgs a) {
     else
       x[h] = cmul(make_double2((double)dre[h], (double)dim_[h]), w);
   }
-  row_forward<L, E>(x, y, lds + c * SC::COL, a.tl, r0);
+  row_forward<L, E, true>(x, y, lds + c * SC::COL, a.tl, r0);
   // row 8 r0 + t has frequency (L / 8) brev3(t) + brev(r0)
   Walk8 w;
   w.template init_shared<C>(a.roots, a.tw_mul * m * brev((unsigned)r0, LOG - 3), a.tw_mul * m * (L / E));
@@ -812,7 +831,7 @@ __global__ __launch_bounds__(L) void k_inv8(PassArgs a) {
   w.template init_shared<C>(a.roots, a.tw_mul * m * brev((unsigned)r0, LOG - 3), a.tw_mul * m * (L / E));
 #pragma unroll
   for (int t = 0; t < E; t++) y[t] = cmulc(y[t], w.at(t));
-  row_inverse<L, E>(y, x, lds + c * SC::COL, a.tl, r0);
+  row_inverse<L, E, true>(y, x, lds + c * SC::COL, a.tl, r0);
   double worst = 0.0;
   const cd wun = omega_direct(a.roots, (unsigned long long)r0 * a.M + m);
   if constexpr (GROUPS) __syncthreads();  // the points are read: the tile takes the coefficients
