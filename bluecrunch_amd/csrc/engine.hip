@@ -710,12 +710,10 @@ int class_id(unsigned long long N) {
 //    workgroups' LDS on a CU (so not with 512 rows), else 8: 8 against 16 columns
 //    is 75 us against 79 us at 2^20 points, 107 us against 100 us at 2^21 and
 //    8.6 ms against 9.2 ms in the 512-row pass at 3 * 2^26.
-// Batched products take the same splits, but
-//  * 16 columns up to 2^16 points and with 64 rows: half the group sums, and tiles of
-//    whole waves (200 of 2^15 points: 206 us against 219 us with eight columns, of
-//    49152 291 us against 319 us, of 12288 120 us against 133 us);
-//  * 64 rows in place of an inner pass of 384 (64 of 98304 points: 180 us against
-//    194 us).
+// Batched products take the same splits, with 16 columns up to 2^17 points: half the
+// group sums and tiles of whole waves (200 products of 32768 points 207 us against
+// 222 us with eight columns, of 49152 289 against 318, of 131072 633 against 698; 16 to 64
+// of 131072 points 3 to 5 % less). At 196608 points the two are equal.
 int default_candidate(const std::vector<Plan> &c, bool batched = false) {
   const unsigned long long N = c[0].N;
   auto find = [&](int P, unsigned long long l0, unsigned long long l1, int c0) {
@@ -731,8 +729,7 @@ int default_candidate(const std::vector<Plan> &c, bool batched = false) {
     unsigned long long rows = 256;
     while (N / rows > max_in) rows *= 2;
     while (rows > 64 && N / rows < 128) rows /= 2;
-    if (batched && N / rows == 384) rows = 64;
-    const int cols = (rows <= 256 && N / rows >= 16 * 384) || (batched && (N <= 65536 || rows == 64)) ? 16 : 8;
+    const int cols = (rows <= 256 && N / rows >= 16 * 384) || (batched && N <= (1ull << 17)) ? 16 : 8;
     const int i = find(2, rows, 0, cols);
     if (i >= 0) return i;
   } else {
