@@ -1076,7 +1076,7 @@ int group_words_for(int G, int b, int cb) {
 int group_words(const Plan &p) { return p.P < 2 ? 0 : group_words_for(p.C[0], p.bits, coef_bits(p)); }
 
 // Coefficients of plan p are written transposed when the last pass has
-// narrow column tiles (see unpack_point); the carry reads them back that way.
+// narrow column tiles (see round_store); the carry reads them back that way.
 bool coef_transposed(const Plan &p) { return p.P >= 2 && p.C[0] < 8; }
 
 // Chunked middle passes of three-pass products: the second forward pass, the

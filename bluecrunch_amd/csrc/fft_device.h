@@ -116,13 +116,6 @@ __device__ __forceinline__ int slot(int row, int c) {
   else return pad16(row * C + c);
 }
 
-// pad16(q + t * S), linear in t when 16 | S (q >= 0).
-template <int S>
-__device__ __forceinline__ int slot_step(int q, int t) {
-  if constexpr (S % 16 == 0) return pad16(q) + t * (S + S / 16);
-  else return pad16(q + t * S);
-}
-
 __device__ __forceinline__ unsigned brev(unsigned v, int bits) {
   return bits ? (__builtin_bitreverse32(v) >> (32 - bits)) : 0u;
 }

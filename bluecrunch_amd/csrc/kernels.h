@@ -60,7 +60,7 @@ constexpr int MARGIN_SLOTS = 64;
 constexpr int MARGIN_STRIDE = 32;
 
 // Batched launches (desc != nullptr): product p = blockIdx.y owns the arrays
-// data + p*N, data_b + p*N, coef + p*2N and margin slot p.
+// data + p*N, data_b + p*N, coef + p*2N and margin_mask + 1 margin slots.
 __device__ __forceinline__ void bind_product(PassArgs &a) {
   if (!a.desc) {
     if (a.pair && blockIdx.y == 1) {
@@ -112,12 +112,6 @@ __device__ __forceinline__ double digit_at(const uint32_t *__restrict__ w, unsig
   unsigned long long v = w[wi];
   if (wi + 1 < wl) v |= (unsigned long long)w[wi + 1] << 32;
   return (double)((v >> sh) & ((1ull << bits) - 1ull));
-}
-
-__device__ __forceinline__ void margin_update(unsigned int *m, double d) {
-  float f = (float)d;
-  // non-negative floats order like their bit patterns
-  atomicMax(m, __float_as_uint(f));
 }
 
 // Nearest integer of x clamped at 0, and the rounding distance into worst.
@@ -967,7 +961,7 @@ constexpr int CWPT = 4;
 constexpr int CT = 256;
 
 struct CarryArgs {
-  const MulDesc *desc;       // batched: product blockIdx.y (local) / blockIdx.x (fix), else nullptr
+  const MulDesc *desc;       // batched: product blockIdx.y, else nullptr
   unsigned long long coef_stride;  // batched: coefficients per product (2N)
   const long long *coef;
   unsigned long long ncoef;
